@@ -55,6 +55,11 @@ struct AttnArgs {
   uint32_t nqb;                        // query blocks per head
   float scale_log2;                    // log2(e) / sqrt(dim)
   int causal;
+  // f32 through f16 planes (attn_planes_kernel): per kv head, then again for V, the inverse scale of its planes and
+  // whether its values are too far apart for them (the f32 MFMA kernel computes those heads). NULL: no planes
+  const float* plane_inv;
+  const uint32_t* plane_flag;
+  uint32_t kv_heads;
 };
 
 __device__ __forceinline__ float halves_max(float x) {
@@ -1029,6 +1034,7 @@ __global__ void __launch_bounds__(ATT_NT, 1) attn32_kernel(AttnArgs a) {
   uint32_t qb, h;
   block_coords(a, qb, h);
   const uint32_t g = h / a.group;
+  if (a.plane_flag && !(a.plane_flag[g] | a.plane_flag[a.kv_heads + g])) return;  // attn_planes_kernel has this head
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 31, hf = lane >> 5;
@@ -1140,6 +1146,278 @@ __global__ void __launch_bounds__(ATT_NT, 1) attn32_kernel(AttnArgs a) {
   }
 }
 
+// ------------------------------------------------------------------------------------ f32 through f16 planes
+// Head dim 64 or 128. Every f32 operand is a power of two times the sum of two f16 planes, hi = f16(v 2^e) and
+// lo = f16(v 2^e - hi) (v to 2^-23 of itself), and each product runs as lo x hi + hi x lo + hi x hi on the 32x32x16 f16
+// MFMA with f32 sums: 3/16 of the cycles of the f32 MFMA. K and V are split once per call into scratch, with one scale per kv head;
+// Q rows and P are split in registers. The planes hold a value to 2^-40 of its head's largest, so a head where some
+// row's largest value lies below 2^-16 of the head's largest, or with an inf or NaN, is flagged and left to the f32
+// MFMA kernel, which is launched behind this one and returns at once for the other heads.
+// below, the two passes over K and V and the third launch cost what the products gain (24 heads of 128, 128 tokens: 23.7 us
+// here, 24.4 us on the f32 MFMA; 16 heads, 64 tokens 17.0 and 13.1, 200 tokens causal 27.1 and 41.8)
+constexpr uint32_t PLANES_MIN_TOKENS = 160;
+constexpr uint32_t PLANE_BLOCKS = 16;  // workgroups per kv head of the scan for the largest values
+
+// The per-workgroup largest row maximum and smallest nonzero one (0: an inf or NaN) of a kv head's rows: K (z 0), V (1).
+template <int DP>
+__global__ void __launch_bounds__(256) attn_amax_kernel(AttnArgs a, uint32_t* __restrict__ part) {
+  constexpr int LPR = DP / 8;  // lanes per row
+  __shared__ uint32_t rmax[4], rmin[4];
+  const uint32_t g = blockIdx.y, z = blockIdx.z;
+  const float* src = (const float*)(z ? a.v : a.k) + (size_t)g * DP;
+  const size_t stride = z ? a.vs : a.ks;
+  const uint32_t sub = threadIdx.x % LPR, r0 = threadIdx.x / LPR;
+  uint32_t big = 0, small = 0xffffffffu;
+  for (uint32_t r = blockIdx.x * (256 / LPR) + r0; r < a.tokens; r += PLANE_BLOCKS * (256 / LPR)) {
+    const float* p = src + r * stride + sub * 8;
+    const u32x4 v0 = *(const u32x4*)p, v1 = *(const u32x4*)(p + 4);
+    uint32_t m = 0;
+#pragma unroll
+    for (int e = 0; e < 4; e++) m = max(m, max(v0[e] & 0x7fffffffu, v1[e] & 0x7fffffffu));
+#pragma unroll
+    for (int d = LPR / 2; d >= 1; d >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, d, LPR));
+    if (m >= 0x7f800000u) small = 0;
+    else if (m) big = max(big, m), small = min(small, m);
+  }
+#pragma unroll
+  for (int d = 32; d >= 1; d >>= 1) {
+    big = max(big, (uint32_t)__shfl_xor((int)big, d, 64));
+    small = min(small, (uint32_t)__shfl_xor((int)small, d, 64));
+  }
+  if ((threadIdx.x & 63) == 0) rmax[threadIdx.x >> 6] = big, rmin[threadIdx.x >> 6] = small;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    uint32_t* p = part + ((z * a.kv_heads + g) * PLANE_BLOCKS + blockIdx.x) * 2;
+    p[0] = max(max(rmax[0], rmax[1]), max(rmax[2], rmax[3]));
+    p[1] = min(min(rmin[0], rmin[1]), min(rmin[2], rmin[3]));
+  }
+}
+
+// biased exponent of the power of two that brings the largest value (its bits) into [2^14, 2^15)
+__device__ __forceinline__ uint32_t attn_plane_exp(uint32_t bits) {
+  const uint32_t e = 268u - (bits >> 23);
+  return e < 253u ? e : 253u;
+}
+
+// 8 f32 values times s -> their f16 planes
+__device__ __forceinline__ void attn_split8(const float (&v)[8], float s, u32x4& hi, u32x4& lo) {
+  const std::true_type f16{};
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const float x = v[2 * i] * s, y = v[2 * i + 1] * s;
+    hi[i] = pack2(x, y, f16);
+    lo[i] = pack2(x - f16_to_f32((uint16_t)(hi[i] & 0xffffu)), y - f16_to_f32((uint16_t)(hi[i] >> 16)), f16);
+  }
+}
+
+// K (z 0) and V (1) -> f16 [tokens, kv_heads, hi | lo, DP], with each head's inverse scale and flag.
+template <int DP>
+__global__ void __launch_bounds__(256) attn_split_kernel(AttnArgs a, const uint32_t* __restrict__ part,
+                                                         uint16_t* __restrict__ kp, uint16_t* __restrict__ vp,
+                                                         float* __restrict__ inv, uint32_t* __restrict__ flag) {
+  constexpr int LPR = DP / 8;
+  const uint32_t g = blockIdx.y, z = blockIdx.z;
+  const uint32_t* p = part + (z * a.kv_heads + g) * PLANE_BLOCKS * 2;
+  uint32_t big = 0, small = 0xffffffffu;
+#pragma unroll
+  for (uint32_t i = 0; i < PLANE_BLOCKS; i++) big = max(big, p[2 * i]), small = min(small, p[2 * i + 1]);
+  const uint32_t se = attn_plane_exp(big);
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    inv[z * a.kv_heads + g] = __uint_as_float((254u - se) << 23);
+    flag[z * a.kv_heads + g] = small == 0u || (big >> 23) > (small >> 23) + 16u ? 1u : 0u;
+  }
+  const uint32_t r = blockIdx.x * (256 / LPR) + threadIdx.x / LPR, d = threadIdx.x % LPR * 8;
+  if (r >= a.tokens) return;
+  const float* src = (const float*)(z ? a.v : a.k) + r * (size_t)(z ? a.vs : a.ks) + (size_t)g * DP + d;
+  const f32x4 v0 = *(const f32x4*)src, v1 = *(const f32x4*)(src + 4);
+  const float v[8] = {v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
+  u32x4 hi, lo;
+  attn_split8(v, __uint_as_float(se << 23), hi, lo);
+  uint16_t* o = (z ? vp : kp) + ((size_t)r * a.kv_heads + g) * 2 * DP + d;
+  *(u32x4*)o = hi;
+  *(u32x4*)(o + DP) = lo;
+}
+
+// NW waves of 32 queries; K and V plane tiles of 64 keys reach two LDS stages by direct-to-LDS loads, the next tile's
+// during this one's products. Fragment layouts as attn_pp_kernel.
+template <int DP, int NW>
+__global__ void __launch_bounds__(64 * NW, 1) attn_planes_kernel(AttnArgs a, const uint16_t* kp, const uint16_t* vp) {
+  constexpr int NCH = DP / 8, KSH = NCH == 16 ? 0 : 1, ROWB = DP * 2;
+  constexpr int PLANE = ATT_BN * ROWB;     // bytes of one plane of a K or V tile
+  constexpr int STAGE = 4 * PLANE;         // K hi, K lo, V hi, V lo
+  constexpr int RPI = 1024 / ROWB;         // rows per load instruction
+  constexpr int IPP = ATT_BN / RPI;        // load instructions per plane
+  constexpr int IPW = 4 * IPP / NW;        // and per wave and tile
+  static_assert(4 * IPP % NW == 0, "the loads split evenly over the waves");
+  __shared__ __attribute__((aligned(1024))) char lds[2 * STAGE];
+
+  uint32_t qb, h;
+  block_coords(a, qb, h);
+  const uint32_t g = h / a.group;
+  if (a.plane_flag[g] | a.plane_flag[a.kv_heads + g]) return;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c = lane & 31, hf = lane >> 5;
+  const uint32_t q0 = qb * 32 * NW, qw = q0 + 32 * wave, qi = qw + c;
+
+  const uint32_t kv_end = a.causal ? min(a.tokens, q0 + 32 * NW) : a.tokens;
+  const int nt = (int)((kv_end + ATT_BN - 1) / ATT_BN);
+  const uint32_t row_elems = a.kv_heads * 2 * DP, bytes = a.tokens * row_elems * 2;
+  const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc((void*)kp, (short)0, (int)bytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc((void*)vp, (short)0, (int)bytes, 0x00020000);
+  auto swz = [](int r) { return (r >> KSH) & (NCH - 1); };
+  auto issue = [&](int t, int stage) {
+#pragma unroll
+    for (int u = 0; u < IPW; u++) {
+      const int j = wave + NW * u, plane = j / IPP, jj = j % IPP;  // plane: K hi, K lo, V hi, V lo
+      const int row = RPI * jj + lane / NCH, logical = (lane % NCH) ^ swz(row);
+      const uint32_t key = (uint32_t)t * ATT_BN + row;
+      const uint32_t off = key < a.tokens ? (key * row_elems + (g * 2 + (plane & 1)) * DP + logical * 8) * 2 : kAttInvalid;
+      dma16(plane < 2 ? rk : rv, lds + stage * STAGE + plane * PLANE + jj * 1024, off);
+    }
+  };
+  if (nt > 0) issue(0, 0);
+
+  // Q planes: query qi, dims 16 s + 8 hf .. + 7, scaled by the row's own power of two
+  u32x4 qh[DP / 16], ql[DP / 16];
+  float sc;  // scores -> log2 units
+  {
+    float v[DP / 16][8];
+    uint32_t m = 0;
+    static_for<0, DP / 16>([&](auto S) {
+      const float* p = (const float*)a.q + (size_t)qi * a.qs + (size_t)h * DP + 16 * S + 8 * hf;
+      f32x4 v0 = {0, 0, 0, 0}, v1 = {0, 0, 0, 0};
+      if (qi < a.tokens) v0 = *(const f32x4*)p, v1 = *(const f32x4*)(p + 4);
+      static_for<0, 4>([&](auto E) {
+        constexpr int e = E;
+        v[S][e] = v0[e];
+        v[S][4 + e] = v1[e];
+        const uint32_t b0 = __float_as_uint(v0[e]) & 0x7fffffffu, b1 = __float_as_uint(v1[e]) & 0x7fffffffu;
+        m = max(m, max(b0 < 0x7f800000u ? b0 : 0u, b1 < 0x7f800000u ? b1 : 0u));
+      });
+    });
+    m = max(m, (uint32_t)__shfl_xor((int)m, 32, 64));
+    const uint32_t se = attn_plane_exp(m);
+    const float s = __uint_as_float(se << 23);
+    static_for<0, DP / 16>([&](auto S) { attn_split8(v[S], s, qh[S], ql[S]); });
+    sc = a.scale_log2 * __uint_as_float((254u - se) << 23) * a.plane_inv[g];
+  }
+  const VtrLane vl = vtr_lane(lane);
+  // V^T fragment: dims 32 db + c, the lane's 8 keys of 16 s .. (rows of ROWB bytes)
+  auto vfrag = [&](const char* vt, int s, int db) -> u32x4 {
+    const char* t = vt + s * 16 * ROWB + (vl.base1 & 8u);
+    const int r1 = 16 * s + (int)vl.k1, r2 = 16 * s + (int)vl.k2;
+    const char* p1 = t + vl.k1 * ROWB + ((((uint32_t)(4 * db) + vl.cc) ^ (uint32_t)swz(r1)) << 4);
+    const char* p2 = t + vl.k2 * ROWB + ((((uint32_t)(4 * db) + vl.cc) ^ (uint32_t)swz(r2)) << 4);
+    const attn_v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) attn_v4s*)p1);
+    const attn_v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) attn_v4s*)p2);
+    const u32x2 l2 = __builtin_bit_cast(u32x2, lo), h2 = __builtin_bit_cast(u32x2, hi);
+    return u32x4{l2.x, l2.y, h2.x, h2.y};
+  };
+
+  f32x16 o[DP / 32];
+  static_for<0, DP / 32>([&](auto D) { o[D] = f32x16{}; });
+  float m = -__builtin_inff(), l = 0.0f;
+  for (int t = 0; t < nt; t++) {
+    const uint32_t k0 = (uint32_t)t * ATT_BN;
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");  // tile t is in, tile t - 1 is read
+    if (t + 1 < nt) issue(t + 1, (t + 1) & 1);
+    if (a.causal && k0 > qw + 31) continue;
+    const char* ks = lds + (t & 1) * STAGE;
+    const char* vs = ks + 2 * PLANE;
+
+    f32x16 sacc[2] = {f32x16{}, f32x16{}};
+    // fragments one step ahead; the scheduling barriers keep the compiler from reading all of them first (it spills)
+    u32x4 kh[2][2], kl[2][2];
+    auto kread = [&](auto S) {
+      constexpr int s = S;
+      static_for<0, 2>([&](auto B) {
+        const int r = 32 * B + c;
+        const char* p = ks + r * ROWB + (((2 * s + hf) ^ swz(r)) << 4);
+        kh[s & 1][B] = *(const u32x4*)p;
+        kl[s & 1][B] = *(const u32x4*)(p + PLANE);
+      });
+    };
+    kread(std::integral_constant<int, 0>{});
+    static_for<0, DP / 16>([&](auto S) {
+      constexpr int s = S;
+      if constexpr (s + 1 < DP / 16) kread(std::integral_constant<int, s + 1>{});
+      static_for<0, 2>([&](auto B) { sacc[B] = mfma_32x32x16<true>(kl[s & 1][B], qh[s], sacc[B]); });
+      static_for<0, 2>([&](auto B) { sacc[B] = mfma_32x32x16<true>(kh[s & 1][B], ql[s], sacc[B]); });
+      static_for<0, 2>([&](auto B) { sacc[B] = mfma_32x32x16<true>(kh[s & 1][B], qh[s], sacc[B]); });
+      __builtin_amdgcn_sched_barrier(0);
+    });
+
+    if ((k0 + ATT_BN > a.tokens) || (a.causal && k0 + ATT_BN - 1 > qw)) {
+      static_for<0, 32>([&](auto I) {
+        constexpr int i = I, b = i / 16, v = i % 16;
+        const uint32_t key = k0 + 32 * b + 8 * (v / 4) + 4 * hf + (v % 4);
+        if (key >= a.tokens || (a.causal && key > qi)) sacc[b][v] = -__builtin_inff();
+      });
+    }
+    float tmax = sacc[0][0];
+    static_for<1, 32>([&](auto I) { tmax = fmaxf(tmax, sacc[I / 16][I % 16]); });
+    tmax = halves_max(tmax) * sc;  // sc > 0
+    const float mn = fmaxf(m, tmax);
+    // the max moves when some query's rises by more than 1 (log2 units): p 2^14 stays below 2^15, in f16's range
+    const bool rescale = __any(mn > m + 1.0f);
+    const float mref = rescale ? mn : m;
+    const float ms = mref == -__builtin_inff() ? 0.0f : mref;
+    const float alpha = rescale ? __builtin_amdgcn_exp2f(m - ms) : 1.0f;
+    if (rescale) m = mn;
+    float ps = 0.0f;
+    u32x4 ph[4], pl[4];
+    const std::true_type f16{};
+    static_for<0, 4>([&](auto S) {
+      constexpr int s = S;
+      static_for<0, 4>([&](auto J) {
+        constexpr int j = J, i0 = 8 * (s % 2) + 2 * j;
+        const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[s / 2][i0], sc, 14.0f - ms));
+        const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[s / 2][i0 + 1], sc, 14.0f - ms));
+        ps += p0 + p1;
+        const uint32_t w = pack2(p0, p1, f16);
+        ph[s][j] = w;
+        pl[s][j] = pack2(p0 - f16_to_f32((uint16_t)(w & 0xffffu)), p1 - f16_to_f32((uint16_t)(w >> 16)), f16);
+      });
+    });
+    l = __builtin_fmaf(l, alpha, ps);
+    static_for<0, DP / 32>([&](auto D) { o[D] *= alpha; });
+    // step i: keys 16 s .., two blocks of 32 dims
+    constexpr int NPV = 4 * (DP / 64);
+    u32x4 vh[2][2], vo[2][2];
+    auto vread = [&](auto I) {
+      constexpr int i = I, s = i / (DP / 64), d0 = i % (DP / 64) * 2;
+      static_for<0, 2>([&](auto D) {
+        vh[i & 1][D] = vfrag(vs, s, d0 + D);
+        vo[i & 1][D] = vfrag(vs + PLANE, s, d0 + D);
+      });
+    };
+    __builtin_amdgcn_sched_barrier(0);
+    vread(std::integral_constant<int, 0>{});
+    static_for<0, NPV>([&](auto I) {
+      constexpr int i = I, s = i / (DP / 64), d0 = i % (DP / 64) * 2;
+      if constexpr (i + 1 < NPV) vread(std::integral_constant<int, i + 1>{});
+      static_for<0, 2>([&](auto D) { o[d0 + D] = mfma_32x32x16<true>(vo[i & 1][D], ph[s], o[d0 + D]); });
+      static_for<0, 2>([&](auto D) { o[d0 + D] = mfma_32x32x16<true>(vh[i & 1][D], pl[s], o[d0 + D]); });
+      static_for<0, 2>([&](auto D) { o[d0 + D] = mfma_32x32x16<true>(vh[i & 1][D], ph[s], o[d0 + D]); });
+      __builtin_amdgcn_sched_barrier(0);
+    });
+  }
+
+  const float inv = a.plane_inv[a.kv_heads + g] / halves_sum(l);
+  if (qi < a.tokens) {
+    float* O = (float*)a.o + (size_t)qi * a.os + (size_t)h * DP;
+    static_for<0, DP / 32>([&](auto D) {
+      constexpr int db = D;
+      static_for<0, 4>([&](auto G) {
+        constexpr int g4 = G;
+        *(f32x4*)(O + 32 * db + 8 * g4 + 4 * hf) = f32x4{o[db][4 * g4] * inv, o[db][4 * g4 + 1] * inv,
+                                                        o[db][4 * g4 + 2] * inv, o[db][4 * g4 + 3] * inv};
+      });
+    });
+  }
+}
+
 template <class Kern>
 hipError_t launch_attn(Kern kern, const AttnArgs& a, hipStream_t s) {
   hipLaunchKernelGGL(kern, dim3(a.nqb * a.heads), dim3(ATT_NT), 0, s, a);
@@ -1158,10 +1436,54 @@ bool attn_dma_ok(const AttnLaunch& L) {
   return kb < kAttInvalid && vb < kAttInvalid;
 }
 bool attn_ring_path(const AttnLaunch& L) { return L.path == 2; }
+
+// f32 through f16 planes: scratch layout (bytes), 0 where the path does not apply
+struct PlanesLayout {
+  size_t vp, part, inv, flag, bytes;
+};
+bool attn_planes_ok(const AttnLaunch& L, PlanesLayout& p) {
+  if (L.dtype != F32 || (L.dim != 64 && L.dim != 128) || L.path != 0 || L.heads == 0 || L.tokens < PLANES_MIN_TOKENS)
+    return false;
+  const uint64_t plane = (uint64_t)L.tokens * L.kv_heads * 2 * L.dim * 2;
+  if (plane >= kAttInvalid || L.kv_heads > 65535) return false;
+  p.vp = (plane + 255) / 256 * 256;
+  p.part = 2 * p.vp;
+  p.inv = p.part + ((size_t)2 * L.kv_heads * PLANE_BLOCKS * 8 + 255) / 256 * 256;
+  p.flag = p.inv + ((size_t)2 * L.kv_heads * 4 + 255) / 256 * 256;
+  p.bytes = p.flag + (size_t)2 * L.kv_heads * 4;
+  return true;
+}
+
+template <int DP>
+hipError_t launch_planes(AttnArgs a, const AttnLaunch& L, const PlanesLayout& p, hipStream_t s) {
+  char* base = (char*)L.scratch;
+  uint16_t *kp = (uint16_t*)base, *vp = (uint16_t*)(base + p.vp);
+  uint32_t* part = (uint32_t*)(base + p.part);
+  a.plane_inv = (const float*)(base + p.inv);
+  a.plane_flag = (const uint32_t*)(base + p.flag);
+  constexpr uint32_t rows = 256 / (DP / 8);
+  hipLaunchKernelGGL(attn_amax_kernel<DP>, dim3(PLANE_BLOCKS, L.kv_heads, 2), dim3(256), 0, s, a, part);
+  hipLaunchKernelGGL(attn_split_kernel<DP>, dim3((L.tokens + rows - 1) / rows, L.kv_heads, 2), dim3(256), 0, s, a, part,
+                     kp, vp, (float*)(base + p.inv), (uint32_t*)(base + p.flag));
+  // 4 waves (128 queries) per workgroup while the workgroups then still fit one round of the CUs, else 8
+  const uint32_t n4 = (L.tokens + 127) / 128;
+  if ((uint64_t)n4 * L.heads <= 256) {
+    a.nqb = n4;
+    hipLaunchKernelGGL((attn_planes_kernel<DP, 4>), dim3(a.nqb * L.heads), dim3(256), 0, s, a, kp, vp);
+  } else {
+    a.nqb = (L.tokens + 255) / 256;
+    hipLaunchKernelGGL((attn_planes_kernel<DP, 8>), dim3(a.nqb * L.heads), dim3(512), 0, s, a, kp, vp);
+  }
+  a.nqb = (L.tokens + ATT_BM - 1) / ATT_BM;
+  return launch_attn(attn32_kernel<DP>, a, s);  // the flagged heads
+}
 }  // namespace
 
-// Only the ring kernel (WE_ATTN_PATH=ring) stages V^T through scratch; the default kernel reads V as it is.
+// The ring kernel (WE_ATTN_PATH=ring) stages V^T through scratch, f32 attention its planes of K and V (without scratch
+// it runs on the f32 MFMA kernel); the default 16-bit kernel reads K and V as they are.
 size_t attention_scratch_bytes(const AttnLaunch& L) {
+  PlanesLayout p;
+  if (attn_planes_ok(L, p)) return p.bytes;
   if (!attn_dma_ok(L) || !attn_ring_path(L)) return 0;
   const size_t tp = (L.tokens + ATT_BN - 1) / ATT_BN * ATT_BN;
   return (size_t)L.kv_heads * 128 * tp * 2;
@@ -1184,6 +1506,11 @@ hipError_t attention_launch(const AttnLaunch& L, hipStream_t s) {
   a.os = L.out_stride;
   a.scale_log2 = 1.4426950408889634f / sqrtf((float)L.dim);
   a.causal = L.causal;
+  a.plane_inv = nullptr;
+  a.plane_flag = nullptr;
+  a.kv_heads = L.kv_heads;
+  PlanesLayout p;
+  if (L.scratch && attn_planes_ok(L, p)) return L.dim == 64 ? launch_planes<64>(a, L, p, s) : launch_planes<128>(a, L, p, s);
   if (attn_dma_ok(L)) {
     a.nqb = (L.tokens + DMA_BM - 1) / DMA_BM;
     const dim3 grid(a.nqb * L.heads);

@@ -146,6 +146,18 @@ int ensure_scratch(we_ctx* ctx, size_t bytes) {
   return WE_OK;
 }
 
+// The scratch of a path that has another one without it: null, and no error left behind, where it cannot be had (a
+// graph is being captured, the allocation cap or the device is full).
+void* try_scratch(we_ctx* ctx, size_t bytes) {
+  if (bytes <= ctx->scratch_bytes) return ctx->scratch;
+  if (ctx->capturing || (ctx->alloc_cap && ctx->held_bytes + bytes > ctx->alloc_cap)) return nullptr;
+  const std::string before = ctx->err;
+  if (ensure_scratch(ctx, bytes) == WE_OK) return ctx->scratch;
+  ctx->err = before;
+  (void)hipGetLastError();
+  return nullptr;
+}
+
 size_t round_size(size_t bytes) { return ((bytes < 4 ? 4 : bytes) + 255) / 256 * 256; }
 
 // Is [p, p + bytes) inside one device allocation of this context?
@@ -1321,7 +1333,9 @@ int we_attention(we_ctx* ctx, uint32_t tokens, uint32_t heads, uint32_t kv_heads
   we::AttnLaunch L{q, k, v, out, dtype, tokens, heads, kv_heads, dim, (uint32_t)qs, (uint32_t)ks, (uint32_t)vs,
                    (uint32_t)os, causal ? 1 : 0, ctx->tune.attn_path, nullptr};
   const size_t need = we::attention_scratch_bytes(L);
-  if (need) {
+  if (need && dtype == WE_F32) {
+    L.scratch = try_scratch(ctx, need);  // null: the kernel that needs none
+  } else if (need) {
     const int rc = ensure_scratch(ctx, need);
     if (rc) return rc;
     L.scratch = ctx->scratch;
