@@ -1,0 +1,8 @@
+// The general GEMM kernels for f32 activations.
+#include "gemm_general.h"
+
+namespace we {
+hipError_t gemm_general_f32(int w_dtype, const GemmArgs& a, uint32_t splits, int cfg, hipStream_t s) {
+  return launch_w<F32>(w_dtype, a, splits, cfg, s);
+}
+}  // namespace we

@@ -54,46 +54,6 @@ constexpr int kRsrcWord3 = 0x00020000;
 constexpr int kCpolNt = 2;  // buffer-load cache policy: nt (non-temporal)
 }  // namespace
 
-// v_and_or_b32 with the mask in a VGPR and the constant in an SGPR (one instruction; the compiler
-// otherwise splits it into an and and an or with literals)
-__device__ __forceinline__ uint32_t and_or(uint32_t x, uint32_t mask, uint32_t c) {
-  uint32_t r;
-  asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(x), "v"(mask), "s"(c));
-  return r;
-}
-
-// eight nibbles (one word) -> eight f16 in k order, exact (13 VALU ops)
-__device__ __forceinline__ u32x4 int4x8_to_f16(uint32_t w, uint32_t mask) {
-  const uint32_t u = w ^ 0x88888888u;  // q + 8 in [0, 15] per nibble
-  const f16x2 mul = {(_Float16)1.0f, (_Float16)0.0625f};
-  const f16x2 add = {(_Float16)-1032.0f, (_Float16)-72.0f};
-  u32x4 r;
-#pragma unroll
-  for (int p = 0; p < 4; p++) {
-    // byte p of u into bytes 0 and 2: lo half gets nibble 2p at bits 0-3, hi half nibble 2p+1 at bits 4-7
-    const uint32_t sel = (uint32_t)p | (0x0cu << 8) | ((uint32_t)p << 16) | (0x0cu << 24);
-    const uint32_t t = __builtin_amdgcn_perm(u, u, sel);
-    const uint32_t v = and_or(t, mask, 0x64006400u);  // mask 0x00f0000f -> lo: 1024 + u0, hi: 1024 + 16 u1
-    const f16x2 h = __builtin_bit_cast(f16x2, v);
-    const f16x2 q = __builtin_elementwise_fma(h, mul, add);  // lo: u0 - 8, hi: u1 - 8
-    r[p] = __builtin_bit_cast(uint32_t, q);
-  }
-  return r;
-}
-
-// eight nibbles -> eight bf16 in k order, exact (small integers)
-__device__ __forceinline__ u32x4 int4x8_to_bf16(uint32_t w) {
-  u32x4 r;
-#pragma unroll
-  for (int p = 0; p < 4; p++) {
-    const int lo = ((int)(w << (28 - 8 * p))) >> 28;
-    const int hi = ((int)(w << (24 - 8 * p))) >> 28;
-    const uint32_t a = __float_as_uint((float)lo), b = __float_as_uint((float)hi);
-    r[p] = (a >> 16) | (b & 0xffff0000u);
-  }
-  return r;
-}
-
 template <bool IS_F16>
 __device__ __forceinline__ f32x4_t mfma16(u32x4 a, u32x4 b, f32x4_t c) {
   if constexpr (IS_F16)

@@ -60,6 +60,7 @@ struct GemmLaunch {
   // 3x3 convolution input (conv_width > 0, the general kernel only): x is a channel-last image
   // [m / conv_width, conv_width, conv_cin] and k runs over (tap, channel), K = 9 * conv_cin
   uint32_t conv_width, conv_cin;
+  const uint32_t* only_if;  // general kernel: a device word, 0: the launch does nothing (NULL: it runs)
   int x_dtype, w_dtype, y_dtype;
   uint32_t m, n, k;
   float scale;
@@ -72,6 +73,8 @@ struct GemmLaunch {
   // 0, or the weights' K when x holds k / k_wrap planes of k_wrap values per row (f32 activations split into bf16
   // planes): k runs over all planes and the weights are read at k mod k_wrap. Fast path only (k_wrap % 64 == 0).
   uint32_t k_wrap;
+  // k_wrap with two f16 planes: the rows' inverse scales (launch_split_f32_f16x2)
+  const float* row_scale;
   // split-K for small M: K in rsplits slices of rkc, partial sums in scratch (rsplits * m * n f32), then a
   // reduce pass that runs the epilogue; rcfg: the tile configuration the slices were sized for (-1: by shape)
   uint32_t rsplits, rkc;
@@ -92,11 +95,20 @@ struct GemmReducePlan {
   int rcfg;  // the tile configuration the slices are sized for, -1: the launch picks by shape
 };
 GemmReducePlan gemm_reduce_plan(const GemmLaunch& L, uint32_t force_splits = 0);  // force_splits: sweeps
+// The tile shape and K slices by predicted time (M > 64); gemm_reduce_plan below that and with a forced tile shape. The
+// allocation-free entry point keeps gemm_reduce_plan, which says what it accepts, and so does a launch whose planned
+// scratch is not to be had.
+GemmReducePlan gemm_plan(const GemmLaunch& L);
 // The straight-line fast path; hipErrorNotSupported when the operands do not qualify.
 hipError_t gemm_fast_launch(const GemmLaunch& L, hipStream_t stream);
 // Would gemm_fast_launch take this launch (types, alignment, extents)? (Not for split-K partial modes.)
 bool gemm_fast_supported(const GemmLaunch& L);
 int pick_gemm_cfg(uint32_t m, uint32_t n, uint32_t splits);
+
+// The 3x3 convolution of an f32 image with f32 or bf16 weights through two f16 planes per f32 operand (gemm_conv.hip):
+// the scratch it needs, 0 where it does not apply (the general kernel runs), and the launch.
+size_t conv_fast_scratch(const GemmLaunch& L);
+hipError_t conv_fast_launch(const GemmLaunch& L, void* scratch, hipStream_t s);
 
 struct Int4Launch {
   const void* x;
@@ -112,7 +124,15 @@ struct Int4Launch {
   uint32_t x_stride, y_stride, x_offset, y_offset;
   uint32_t flags;
   int path;  // Tuning::int4_path
+  int cfg;   // Tuning::gemm_cfg (the tiled kernel)
+  // split-K of the tiled kernel: K in rsplits slices of rkc, partial sums in scratch (rsplits * m * n f32)
+  uint32_t rsplits, rkc;
+  void* scratch;
 };
+// M > 16, 16-bit x: tiles of gemm_lds.h that share each weight read over 32 to 128 rows (gemm_int4.hip)
+bool int4_gemm_supported(const Int4Launch& L);
+GemmReducePlan int4_gemm_plan(const Int4Launch& L);
+hipError_t int4_gemm_launch(const Int4Launch& L, hipStream_t stream);
 hipError_t int4_launch(const Int4Launch& L, hipStream_t stream);
 
 // peak probes (peak.hip): kinds as WE_PEAK_* of we.h
@@ -150,7 +170,7 @@ void* noalloc_scratch(int device);
 bool noalloc_claim(int device, const void* owner);
 void noalloc_release(int device, const void* owner);
 
-// Can gemm_fast_launch run this GEMM with the fused q/k epilogue (fast path, a head-aligned tile chosen, no
+// Can gemm_fast_launch run this GEMM (planned: rsplits, rcfg) with the fused q/k epilogue (fast path, a head-aligned tile, no
 // split-K plan)? qk_cols / q_cols must be set in L.
 bool gemm_qk_fusable(const GemmLaunch& L);
 
@@ -161,6 +181,15 @@ hipError_t launch_unpack_fp8(const void* packed, size_t n, const float* scale, f
 // whose sum is each value exactly
 hipError_t launch_split_f32_planes(const float* x, uint32_t m, uint32_t k, uint32_t x_stride, uint16_t* out,
                                    hipStream_t s);
+// Rows of f32 or bf16 [m, k] (16-byte aligned, k % 8 == 0) -> `planes` f16 planes of kp values (zeros past k) per row,
+// scaled by a power of two of the row's own; inverse scales to inv[m]. lo_at < 0: the hi plane alone.
+hipError_t launch_split_f32_f16x2(const void* x, int dtype, uint32_t m, uint32_t k, uint32_t x_stride, uint16_t* out,
+                                  uint32_t kp, int planes, int lo_at, int hi_at, float* inv, hipStream_t s);
+// An f32 image [pixels, cin] -> f16 [pixels, 2, cin] (lo, hi) with one scale: its inverse to *inv, and 1 to *flag (else 0)
+// where the pixels' values lie too far apart for one scale; part: 2 kImageParts words
+constexpr uint32_t kImageParts = 512;
+hipError_t launch_image_f16x2(const float* x, uint32_t pixels, uint32_t cin, uint32_t* part, uint16_t* out, float* inv,
+                              uint32_t* flag, hipStream_t s);
 hipError_t launch_dequant_int4(const uint32_t* w, const uint16_t* sc, uint32_t rows, uint32_t k, uint32_t group,
                                float* out, hipStream_t s);
 hipError_t launch_elementwise(int op, size_t n, size_t d, int dtype, const void* a, const void* b, const void* c,

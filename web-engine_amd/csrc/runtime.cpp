@@ -1013,7 +1013,21 @@ int matmul_impl(we_ctx* ctx, const we_matmul_params* p, int x_dtype, const void*
     L.y_offset = p->y_offset;
     L.flags = flags;
     L.path = ctx->tune.int4_path;
-    hipError_t e = we::int4_launch(L, ctx->compute);
+    L.cfg = ctx->tune.gemm_cfg;
+    L.rsplits = 1;
+    hipError_t e;
+    if (we::int4_gemm_supported(L)) {
+      const we::GemmReducePlan rp = we::int4_gemm_plan(L);
+      if (rp.rsplits > 1) {
+        // the partial sums' scratch where it is to be had; else (capturing, allocation cap) full K per tile
+        L.scratch = !noalloc ? try_scratch(ctx, rp.scratch_bytes)
+                    : rp.scratch_bytes <= we::kNoallocScratchBytes ? we::noalloc_scratch(ctx->device) : nullptr;
+        if (L.scratch) L.rsplits = rp.rsplits, L.rkc = rp.rkc;
+      }
+      e = we::int4_gemm_launch(L, ctx->compute);
+    } else {
+      e = we::int4_launch(L, ctx->compute);
+    }
     if (e != hipSuccess) return hip_fail(ctx, e, "int4 launch");
     return WE_OK;
   }
