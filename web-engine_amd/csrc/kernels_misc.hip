@@ -61,6 +61,150 @@ __global__ void __launch_bounds__(256) split_f32_planes_kernel(const float* __re
                                            h[p][4] | (h[p][5] << 16), h[p][6] | (h[p][7] << 16)};
 }
 
+// ------------------------------------------------------------------ f32 operands as two f16 planes
+// v = 2^-e (hi + lo): with the row scaled by 2^e so that its largest finite |v| lies in [2^14, 2^15), hi = f16(v 2^e) and
+// lo = f16(v 2^e - hi) hold v to 2^-23 of itself down to 2^-18 of the row's largest, and to 2^-40 of that largest below.
+// The rounding of the sums in f32 is larger than that (rel. error of 1024 x 6144 x 6144 against f64: see the GEMM's
+// dispatch). inf stays inf with a NaN beside it, as in the three bf16 planes.
+// The biased exponent of the scale for the largest finite |v| (its bits), and the inverse scale.
+__device__ __forceinline__ uint32_t plane_scale_exp(uint32_t amax_bits) {
+  const uint32_t e = 127u + 14u + 127u - (amax_bits >> 23);  // 2^(14 - (exponent - 127)), subnormals as exponent 0
+  return e < 253u ? e : 253u;
+}
+__device__ __forceinline__ uint32_t finite_bits(float v) {
+  const uint32_t b = __float_as_uint(v) & 0x7fffffffu;
+  return b < 0x7f800000u ? b : 0u;
+}
+__device__ __forceinline__ uint32_t block_max256(uint32_t v, uint32_t* red) {
+#pragma unroll
+  for (int d = 32; d >= 1; d >>= 1) v = max(v, (uint32_t)__shfl_xor((int)v, d, 64));
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  __syncthreads();
+  return max(max(red[0], red[1]), max(red[2], red[3]));
+}
+template <int DT>
+__device__ __forceinline__ void load8(const void* p, size_t i, float (&v)[8]) {
+  if constexpr (DT == F32) {
+    const f32x4 a = *(const f32x4*)((const float*)p + i), b = *(const f32x4*)((const float*)p + i + 4);
+#pragma unroll
+    for (int e = 0; e < 4; e++) v[e] = a[e], v[4 + e] = b[e];
+  } else {
+    const u32x4 a = *(const u32x4*)((const uint16_t*)p + i);
+#pragma unroll
+    for (int e = 0; e < 8; e++) v[e] = bf16_to_f32((uint16_t)(a[e / 2] >> (16 * (e & 1))));
+  }
+}
+__device__ __forceinline__ void split_f16x2(const float (&v)[8], float s, u32x4& lo, u32x4& hi) {
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const float a = v[2 * i] * s, b = v[2 * i + 1] * s;
+    const uint32_t ha = f32_to_f16(a), hb = f32_to_f16(b);
+    hi[i] = ha | (hb << 16);
+    lo[i] = (uint32_t)f32_to_f16(a - f16_to_f32((uint16_t)ha)) | ((uint32_t)f32_to_f16(b - f16_to_f32((uint16_t)hb)) << 16);
+  }
+}
+
+// One workgroup per row [k values at src + row * stride] -> f16 planes at out + row * planes * kp, zeros past k: plane
+// lo_at holds lo, plane hi_at hi (lo_at < 0: hi alone). The row's inverse scale goes to inv[row]. Two reads of the row
+// (the second from L2): k % 8 == 0, rows and out 16-byte aligned.
+template <int DT>
+__global__ void __launch_bounds__(256) split_f32_f16x2_kernel(const void* __restrict__ src, uint32_t k, uint32_t stride,
+                                                              uint16_t* __restrict__ out, uint32_t kp, int planes,
+                                                              int lo_at, int hi_at, float* __restrict__ inv) {
+  __shared__ uint32_t red[4];
+  const size_t row = blockIdx.x, base = row * stride;
+  uint32_t m = 0;
+  for (uint32_t i = threadIdx.x * 8; i < k; i += 2048) {
+    float v[8];
+    load8<DT>(src, base + i, v);
+#pragma unroll
+    for (int e = 0; e < 8; e++) m = max(m, finite_bits(v[e]));
+  }
+  const uint32_t se = plane_scale_exp(block_max256(m, red));
+  const float s = __uint_as_float(se << 23);
+  if (threadIdx.x == 0) inv[row] = __uint_as_float((254u - se) << 23);
+  uint16_t* dst = out + row * (size_t)planes * kp;
+  for (uint32_t i = threadIdx.x * 8; i < kp; i += 2048) {
+    float v[8] = {};
+    if (i < k) load8<DT>(src, base + i, v);
+    u32x4 lo, hi;
+    split_f16x2(v, s, lo, hi);
+    *(u32x4*)(dst + (size_t)hi_at * kp + i) = hi;
+    if (lo_at >= 0) *(u32x4*)(dst + (size_t)lo_at * kp + i) = lo;
+  }
+}
+
+hipError_t launch_split_f32_f16x2(const void* x, int dtype, uint32_t m, uint32_t k, uint32_t x_stride, uint16_t* out,
+                                  uint32_t kp, int planes, int lo_at, int hi_at, float* inv, hipStream_t s) {
+  if (m == 0) return hipSuccess;
+  const auto kern = dtype == F32 ? split_f32_f16x2_kernel<F32> : split_f32_f16x2_kernel<BF16>;
+  hipLaunchKernelGGL(kern, dim3(m), dim3(256), 0, s, x, k, x_stride, out, kp, planes, lo_at, hi_at, inv);
+  return hipGetLastError();
+}
+
+// An f32 image (cin values per pixel, cin % 8 == 0) -> per pixel the lo and the hi plane of its cin values, one scale for
+// the whole image (a convolution's sums mix pixels): the largest pixel maximum and the smallest nonzero one per workgroup
+// into part, then the split, whose workgroups each reduce part. The planes hold a value to 2^-40 of the image's largest: an
+// image with a pixel whose largest value lies below 2^-16 of that is flagged, and the general kernel takes it.
+__global__ void __launch_bounds__(256) image_amax_kernel(const float* __restrict__ x, uint32_t pixels, uint32_t cin,
+                                                         uint32_t* __restrict__ part) {
+  __shared__ uint32_t red[4], red2[4];
+  const uint32_t sub = threadIdx.x & 15u;  // 16 lanes per pixel
+  uint32_t big = 0, inv_small = 0;         // inv_small: the complement of the smallest, so both reduce by max
+  for (uint32_t p = blockIdx.x * 16 + (threadIdx.x >> 4); p < pixels; p += kImageParts * 16) {
+    uint32_t m = 0;
+    for (uint32_t c = sub * 8; c < cin; c += 128) {
+      float v[8];
+      load8<F32>(x, (size_t)p * cin + c, v);
+#pragma unroll
+      for (int e = 0; e < 8; e++) m = max(m, finite_bits(v[e]));
+    }
+#pragma unroll
+    for (int d = 8; d >= 1; d >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, d, 16));
+    if (m) big = max(big, m), inv_small = max(inv_small, ~m);
+  }
+  big = block_max256(big, red);
+  inv_small = block_max256(inv_small, red2);
+  if (threadIdx.x == 0) {
+    part[blockIdx.x] = big;
+    part[kImageParts + blockIdx.x] = inv_small;
+  }
+}
+__global__ void __launch_bounds__(256) image_f16x2_kernel(const float* __restrict__ x, size_t n, uint32_t cin,
+                                                          const uint32_t* __restrict__ part, uint16_t* __restrict__ out,
+                                                          float* __restrict__ inv, uint32_t* __restrict__ flag) {
+  __shared__ uint32_t red[4], red2[4];
+  static_assert(kImageParts == 512, "two parts per thread");
+  const uint32_t t = threadIdx.x, big = block_max256(max(part[t], part[256 + t]), red);
+  if (blockIdx.x == 0) {  // workgroup-uniform
+    const uint32_t small = ~block_max256(max(part[kImageParts + t], part[kImageParts + 256 + t]), red2);
+    if (t == 0) *flag = (big >> 23) > (small >> 23) + 16u ? 1u : 0u;
+  }
+  const uint32_t se = plane_scale_exp(big);
+  const float s = __uint_as_float(se << 23);
+  if (blockIdx.x == 0 && t == 0) *inv = __uint_as_float((254u - se) << 23);
+  const size_t i = ((size_t)blockIdx.x * 256 + t) * 8;
+  if (i >= n) return;
+  float v[8];
+  load8<F32>(x, i, v);
+  u32x4 lo, hi;
+  split_f16x2(v, s, lo, hi);
+  uint16_t* dst = out + i / cin * 2 * cin + i % cin;
+  *(u32x4*)dst = lo;
+  *(u32x4*)(dst + cin) = hi;
+}
+
+hipError_t launch_image_f16x2(const float* x, uint32_t pixels, uint32_t cin, uint32_t* part, uint16_t* out, float* inv,
+                              uint32_t* flag, hipStream_t s) {
+  const size_t n = (size_t)pixels * cin;
+  hipLaunchKernelGGL(image_amax_kernel, dim3(kImageParts), dim3(256), 0, s, x, pixels, cin, part);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(image_f16x2_kernel, dim3((unsigned)((n / 8 + 255) / 256)), dim3(256), 0, s, x, n, cin, part, out, inv,
+                     flag);
+  return hipGetLastError();
+}
+
 hipError_t launch_split_f32_planes(const float* x, uint32_t m, uint32_t k, uint32_t x_stride, uint16_t* out,
                                    hipStream_t s) {
   const size_t n = (size_t)m * (k / 8);

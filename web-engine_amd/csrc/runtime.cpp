@@ -1038,26 +1038,41 @@ int matmul_impl(we_ctx* ctx, const we_matmul_params* p, int x_dtype, const void*
   if (rc) return rc;
   we::GemmLaunch L;
   fill_gemm(L, ctx->tune, p, x_dtype, x, w_dtype, w, y_dtype, y, bias, flags, gate, res, mul, splits, kc);
-  // f32 activations (the reference's own dtype) on the fast path: x is split once into three exact bf16 planes along K
-  // in scratch ([M, 3K]: hi | mid | lo, summing to x exactly) and the fast kernel runs one GEMM over 3K with the
-  // weights read at k mod K, so each product keeps all 24 bits of x. Taken when the fast kernel accepts the planes
+  // f32 activations (the reference's own dtype) on the fast path: x is split once into 16-bit planes along K in scratch and
+  // the fast kernel runs one GEMM over all planes with the weights read at k mod K. fp8 weights (exact in f16): two f16
+  // planes [M, 2K] (lo | hi), each row scaled by a power of two of its own, which hold x to 2^-23; bf16 weights, whose
+  // range f16 lacks: three bf16 planes [M, 3K] (hi | mid | lo) that sum to x exactly. A third fewer products and fewer f32
+  // roundings: 1024 x 6144 x 6144 fp8 error against f64 9.1e-7 -> 4.2e-7. Taken when the fast kernel accepts the planes
   // (fp8 or bf16 weights, K a multiple of 64, aligned rows); otherwise, for the allocation-free entry point and for
   // split-K partial modes, the general kernel splits x into the same planes tile by tile.
-  size_t plane_bytes = 0;
+  if (L.conv_width && !noalloc) {
+    const size_t need = we::conv_fast_scratch(L);
+    void* scratch = need ? try_scratch(ctx, need) : nullptr;
+    if (scratch) {
+      const hipError_t e = we::conv_fast_launch(L, scratch, ctx->compute);
+      return e == hipSuccess ? WE_OK : hip_fail(ctx, e, "convolution launch");
+    }
+  }
+  size_t plane_bytes = 0, scale_at = 0;
   if (x_dtype == WE_F32 && !noalloc && !split && !L.generic && !L.conv_width && p->k % 64 == 0 &&
       (w_dtype == WE_FP8_E4M3 || w_dtype == WE_BF16) && (uintptr_t)x % 16 == 0 &&
       (uint64_t)p->m * p->k * 3 <= (1ull << 30)) {
     we::GemmLaunch P = L;
     P.x = (const void*)(uintptr_t)256;  // placeholder with the scratch's alignment, for the check
-    P.x_dtype = WE_BF16;
-    P.k = 3 * p->k;
+    const uint32_t planes = w_dtype == WE_FP8_E4M3 ? 2 : 3;
+    P.x_dtype = planes == 2 ? WE_F16 : WE_BF16;
+    P.k = planes * p->k;
     P.kc = P.k;
     P.k_wrap = p->k;
-    P.x_stride = 3 * p->k;
+    P.x_stride = planes * p->k;
     P.x_offset = 0;
     if (we::gemm_fast_supported(P)) {
       L = P;
-      plane_bytes = ((uint64_t)p->m * 3 * p->k * 2 + 255) / 256 * 256;
+      plane_bytes = ((uint64_t)p->m * planes * p->k * 2 + 255) / 256 * 256;
+      if (planes == 2) {
+        scale_at = plane_bytes;
+        plane_bytes += ((uint64_t)p->m * 4 + 255) / 256 * 256;
+      }
     }
   }
   bool qk_fused = false;
@@ -1084,8 +1099,16 @@ int matmul_impl(we_ctx* ctx, const we_matmul_params* p, int x_dtype, const void*
     const int rc = ensure_scratch(ctx, plane_bytes + (rp.rsplits > 1 ? rp.scratch_bytes : 0));
     if (rc) return rc;
     L.x = ctx->scratch;
-    const hipError_t e = we::launch_split_f32_planes((const float*)x + p->x_offset, p->m, p->k, p->x_stride,
-                                                     (uint16_t*)ctx->scratch, ctx->compute);
+    const float* xs = (const float*)x + p->x_offset;
+    hipError_t e;
+    if (scale_at) {
+      float* inv = (float*)((char*)ctx->scratch + scale_at);
+      L.row_scale = inv;
+      e = we::launch_split_f32_f16x2(xs, WE_F32, p->m, p->k, p->x_stride, (uint16_t*)ctx->scratch, p->k, 2, 0, 1, inv,
+                                     ctx->compute);
+    } else {
+      e = we::launch_split_f32_planes(xs, p->m, p->k, p->x_stride, (uint16_t*)ctx->scratch, ctx->compute);
+    }
     if (e != hipSuccess) return hip_fail(ctx, e, "f32 plane split launch");
     if (rp.rsplits > 1) {
       L.scratch = (char*)ctx->scratch + plane_bytes;
