@@ -85,6 +85,12 @@ uint32_t cfg_bn(int cfg) {
                                                                : 64;
 }
 
+// the tile shape of a launch: forced, planned, or by shape
+int launch_cfg_of(const GemmLaunch& L) {
+  const uint32_t splits = L.rsplits > 1 ? L.rsplits : L.splits < 1 ? 1 : L.splits;
+  return L.cfg >= 0 ? L.cfg : L.rcfg >= 0 ? L.rcfg : pick_fast_cfg(L.m, L.n, splits, L.w_dtype == FP8);
+}
+
 }  // namespace
 
 GemmReducePlan gemm_reduce_plan(const GemmLaunch& L, uint32_t force_splits) {
@@ -135,13 +141,72 @@ GemmReducePlan gemm_reduce_plan(const GemmLaunch& L, uint32_t force_splits) {
   return p;
 }
 
+namespace {
+
+bool qk_fusable_cfg(int cfg) { return cfg == GEMM_CFG_256x128 || cfg == GEMM_CFG_128x128; }
+
+// Predicted time of a launch, in us: `launch`, then rounds of tiles (a full round 1; the last, partly filled one part +
+// part_f * its fraction: the chip runs at its power limit, so tiles run faster when fewer CUs are busy), each tile `block`
+// per 64 k and `tile` once, and the split-K partial sums' bytes. Fitted to a sweep of tile shapes and slice counts over 37
+// shapes of M 65 .. 4096, N 1040 .. 18944, K 2048 .. 32768 (rms error 6%): against pick_fast_cfg and gemm_reduce_plan the
+// choice gains 12% (fp8 weights), 26% (f16 planes of f32) and 10% (16-bit weights) in the mean over those shapes.
+// 700 x 3072 x 12288 fp8 96.6 -> 67.2 us (256 x 256, 6 slices), 1500 x 3072 x 12288 151 -> 107, 300 x 18000 x 2048
+// 55 -> 40 (128 x 128), 128 x 3072 x 12288 36 -> 26 (64 x 64, 8 slices).
+struct CostModel {
+  double launch, part[2], part_f[2], reduce, reduce_mb;  // part: one, several workgroups per CU
+  double block[6], tile[6];                              // by GemmCfgId
+};
+constexpr CostModel kCostFp8 = {7.2, {0.80, 0.46}, {0.147, 0.494}, 0.3, 0.293,
+                                {1.315, 0.912, 1.026, 0.630, 0, 1.241}, {4.5, 2.7, 1.4, 0.0, 0, 2.0}};
+constexpr CostModel kCostPlanes = {4.7, {0.767, 0.406}, {0.203, 0.658}, 0.0, 0.347,
+                                   {1.436, 0.971, 1.008, 0.666, 0, 1.255}, {1.2, 0.1, 0.9, 0.0, 0, 1.0}};
+constexpr CostModel kCost16 = {8.5, {0.874, 0.648}, {0.142, 0.234}, 0.4, 0.254,
+                               {1.498, 0.898, 0.700, 0.456, 0, 1.186}, {4.0, 2.4, 1.2, 5.0, 0, 3.0}};
+
+}  // namespace
+
+GemmReducePlan gemm_plan(const GemmLaunch& L) {
+  if (L.cfg >= 0 || L.m <= 64 || L.n == 0 || L.generic || L.splits > 1 || (L.flags & WE_EPI_SPLIT_K_BIT) || L.k < 512 ||
+      !fast_supported(L, L.k))
+    return gemm_reduce_plan(L);
+  const bool w8 = L.w_dtype == FP8;
+  const CostModel& c = !w8 ? kCost16 : L.k_wrap ? kCostPlanes : kCostFp8;
+  // workgroups per CU by their LDS: 64 x 64 36 or 48 KB, 128 x 128 72 or 96 KB
+  const uint32_t per_cu[6] = {1, 1, w8 ? 2u : 1u, w8 ? 4u : 3u, 1, 1};
+  GemmReducePlan best{1, L.k, 0, GEMM_CFG_128x128};
+  double best_us = 1e30;
+  for (const int cfg : {GEMM_CFG_256x256, GEMM_CFG_256x192, GEMM_CFG_256x128, GEMM_CFG_128x128, GEMM_CFG_64x64}) {
+    if (cfg_bm(cfg) == 256 && L.m < 256) continue;
+    const uint64_t tiles = (uint64_t)((L.m + cfg_bm(cfg) - 1) / cfg_bm(cfg)) * ((L.n + cfg_bn(cfg) - 1) / cfg_bn(cfg));
+    const uint64_t slots = (uint64_t)kCUs * per_cu[cfg];
+    const int several = per_cu[cfg] > 1 || cfg == GEMM_CFG_128x128;
+    // slices only where the tiles fill at most half of the CUs (128 x 128: twice that), as swept
+    const uint32_t most = tiles * 2 <= kCUs * (cfg == GEMM_CFG_128x128 ? 2u : 1u) ? std::min(8u, L.k / 256) : 1u;
+    for (uint32_t rs = 1; rs <= most; rs++) {
+      const uint32_t kc = (L.k + rs * BK - 1) / (rs * BK) * BK;
+      const uint32_t slices = (L.k + kc - 1) / kc;
+      if (slices != rs) continue;
+      const uint64_t full = tiles * slices / slots, rest = tiles * slices % slots;
+      const double rounds = (double)full + (rest ? c.part[several] + c.part_f[several] * (double)rest / (double)slots : 0.0);
+      double us = c.launch + rounds * ((double)((kc + BK - 1) / BK) * c.block[cfg] + c.tile[cfg]);
+      if (slices > 1) us += c.reduce + c.reduce_mb * 4e-6 * L.m * (double)L.n * slices;
+      // q / k norm and RoPE outside the epilogue: a pass over those columns
+      if (L.qk_cols && (slices > 1 || !qk_fusable_cfg(cfg))) us += 4.0 + 4.0 * L.m * (double)L.qk_cols / 3e6;
+      if (us < best_us) {
+        best_us = us;
+        best = GemmReducePlan{slices, slices > 1 ? kc : L.k, slices > 1 ? (size_t)slices * L.m * L.n * 4 : 0, cfg};
+      }
+    }
+  }
+  return best;
+}
+
 bool gemm_qk_fusable(const GemmLaunch& L) {
-  if (L.generic || L.splits > 1 || L.flags & ~WE_EPI_BIAS_BIT || L.mul || L.gate || L.res) return false;
+  if (L.generic || L.splits > 1 || L.rsplits > 1 || L.flags & ~WE_EPI_BIAS_BIT || L.mul || L.gate || L.res) return false;
   if (L.y_dtype == F32 || !fast_supported(L, L.k)) return false;
-  if (gemm_reduce_plan(L, 0).rsplits > 1) return false;
-  const int cfg = L.cfg >= 0 ? L.cfg : pick_fast_cfg(L.m, L.n, 1, L.w_dtype == FP8);
+  const int cfg = launch_cfg_of(L);
   // head-aligned tiles with 64-column waves outside the ping-pong kernels: 256 x 128 (4 x 2), 128 x 128 (2 x 2)
-  if (cfg != GEMM_CFG_256x128 && cfg != GEMM_CFG_128x128) return false;
+  if (!qk_fusable_cfg(cfg)) return false;
   const uint32_t bn = cfg_bn(cfg);
   return L.qk_cols % bn == 0 && L.q_cols % bn == 0 && L.qk_cols <= L.n && (L.y_stride % 4) == 0 &&
          (L.y_offset % 4) == 0 && ((uintptr_t)L.y % 16) == 0 && ((uintptr_t)L.qk_norm_q % 16) == 0 &&
@@ -215,9 +280,7 @@ hipError_t gemm_fast_launch(const GemmLaunch& L, hipStream_t stream) {
     a.part = (float*)L.scratch;
     a.rsplits = splits;
   }
-  const int cfg = L.cfg >= 0                ? L.cfg
-                  : reduce && L.rcfg >= 0 ? L.rcfg
-                                          : pick_fast_cfg(L.m, L.n, splits, L.w_dtype == FP8);
+  const int cfg = launch_cfg_of(L);
   const int rx = L.reduce_xcd;
   if (f16) {
     if (L.w_dtype == FP8) return gemm_lds_f16_fp8(a, splits, cfg, rx, stream);

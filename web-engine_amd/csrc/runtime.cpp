@@ -1075,8 +1075,8 @@ int matmul_impl(we_ctx* ctx, const we_matmul_params* p, int x_dtype, const void*
       }
     }
   }
-  bool qk_fused = false;
-  if (qk && qk->q_heads + qk->k_heads) {
+  const bool has_qk = qk && qk->q_heads + qk->k_heads;
+  if (has_qk) {
     L.qk_cols = (qk->q_heads + qk->k_heads) * 128;
     L.q_cols = qk->q_heads * 128;
     L.qk_rope_from = qk->rope_from;
@@ -1086,57 +1086,57 @@ int matmul_impl(we_ctx* ctx, const we_matmul_params* p, int x_dtype, const void*
     L.qk_norm_k = qk->norm_k;
     L.qk_cos = qk->cos_t;
     L.qk_sin = qk->sin_t;
-    qk_fused = we::gemm_qk_fusable(L);
-    if (!qk_fused) L.qk_cols = L.q_cols = 0;  // the plain GEMM, then the q/k pass below
   }
   we::GemmReducePlan rp{1, L.k, 0, -1};
-  if (ctx->tune.gemm_splitk != 0) {  // 0: split-K off; n > 0: n slices (sweeps)
-    const uint32_t force = ctx->tune.gemm_splitk > 0 ? (uint32_t)ctx->tune.gemm_splitk : 0u;
-    rp = we::gemm_reduce_plan(L, force);
+  char* scratch = nullptr;  // the planes of x (plane_bytes), then the split-K partial sums
+  if (ctx->tune.gemm_splitk > 0) {  // that many slices (sweeps)
+    rp = we::gemm_reduce_plan(L, (uint32_t)ctx->tune.gemm_splitk);
+  } else if (ctx->tune.gemm_splitk < 0) {
+    rp = noalloc ? we::gemm_reduce_plan(L) : we::gemm_plan(L);
+    if (!noalloc && rp.rsplits > 1) {
+      scratch = (char*)try_scratch(ctx, plane_bytes + rp.scratch_bytes);
+      if (!scratch) rp = we::gemm_reduce_plan(L);
+    }
+  }
+  const size_t part_bytes = rp.rsplits > 1 ? rp.scratch_bytes : 0;
+  if (!scratch && plane_bytes + part_bytes) {
+    if (noalloc) {
+      // the device's fixed scratch array: no allocation, a hard size limit
+      if (part_bytes > we::kNoallocScratchBytes)
+        return fail(ctx, WE_EINVAL,
+                    "this GEMM (M %u, N %u, K %u) needs %zu bytes of split-K scratch; the allocation-free entry "
+                    "point has %zu (use we_matmul)",
+                    p->m, p->n, p->k, part_bytes, we::kNoallocScratchBytes);
+      scratch = (char*)we::noalloc_scratch(ctx->device);
+      if (!scratch) return fail(ctx, WE_EHIP, "allocation-free scratch of device %d is not set up", ctx->device);
+    } else {
+      const int rc = ensure_scratch(ctx, plane_bytes + part_bytes);
+      if (rc) return rc;
+      scratch = (char*)ctx->scratch;
+    }
   }
   if (plane_bytes) {
-    // scratch: the planes of x, then the split-K partial sums (if any)
-    const int rc = ensure_scratch(ctx, plane_bytes + (rp.rsplits > 1 ? rp.scratch_bytes : 0));
-    if (rc) return rc;
-    L.x = ctx->scratch;
+    L.x = scratch;
     const float* xs = (const float*)x + p->x_offset;
     hipError_t e;
     if (scale_at) {
-      float* inv = (float*)((char*)ctx->scratch + scale_at);
+      float* inv = (float*)(scratch + scale_at);
       L.row_scale = inv;
-      e = we::launch_split_f32_f16x2(xs, WE_F32, p->m, p->k, p->x_stride, (uint16_t*)ctx->scratch, p->k, 2, 0, 1, inv,
+      e = we::launch_split_f32_f16x2(xs, WE_F32, p->m, p->k, p->x_stride, (uint16_t*)scratch, p->k, 2, 0, 1, inv,
                                      ctx->compute);
     } else {
-      e = we::launch_split_f32_planes(xs, p->m, p->k, p->x_stride, (uint16_t*)ctx->scratch, ctx->compute);
+      e = we::launch_split_f32_planes(xs, p->m, p->k, p->x_stride, (uint16_t*)scratch, ctx->compute);
     }
     if (e != hipSuccess) return hip_fail(ctx, e, "f32 plane split launch");
-    if (rp.rsplits > 1) {
-      L.scratch = (char*)ctx->scratch + plane_bytes;
-      L.rsplits = rp.rsplits;
-      L.rkc = rp.rkc;
-      L.rcfg = rp.rcfg;
-    }
-  } else {
-    if (rp.rsplits > 1) {
-      if (noalloc) {
-        // the device's fixed scratch array: no allocation, a hard size limit
-        if (rp.scratch_bytes > we::kNoallocScratchBytes)
-          return fail(ctx, WE_EINVAL,
-                      "this GEMM (M %u, N %u, K %u) needs %zu bytes of split-K scratch; the allocation-free entry "
-                      "point has %zu (use we_matmul)",
-                      p->m, p->n, p->k, rp.scratch_bytes, we::kNoallocScratchBytes);
-        L.scratch = we::noalloc_scratch(ctx->device);
-        if (!L.scratch) return fail(ctx, WE_EHIP, "allocation-free scratch of device %d is not set up", ctx->device);
-      } else {
-        const int rc = ensure_scratch(ctx, rp.scratch_bytes);
-        if (rc) return rc;
-        L.scratch = ctx->scratch;
-      }
-      L.rsplits = rp.rsplits;
-      L.rkc = rp.rkc;
-      L.rcfg = rp.rcfg;
-    }
   }
+  if (part_bytes) {
+    L.scratch = scratch + plane_bytes;
+    L.rsplits = rp.rsplits;
+    L.rkc = rp.rkc;
+  }
+  L.rcfg = rp.rcfg;
+  const bool qk_fused = has_qk && we::gemm_qk_fusable(L);
+  if (!qk_fused) L.qk_cols = L.q_cols = 0;  // the plain GEMM, then the q/k pass below
   hipError_t e = we::gemm_launch(L, ctx->compute);
   if (e != hipSuccess) return hip_fail(ctx, e, "gemm launch");
   if (qk && !qk_fused) {
