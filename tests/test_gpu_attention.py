@@ -197,3 +197,39 @@ def test_tiny_and_block_edge_token_counts(graph, tokens, causal, dtype):
         got = run(graph, q, k, v, shape, dtype)
         want = O.attention(qv, kv, vv, tokens, heads, kv_heads, dim, causal)
         assert O.rel_error(got, want) < 1e-2
+
+
+@pytest.mark.parametrize("tokens,heads,kv_heads,dim,causal", [
+    (160, 4, 2, 128, False), (193, 3, 1, 64, True), (257, 4, 4, 128, True), (600, 64, 8, 64, False), (400, 72, 8, 128, True)])
+def test_f32_planes(graph, tune, tokens, heads, kv_heads, dim, causal):
+    """f32 through f16 planes (4 and 8 waves per workgroup, ragged tiles, causal, GQA), values down to 2^-14 of their head's
+    largest, against the oracle at the reference's 1e-5 bar and against the f32 MFMA kernel. One kv head's V is scaled up by
+    2^100 and back: the planes' powers of two are exact."""
+    q, k, v = lcg_random(tokens, [tokens * heads * dim, tokens * kv_heads * dim, tokens * kv_heads * dim])
+    k.reshape(tokens, kv_heads, dim)[3] *= np.float32(2.0 ** -14)
+    shape = we.AttentionShape(tokens, heads, kv_heads, dim, causal=causal)
+    got = run(graph, q, k, v, shape, we.F32)
+    assert np.abs(got - O.attention(q, k, v, tokens, heads, kv_heads, dim, causal)).max() < 1e-5
+    big = run(graph, q, k, v * np.float32(2.0 ** 100), shape, we.F32)
+    assert np.array_equal(big * 2.0 ** -100, got)
+    tune(attn_path=1)
+    assert np.abs(got - run(graph, q, k, v, shape, we.F32)).max() < 4e-6
+
+
+def test_f32_planes_leave_wide_heads_to_the_f32_kernel(graph, tune):
+    """Heads the planes cannot hold (a row 2^-20 of the largest, the lowest float as a padding value, an inf) are those of
+    the f32 MFMA kernel bit for bit; the other kv heads match the oracle."""
+    tokens, heads, kv_heads, dim = 200, 8, 4, 128
+    q, k, v = lcg_random(21, [tokens * heads * dim, tokens * kv_heads * dim, tokens * kv_heads * dim])
+    clean = O.attention(q, k, v, tokens, heads, kv_heads, dim, True).reshape(tokens, heads, dim)
+    v3, k3 = v.reshape(tokens, kv_heads, dim), k.reshape(tokens, kv_heads, dim)
+    k3[5, 0] *= np.float32(2.0 ** -20)
+    v3[-1, 1] = np.finfo(np.float32).min
+    v3[-1, 2, 7] = np.inf
+    shape = we.AttentionShape(tokens, heads, kv_heads, dim, causal=True)
+    got = run(graph, q, k, v, shape, we.F32).reshape(tokens, heads, dim)
+    tune(attn_path=1)
+    f32 = run(graph, q, k, v, shape, we.F32).reshape(tokens, heads, dim)
+    assert np.array_equal(got[:, :6], f32[:, :6], equal_nan=True)
+    assert np.abs(got[:-1, 2:4] - clean[:-1, 2:4]).max() < 1e-5  # every query but the last sees none of the padding
+    assert np.abs(got[:, 6:] - clean[:, 6:]).max() < 1e-5

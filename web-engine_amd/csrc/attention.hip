@@ -6,7 +6,7 @@
 // token's, so q, k and v can be column slices of one fused QKV projection output.
 //
 // Work split: a wave owns 32 queries of one head and walks the keys in tiles of 64 shared through LDS with
-// the other waves of its workgroup. Four kernels:
+// the other waves of its workgroup. The kernels:
 //   * attn16_kernel / attn32_kernel: any head dim up to 128; 4 waves (128 queries), tiles staged through
 //     registers.
 //   * attn_pp_kernel (head dim 128, 16-bit, the default there): 8 waves (256 queries); K and V tiles
@@ -30,8 +30,8 @@
 //   * K rows and V^T rows are XOR-swizzled by 16-byte chunk so the MFMA operand reads are bank-conflict free.
 //   * LDS is double-buffered: the next tile's loads are in flight during this tile's MFMAs, then stored to
 //     the other buffer; one barrier per tile.
-// f32 kernel (reference f32 API, 32x32x2 f32 MFMA, exact f32 products): same work split, a single LDS
-// buffer, P kept in f32.
+// f32: attn_planes_kernel (head dims 64 and 128, 160 tokens or more: two f16 planes per operand on the 32x32x16 f16 MFMA),
+// and attn32_kernel (32x32x2 f32 MFMA, exact f32 products, a single LDS buffer, P kept in f32) for the rest.
 #include <cstdlib>
 #include <cstring>
 
@@ -1266,14 +1266,19 @@ __global__ void __launch_bounds__(64 * NW, 1) attn_planes_kernel(AttnArgs a, con
   const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc((void*)kp, (short)0, (int)bytes, 0x00020000);
   const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc((void*)vp, (short)0, (int)bytes, 0x00020000);
   auto swz = [](int r) { return (r >> KSH) & (NCH - 1); };
+  // Load u of a wave fills rows RPI wave + RPI NW (u % PPW) .. of plane u / PPW (K hi, K lo, V hi, V lo). RPI NW is a multiple
+  // of 16, so a lane's swizzled chunk is the same in every load and its offsets differ by uniform steps. Keys past the last
+  // token lie past the buffer's end and load zeros.
+  constexpr int PPW = IPP / NW;
+  static_assert(PPW >= 1 && (RPI * NW) % 16 == 0, "whole loads per plane, one swizzled chunk per lane");
+  const uint32_t lrow = RPI * wave + lane / NCH;
+  const uint32_t lane_off = (lrow * row_elems + g * 2 * DP + ((lane % NCH) ^ swz((int)lrow)) * 8) * 2;
   auto issue = [&](int t, int stage) {
 #pragma unroll
     for (int u = 0; u < IPW; u++) {
-      const int j = wave + NW * u, plane = j / IPP, jj = j % IPP;  // plane: K hi, K lo, V hi, V lo
-      const int row = RPI * jj + lane / NCH, logical = (lane % NCH) ^ swz(row);
-      const uint32_t key = (uint32_t)t * ATT_BN + row;
-      const uint32_t off = key < a.tokens ? (key * row_elems + (g * 2 + (plane & 1)) * DP + logical * 8) * 2 : kAttInvalid;
-      dma16(plane < 2 ? rk : rv, lds + stage * STAGE + plane * PLANE + jj * 1024, off);
+      const int plane = u / PPW, ju = u % PPW;
+      const uint32_t step = ((uint32_t)(t * ATT_BN + RPI * NW * ju) * row_elems + (plane & 1) * DP) * 2;
+      dma16(plane < 2 ? rk : rv, lds + stage * STAGE + plane * PLANE + (wave + NW * ju) * 1024, lane_off + step);
     }
   };
   if (nt > 0) issue(0, 0);
@@ -1303,12 +1308,15 @@ __global__ void __launch_bounds__(64 * NW, 1) attn_planes_kernel(AttnArgs a, con
     sc = a.scale_log2 * __uint_as_float((254u - se) << 23) * a.plane_inv[g];
   }
   const VtrLane vl = vtr_lane(lane);
-  // V^T fragment: dims 32 db + c, the lane's 8 keys of 16 s .. (rows of ROWB bytes)
-  auto vfrag = [&](const char* vt, int s, int db) -> u32x4 {
-    const char* t = vt + s * 16 * ROWB + (vl.base1 & 8u);
-    const int r1 = 16 * s + (int)vl.k1, r2 = 16 * s + (int)vl.k2;
-    const char* p1 = t + vl.k1 * ROWB + ((((uint32_t)(4 * db) + vl.cc) ^ (uint32_t)swz(r1)) << 4);
-    const char* p2 = t + vl.k2 * ROWB + ((((uint32_t)(4 * db) + vl.cc) ^ (uint32_t)swz(r2)) << 4);
+  // V^T fragment: dims 32 db + c, the lane's 8 keys of 16 s .. (rows of ROWB bytes). The chunk index (4 db + cc) ^ swz(key)
+  // is 4 db ^ (cc ^ swz(key)), and swz does not see the 16 s: one base per read, the block by an XOR
+  const uint32_t vb1 = vl.k1 * ROWB + ((vl.cc ^ (uint32_t)swz((int)vl.k1)) << 4) + (vl.base1 & 8u);
+  // (the second read's key is 8 further: swz differs in one bit)
+  constexpr uint32_t X2 = NCH == 16 ? 8u << 4 : 4u << 4;
+  const uint32_t kb = c * ROWB + ((hf ^ swz(c)) << 4);  // K row c (32 b: the same swizzle), dims 16 s: chunk 2 s + hf
+  auto vfrag = [&](uint32_t v1, int plane, int s, int db) -> u32x4 {
+    const char* p1 = lds + ((v1 ^ (uint32_t)(db << 6)) + plane * PLANE + s * 16 * ROWB);
+    const char* p2 = lds + ((v1 ^ (uint32_t)(db << 6) ^ X2) + plane * PLANE + (s * 16 + 8) * ROWB);
     const attn_v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) attn_v4s*)p1);
     const attn_v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) attn_v4s*)p2);
     const u32x2 l2 = __builtin_bit_cast(u32x2, lo), h2 = __builtin_bit_cast(u32x2, hi);
@@ -1323,28 +1331,28 @@ __global__ void __launch_bounds__(64 * NW, 1) attn_planes_kernel(AttnArgs a, con
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");  // tile t is in, tile t - 1 is read
     if (t + 1 < nt) issue(t + 1, (t + 1) & 1);
     if (a.causal && k0 > qw + 31) continue;
-    const char* ks = lds + (t & 1) * STAGE;
-    const char* vs = ks + 2 * PLANE;
+    // this tile's bases (a stage is a multiple of what the XORs touch), opaque so that the compiler does not keep every
+    // XORed address in a register across tiles
+    uint32_t kt = kb + (uint32_t)(t & 1) * STAGE, vt = vb1 + (uint32_t)(t & 1) * STAGE + 2 * PLANE;
+    asm volatile("" : "+v"(kt), "+v"(vt));
 
     f32x16 sacc[2] = {f32x16{}, f32x16{}};
-    // fragments one step ahead; the scheduling barriers keep the compiler from reading all of them first (it spills)
-    u32x4 kh[2][2], kl[2][2];
-    auto kread = [&](auto S) {
-      constexpr int s = S;
-      static_for<0, 2>([&](auto B) {
-        const int r = 32 * B + c;
-        const char* p = ks + r * ROWB + (((2 * s + hf) ^ swz(r)) << 4);
-        kh[s & 1][B] = *(const u32x4*)p;
-        kl[s & 1][B] = *(const u32x4*)(p + PLANE);
-      });
+    // steps (dims 16 s .., key half b) with the fragments one step ahead; the scheduling barriers keep the compiler from
+    // reading more of them first (it spills, and a spilled register's reload waits for the tile loads in flight)
+    u32x4 kh[2], kl[2];
+    auto kread = [&](auto I) {
+      constexpr int i = I, st = i / 2, b = i % 2;
+      const char* p = lds + ((kt ^ (uint32_t)(st << 5)) + 32 * b * ROWB);
+      kh[i & 1] = *(const u32x4*)p;
+      kl[i & 1] = *(const u32x4*)(p + PLANE);
     };
     kread(std::integral_constant<int, 0>{});
-    static_for<0, DP / 16>([&](auto S) {
-      constexpr int s = S;
-      if constexpr (s + 1 < DP / 16) kread(std::integral_constant<int, s + 1>{});
-      static_for<0, 2>([&](auto B) { sacc[B] = mfma_32x32x16<true>(kl[s & 1][B], qh[s], sacc[B]); });
-      static_for<0, 2>([&](auto B) { sacc[B] = mfma_32x32x16<true>(kh[s & 1][B], ql[s], sacc[B]); });
-      static_for<0, 2>([&](auto B) { sacc[B] = mfma_32x32x16<true>(kh[s & 1][B], qh[s], sacc[B]); });
+    static_for<0, DP / 8>([&](auto I) {
+      constexpr int i = I, st = i / 2, b = i % 2;
+      if constexpr (i + 1 < DP / 8) kread(std::integral_constant<int, i + 1>{});
+      sacc[b] = mfma_32x32x16<true>(kl[i & 1], qh[st], sacc[b]);
+      sacc[b] = mfma_32x32x16<true>(kh[i & 1], ql[st], sacc[b]);
+      sacc[b] = mfma_32x32x16<true>(kh[i & 1], qh[st], sacc[b]);
       __builtin_amdgcn_sched_barrier(0);
     });
 
@@ -1382,24 +1390,22 @@ __global__ void __launch_bounds__(64 * NW, 1) attn_planes_kernel(AttnArgs a, con
     });
     l = __builtin_fmaf(l, alpha, ps);
     static_for<0, DP / 32>([&](auto D) { o[D] *= alpha; });
-    // step i: keys 16 s .., two blocks of 32 dims
-    constexpr int NPV = 4 * (DP / 64);
-    u32x4 vh[2][2], vo[2][2];
+    // steps (keys 16 s .., dims 32 d ..) likewise
+    constexpr int ND = DP / 32;
+    u32x4 vh[2], vo[2];
     auto vread = [&](auto I) {
-      constexpr int i = I, s = i / (DP / 64), d0 = i % (DP / 64) * 2;
-      static_for<0, 2>([&](auto D) {
-        vh[i & 1][D] = vfrag(vs, s, d0 + D);
-        vo[i & 1][D] = vfrag(vs + PLANE, s, d0 + D);
-      });
+      constexpr int i = I;
+      vh[i & 1] = vfrag(vt, 0, i / ND, i % ND);
+      vo[i & 1] = vfrag(vt, 1, i / ND, i % ND);
     };
     __builtin_amdgcn_sched_barrier(0);
     vread(std::integral_constant<int, 0>{});
-    static_for<0, NPV>([&](auto I) {
-      constexpr int i = I, s = i / (DP / 64), d0 = i % (DP / 64) * 2;
-      if constexpr (i + 1 < NPV) vread(std::integral_constant<int, i + 1>{});
-      static_for<0, 2>([&](auto D) { o[d0 + D] = mfma_32x32x16<true>(vo[i & 1][D], ph[s], o[d0 + D]); });
-      static_for<0, 2>([&](auto D) { o[d0 + D] = mfma_32x32x16<true>(vh[i & 1][D], pl[s], o[d0 + D]); });
-      static_for<0, 2>([&](auto D) { o[d0 + D] = mfma_32x32x16<true>(vh[i & 1][D], ph[s], o[d0 + D]); });
+    static_for<0, 4 * ND>([&](auto I) {
+      constexpr int i = I, st = i / ND, d = i % ND;
+      if constexpr (i + 1 < 4 * ND) vread(std::integral_constant<int, i + 1>{});
+      o[d] = mfma_32x32x16<true>(vo[i & 1], ph[st], o[d]);
+      o[d] = mfma_32x32x16<true>(vh[i & 1], pl[st], o[d]);
+      o[d] = mfma_32x32x16<true>(vh[i & 1], ph[st], o[d]);
       __builtin_amdgcn_sched_barrier(0);
     });
   }
