@@ -197,8 +197,11 @@ int we_conv3x3_params(we_ctx* ctx, uint32_t height, uint32_t width, uint32_t cin
 /* y = x . W^T * scale with W [N, K] as stored (fp8 / bf16 / f16 / f32 / int4). Replaces matmulWgsl
  * (src/kernels/matmul.ts:118-178) dispatched by linear() (src/model/ops.ts:61-73).
  * x: x_dtype in {F32, F16, BF16}; y: y_dtype in {F32, F16, BF16}; w_scales: int4 only, f16 [N, K/group];
- * bias: f32 [N] with WE_EPI_BIAS. Accumulation is fp32 on bf16/f16 MFMA (f32 operands are split into
- * three bf16 planes whose sum is the f32 value exactly, so every product keeps all 24 mantissa bits). */
+ * bias: f32 [N] with WE_EPI_BIAS. Accumulation is fp32 on bf16/f16 MFMA. f32 operands are split into 16-bit planes that are
+ * multiplied plane by plane: three bf16 planes whose sum is the f32 value exactly, or, for f32 x against fp8 weights and for
+ * the 3x3 convolution of an f32 image, two f16 planes scaled by a power of two (per row of x or W, per image), which hold a
+ * value to 2^-23 of itself down to 2^-18 of its row's or image's largest and to 2^-40 of that largest below; an image whose
+ * pixels lie further apart than 2^16 takes the three planes. */
 int we_matmul(we_ctx* ctx, const we_matmul_params* p, int x_dtype, const void* x, int w_dtype, const void* w,
               const void* w_scales, uint32_t group, int y_dtype, void* y, const float* bias, uint32_t flags);
 /* we_matmul that allocates nothing. No counterpart in the reference: for callers that cannot allocate device memory
@@ -302,7 +305,9 @@ int we_qk_norm_rope(we_ctx* ctx, uint32_t tokens, uint32_t heads, uint32_t head_
 /* out[t, h] = softmax(q[t, h] . k[j, g]^T / sqrt(dim)) . v[j, g] over keys j (causal: j <= t), g = h / (heads /
  * kv_heads); fails with "heads must be a multiple of kvHeads" (attention.ts:23). Token t of q starts at
  * t * q_stride elements (0 = heads * dim; k and v: 0 = kv_heads * dim; out: 0 = heads * dim), so q, k and v
- * may be slices of one fused QKV row. dtype F32 (exact f32 products), BF16 or F16 (fp32 scores, softmax and
+ * may be slices of one fused QKV row. dtype F32 (head dims 64 and 128 from 160 tokens on: two f16 planes per
+ * operand, as in we_matmul, one scale per kv head, heads whose rows lie further apart than 2^16 or that hold an inf or NaN
+ * on the f32 MFMA; else exact f32 products), BF16 or F16 (fp32 scores, softmax and
  * accumulation; probabilities rounded to the operand type). dim: a multiple of 8 (F32: 4), at most 128.
  * The reference's `chunk` only bounds its score buffer; no score matrix exists here, so it has no analogue. */
 int we_attention(we_ctx* ctx, uint32_t tokens, uint32_t heads, uint32_t kv_heads, uint32_t dim, int causal, int dtype,

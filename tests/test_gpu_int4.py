@@ -163,3 +163,28 @@ def test_tiny_shapes(graph, m, n, k, group):
     got = run(graph, m, n, k, group, words, scales, x, we.F16, we.F32)
     want = O.matmul(O.matmul_params(m, n, k, 1.0), ox, x, O.INT4, words, scales=scales, group=group)
     assert O.rel_error(got, want) < 1e-5
+
+
+@pytest.mark.parametrize("m,n,k,group,x_dt,y_dt,flags", [
+    (33, 2061, 4096, 64, we.F16, we.F32, 0),            # 64 x 64 tiles, K slices, a ragged last column tile
+    (64, 4100, 1536, 128, we.BF16, we.F16, we.EPI_BIAS),  # two 64-k blocks per scale group
+    (65, 1200, 4096, 4096, we.F16, we.F32, we.EPI_GELU),  # 128 x 128 tiles, one group per row
+    (129, 700, 4096, 64, we.BF16, we.F32, 0), (300, 1024, 1344, 192, we.F16, we.BF16, 0)])
+def test_tiles_for_many_rows(graph, tune, m, n, k, group, x_dt, y_dt, flags):
+    """M > 32 with a large weight matrix: the GEMM tiles (ragged tiles, K slices, scale buffers refilled every 8 blocks)
+    against the oracle, and against the GEMV kernels, which sum the same exact products in another order (f32: 2e-6)."""
+    rng = np.random.default_rng(m + n)
+    words, scales, x, ox = make(rng, m, n, k, group, x_dt)
+    bias = rng.uniform(-1, 1, n).astype(np.float32) if flags & we.EPI_BIAS else None
+    got = run(graph, m, n, k, group, words, scales, x, x_dt, y_dt, bias=bias, flags=flags)
+    want = O.matmul(O.matmul_params(m, n, k, 1.0), ox, x, O.INT4, words, scales=scales, group=group)
+    if bias is not None:
+        want = want + np.tile(bias.astype(np.float64), m)
+    if flags & we.EPI_GELU:
+        want = O.gelu_tanh(want)
+    tol = {we.F32: 1e-4 if flags & we.EPI_GELU else 1e-5, we.F16: 2e-3, we.BF16: 1e-2}[y_dt]
+    assert O.rel_error(got, want) < tol
+    if y_dt == we.F32:
+        tune(int4_path=1)
+        gemv = run(graph, m, n, k, group, words, scales, x, x_dt, y_dt, bias=bias, flags=flags)
+        assert O.rel_error(got, gemv) < 2e-6

@@ -689,6 +689,94 @@ def test_conv3x3_refusals(graph):
         graph.matmul(p, we.F16, b, we.INT4, b, we.F32, b, scales=b, group=64)
 
 
+@pytest.mark.parametrize("h,w,cin,cout,w_dt,y_dt,flags,cfg", [
+    (9, 11, 8, 12, we.F32, we.F32, 0, -1), (17, 16, 40, 64, we.F32, we.F32, we.EPI_BIAS, 3),
+    (23, 13, 96, 130, we.BF16, we.BF16, 0, 2), (33, 32, 72, 200, we.F32, we.F32, we.EPI_ACCUMULATE, 5),
+    (40, 29, 128, 96, we.BF16, we.F32, we.EPI_GELU, 5)])
+def test_conv3x3_planes(graph, tune, h, w, cin, cout, w_dt, y_dt, flags, cfg):
+    """f32 images through f16 planes on every tile shape and in K slices: cin whose segments need padding to 64, taps that
+    straddle 64-k blocks, ragged tiles; an image and weights far from 1 and one weight row 2^-60 of the others."""
+    rng = np.random.default_rng(h * w + cin)
+    x = rng.standard_normal(h * w * cin).astype(np.float32) * np.float32(2.0 ** 40)
+    wt = rng.standard_normal((cout, 9 * cin)).astype(np.float32) * np.float32(2.0 ** -40 * cin ** -0.5)
+    wt[3] *= np.float32(2.0 ** -60)
+    if w_dt == we.BF16:
+        w_store = O.bf16_rne(wt.reshape(-1))
+        w_oracle, ow = w_store, O.BF16
+    else:
+        w_store = w_oracle = wt.reshape(-1)
+        ow = O.F32
+    p = we.conv3x3_params(h, w, cin, cout, graph=graph)
+    bias = rng.uniform(-1, 1, cout).astype(np.float32) if flags & we.EPI_BIAS else None
+    y0 = rng.standard_normal(h * w * cout).astype(np.float32) if flags & we.EPI_ACCUMULATE else None
+    want = O.matmul(O.conv3x3_params(h, w, cin, cout), O.F32, x, ow, w_oracle)
+    if bias is not None:
+        want = want + np.tile(bias.astype(np.float64), h * w)
+    if y0 is not None:
+        want = want + y0.astype(np.float64)
+    if flags & we.EPI_GELU:
+        want = O.gelu_tanh(want)
+    tune(gemm_cfg=cfg)
+    got = run(graph, p, x, we.F32, w_store, w_dt, y_dt, flags=flags, bias=bias, y_init=y0)
+    assert O.rel_error(got, want) < (1e-4 if flags & we.EPI_GELU else TOL[y_dt])
+    if not flags and y_dt == we.F32:  # the tiny row by its own size
+        assert O.rel_error(got.reshape(-1, cout)[:, 3], want.reshape(-1, cout)[:, 3]) < TOL[y_dt]
+
+
+def test_conv3x3_planes_leave_wide_images_to_the_general_kernel(graph, tune):
+    """An image with pixels below 2^-16 of its largest value, which one scale cannot hold to f32's precision: the general
+    kernel's result bit for bit. An inf poisons the pixels around it as there, and no others."""
+    h, w, cin, cout = 20, 24, 64, 48
+    rng = np.random.default_rng(3)
+    x = rng.standard_normal((h, w, cin)).astype(np.float32)
+    x[:10] *= np.float32(2.0 ** -30)
+    wt = rng.standard_normal(cout * 9 * cin).astype(np.float32)
+    p = we.conv3x3_params(h, w, cin, cout, graph=graph)
+    wide = run(graph, p, x.reshape(-1), we.F32, wt, we.F32, we.F32)
+    x2 = rng.standard_normal((h, w, cin)).astype(np.float32)
+    x2[5, 6, 7] = np.inf
+    inf = run(graph, p, x2.reshape(-1), we.F32, wt, we.F32, we.F32)
+    tune(gemm_generic=1)
+    assert np.array_equal(wide, run(graph, p, x.reshape(-1), we.F32, wt, we.F32, we.F32))
+    general = run(graph, p, x2.reshape(-1), we.F32, wt, we.F32, we.F32)
+    assert np.array_equal(np.isfinite(inf), np.isfinite(general))
+    ok = np.isfinite(general)
+    assert O.rel_error(inf[ok], general[ok]) < 4e-6
+
+
+@pytest.mark.parametrize("k", [128, 1024])  # two f16 planes; three bf16 planes (a K-sliced plan)
+def test_f32_rows_of_any_scale(graph, k):
+    """The two f16 planes of an f32 row carry a power of two of the row's own: rows at 2^100, 2^-100, all zeros and with one
+    value 2^12 above the rest, each to f32's precision by its own size."""
+    m, n = 70, 512
+    rng = np.random.default_rng(8)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    x[1] *= np.float32(2.0 ** 100)
+    x[2] *= np.float32(2.0 ** -100)
+    x[3] = 0
+    x[4, 9] = 4096.0
+    w_store, w_oracle, ow = make_weights(rng, n, k, we.FP8)
+    p = we.matmul_params(m, n, k, 0.02, graph=graph)
+    got = run(graph, p, x.reshape(-1), we.F32, w_store, we.FP8, we.F32).reshape(m, n)
+    want = O.matmul(O.matmul_params(m, n, k, 0.02), O.F32, x.reshape(-1), ow, w_oracle).reshape(m, n)
+    assert not got[3].any()
+    for r in (0, 1, 2, 4, m - 1):
+        assert O.rel_error(got[r], want[r]) < 1e-5
+
+
+@pytest.mark.parametrize("m,n,k,w_dt", [(65, 1040, 2048, we.FP8), (129, 520, 4096, we.BF16), (300, 1028, 1024, we.FP8),
+                                        (520, 260, 3072, we.FP8), (700, 400, 512, we.BF16)])
+def test_planned_tiles_and_slices(graph, m, n, k, w_dt):
+    """M > 64: whatever tile shape and K slices the cost model picks (few tiles: 64 x 64 and 256 x 256 in slices, ragged
+    last tiles), against the oracle."""
+    rng = np.random.default_rng(m)
+    x_store, x_oracle, ox = encode_act(rng.standard_normal(m * k).astype(np.float32), we.BF16)
+    w_store, w_oracle, ow = make_weights(rng, n, k, w_dt)
+    p = we.matmul_params(m, n, k, 0.05, graph=graph)
+    got = run(graph, p, x_store, we.BF16, w_store, w_dt, we.F32)
+    assert O.rel_error(got, O.matmul(O.matmul_params(m, n, k, 0.05), ox, x_oracle, ow, w_oracle)) < TOL_F32_OUT
+
+
 F32_FAST_CASES = [
     # (m, n, k, weights, flags): ragged tiles, the small-M split-K plan over the planes, the reference's Krea layer
     # shape, bf16 weights, and the fused epilogues
@@ -700,10 +788,10 @@ F32_FAST_CASES = [
 @pytest.mark.parametrize("m,n,k,w_dt,flags", F32_FAST_CASES)
 def test_f32_activations_on_the_fast_path(graph, tune, m, n, k, w_dt, flags):
     """f32 x, the reference's own activation dtype (src/kernels/matmul.ts:129-131), with fp8 or bf16 weights and K a
-    multiple of 64: split into three exact bf16 planes and run by the fast kernel over 3K. It matches the float64
-    oracle at the reference's 1e-5 bar, and the general kernel (which splits x into the same planes tile by tile)
-    to 4e-6: every product is exact in both, only the f32 summation order differs (at K = 3072, sums of ~200 move by
-    ~1.5e-6 of max|y| between two orders)."""
+    multiple of 64: split into two f16 planes (fp8 weights) or three exact bf16 planes (bf16 weights) and run by the
+    fast kernel over all of them. It matches the float64 oracle at the reference's 1e-5 bar, and the general kernel
+    (three bf16 planes tile by tile) to 4e-6: the f32 summation order differs (at K = 3072, sums of ~200 move by
+    ~1.5e-6 of max|y| between two orders), the f16 planes hold x to 2^-23."""
     rng = np.random.default_rng(m + n + k)
     x = rng.standard_normal(m * k).astype(np.float32)
     w_store, w_oracle, ow = make_weights(rng, n, k, w_dt)
@@ -815,3 +903,35 @@ def test_tiny_shapes(graph, m, n, k, w_dt, x_dt):
     got = run(graph, p, x_store, x_dt, w, w_dt, we.F32)
     want = O.matmul(O.matmul_params(m, n, k, 0.5), ox, x_oracle, ow, w)
     assert O.rel_error(got, want) < TOL_F32_OUT
+
+
+@pytest.mark.parametrize("m,n,k,epi", [(1030, 16400, 3072, "plain"), (1030, 16400, 3072, "swiglu"), (300, 33000, 2048, "bias")])
+def test_split_last_round(graph, m, n, k, epi):
+    """More than one round of 256-row tiles with a small remainder: the tiles of the last round run in K slices and a reduce
+    pass, ragged in both directions, with the epilogues that read a second operand; rows of the first and of the last tiles
+    against the oracle (f32 x: the two-plane path, where the plan picks 256 x 256)."""
+    rng = np.random.default_rng(m + n)
+    x = rng.standard_normal(m * k).astype(np.float32)
+    w_store, w_oracle, ow = make_weights(rng, n, k, we.FP8)
+    p = we.matmul_params(m, n, k, 0.02, graph=graph)
+    mark = graph.mark()
+    xb, wb, y = graph.buffer(x), graph.buffer(w_store), graph.buffer(m * n * 4)
+    aux = rng.standard_normal(m * n).astype(np.float32)
+    bias = rng.uniform(-1, 1, n).astype(np.float32)
+    if epi == "swiglu":
+        ab = graph.buffer(aux)
+        graph.matmul(p, we.F32, xb, we.FP8, wb, we.F32, y, mul=we.MUL_SWIGLU, aux=ab)
+    elif epi == "bias":
+        graph.matmul(p, we.F32, xb, we.FP8, wb, we.F32, y, bias=graph.buffer(bias), flags=we.EPI_BIAS)
+    else:
+        graph.matmul(p, we.F32, xb, we.FP8, wb, we.F32, y)
+    got = graph.read(y, dtype=np.float32).astype(np.float64).reshape(m, n)
+    graph.release(mark)
+    for rows in ((0, 3), (m - 7, m)):
+        want = O.matmul_rows(O.matmul_params(m, n, k, 0.02), O.F32, x, ow, w_oracle, *rows).reshape(m, n)[rows[0]:rows[1]]
+        if epi == "swiglu":
+            a = aux.reshape(m, n)[rows[0]:rows[1]].astype(np.float64)
+            want = a / (1 + np.exp(-a)) * want
+        elif epi == "bias":
+            want = want + bias.astype(np.float64)
+        assert O.rel_error(got[rows[0]:rows[1]].ravel(), want.ravel()) < TOL_F32_OUT

@@ -52,10 +52,11 @@ hipError_t gemm_launch(const GemmLaunch& L, hipStream_t stream) {
   a.aligned = aligned16(L.x, L.x_offset, L.x_stride, xb) && aligned16(L.w, L.w_offset, L.w_stride, wb) &&
               ((uint64_t)a.kc * xb) % 16 == 0 && ((uint64_t)a.kc * wb) % 16 == 0;
   // f32 x against 16-bit or fp8 weights holds three planes of x: a 128 x 128 tile takes 128 KB, one workgroup of 4 waves per
-  // CU. 64 x 64 runs the small products of a LoRA update faster (1024 x 32 x 6144 in 24 K slices: 29.8 -> 18.2 us, 1024 x
-  // 6144 x 32: 73 -> 35 us)
-  const int by_shape = pick_gemm_cfg(L.m, L.n, splits);
-  const int cfg = L.cfg >= 0 ? L.cfg : L.x_dtype == F32 && L.m > 64 ? (int)GEMM_CFG_64x64 : by_shape;
+  // CU. 64 x 64 is faster where such tiles leave half of the CUs idle or K is short: 1024 x 32 x 6144 in 24 K slices 29.8 ->
+  // 18.2 us, 1024 x 6144 x 32 73 -> 35, 300 x 3072 x 3080 529 -> 274; not at 1024 x 3072 x 3080 (286, 304 with 64 x 64)
+  const uint64_t tiles128 = (uint64_t)((L.m + 127) / 128) * ((L.n + 127) / 128) * splits;
+  const bool small = L.x_dtype == F32 && L.m > 64 && (tiles128 < 128 || L.k <= 256 || L.n <= 64);
+  const int cfg = L.cfg >= 0 ? L.cfg : small ? (int)GEMM_CFG_64x64 : pick_gemm_cfg(L.m, L.n, splits);
   switch (L.x_dtype) {
     case BF16: return gemm_general_bf16(L.w_dtype, a, splits, cfg, stream);
     case F16: return gemm_general_f16(L.w_dtype, a, splits, cfg, stream);

@@ -94,7 +94,7 @@ int launch_cfg_of(const GemmLaunch& L) {
 }  // namespace
 
 GemmReducePlan gemm_reduce_plan(const GemmLaunch& L, uint32_t force_splits) {
-  GemmReducePlan p{1, L.k, 0, -1};
+  GemmReducePlan p{1, L.k, 0, -1, 1};
   if (L.generic || (L.splits > 1) || (L.flags & WE_EPI_SPLIT_K_BIT) || L.m == 0 || L.n == 0) return p;
   if (L.k < 512 || !fast_supported(L, L.k)) return p;
   const int cfg = L.cfg >= 0 ? L.cfg : pick_fast_cfg(L.m, L.n, 1, L.w_dtype == FP8);
@@ -169,32 +169,60 @@ GemmReducePlan gemm_plan(const GemmLaunch& L) {
   if (L.cfg >= 0 || L.m <= 64 || L.n == 0 || L.generic || L.splits > 1 || (L.flags & WE_EPI_SPLIT_K_BIT) || L.k < 512 ||
       !fast_supported(L, L.k))
     return gemm_reduce_plan(L);
-  const bool w8 = L.w_dtype == FP8;
+  const bool w8 = L.w_dtype == FP8, three = L.k_wrap && L.k == 3 * L.k_wrap;
   const CostModel& c = !w8 ? kCost16 : L.k_wrap ? kCostPlanes : kCostFp8;
   // workgroups per CU by their LDS: 64 x 64 36 or 48 KB, 128 x 128 72 or 96 KB
   const uint32_t per_cu[6] = {1, 1, w8 ? 2u : 1u, w8 ? 4u : 3u, 1, 1};
-  GemmReducePlan best{1, L.k, 0, GEMM_CFG_128x128};
-  double best_us = 1e30;
-  for (const int cfg : {GEMM_CFG_256x256, GEMM_CFG_256x192, GEMM_CFG_256x128, GEMM_CFG_128x128, GEMM_CFG_64x64}) {
-    if (cfg_bm(cfg) == 256 && L.m < 256) continue;
+  auto predict = [&](int cfg, uint32_t slices, uint32_t kc) {
     const uint64_t tiles = (uint64_t)((L.m + cfg_bm(cfg) - 1) / cfg_bm(cfg)) * ((L.n + cfg_bn(cfg) - 1) / cfg_bn(cfg));
     const uint64_t slots = (uint64_t)kCUs * per_cu[cfg];
     const int several = per_cu[cfg] > 1 || cfg == GEMM_CFG_128x128;
+    const uint64_t full = tiles * slices / slots, rest = tiles * slices % slots;
+    const double rounds = (double)full + (rest ? c.part[several] + c.part_f[several] * (double)rest / (double)slots : 0.0);
+    double us = c.launch + rounds * ((double)((kc + BK - 1) / BK) * c.block[cfg] + c.tile[cfg]);
+    if (slices > 1) us += c.reduce + c.reduce_mb * 4e-6 * L.m * (double)L.n * slices;
+    // q / k norm and RoPE: a pass over those columns, or in the epilogue for about the same time less a launch (2500 x 6144
+    // x 4096 bf16: 129.6 us with 256 x 256 tiles and the pass, 150.9 us fused in 256 x 128 tiles)
+    if (L.qk_cols) us += (slices > 1 || !qk_fusable_cfg(cfg) ? 4.0 : 0.0) + 4.0 * L.m * (double)L.qk_cols / 3e6;
+    return us;
+  };
+  // The older rules' choice stays unless another is predicted 4% faster (the model's error is of that order: 1500 x 4608 x
+  // 3072 took 55.2 us in the 256 x 128 tiles that it put 2% ahead of the 128 x 128 ones, 54.2 us).
+  GemmReducePlan best = gemm_reduce_plan(L);
+  const uint32_t older = best.rsplits;
+  best.rcfg = best.rcfg >= 0 ? best.rcfg : pick_fast_cfg(L.m, L.n, best.rsplits, w8);
+  double best_us = 0.96 * predict(best.rcfg, best.rsplits, best.rsplits > 1 ? best.rkc : L.k);
+  for (const int cfg : {GEMM_CFG_256x256, GEMM_CFG_256x192, GEMM_CFG_256x128, GEMM_CFG_128x128, GEMM_CFG_64x64}) {
+    if (cfg_bm(cfg) == 256 && L.m < 256) continue;
+    const uint64_t tiles = (uint64_t)((L.m + cfg_bm(cfg) - 1) / cfg_bm(cfg)) * ((L.n + cfg_bn(cfg) - 1) / cfg_bn(cfg));
     // slices only where the tiles fill at most half of the CUs (128 x 128: twice that), as swept
     const uint32_t most = tiles * 2 <= kCUs * (cfg == GEMM_CFG_128x128 ? 2u : 1u) ? std::min(8u, L.k / 256) : 1u;
-    for (uint32_t rs = 1; rs <= most; rs++) {
+    // three planes of x: no fewer slices than the older plan, whose shorter sums round less (128 x 2048 x 8192 1.6e-7)
+    for (uint32_t rs = three ? older : 1; rs <= most; rs++) {
       const uint32_t kc = (L.k + rs * BK - 1) / (rs * BK) * BK;
-      const uint32_t slices = (L.k + kc - 1) / kc;
-      if (slices != rs) continue;
-      const uint64_t full = tiles * slices / slots, rest = tiles * slices % slots;
-      const double rounds = (double)full + (rest ? c.part[several] + c.part_f[several] * (double)rest / (double)slots : 0.0);
-      double us = c.launch + rounds * ((double)((kc + BK - 1) / BK) * c.block[cfg] + c.tile[cfg]);
-      if (slices > 1) us += c.reduce + c.reduce_mb * 4e-6 * L.m * (double)L.n * slices;
-      // q / k norm and RoPE outside the epilogue: a pass over those columns
-      if (L.qk_cols && (slices > 1 || !qk_fusable_cfg(cfg))) us += 4.0 + 4.0 * L.m * (double)L.qk_cols / 3e6;
+      if ((L.k + kc - 1) / kc != rs) continue;
+      const double us = predict(cfg, rs, kc);
       if (us < best_us) {
         best_us = us;
-        best = GemmReducePlan{slices, slices > 1 ? kc : L.k, slices > 1 ? (size_t)slices * L.m * L.n * 4 : 0, cfg};
+        best = GemmReducePlan{rs, rs > 1 ? kc : L.k, rs > 1 ? (size_t)rs * L.m * L.n * 4 : 0, cfg, 1};
+      }
+    }
+    // One workgroup per CU and a last round of at most half of them: its tiles in as many K slices as fill the round
+    // (1103 x 16384 x 6144 f32: 320 tiles of 256 x 256 in 1.25 rounds instead of 2, less 25 us for the partial sums; the
+    // gated MLP of 1103 rows 1346 -> 1176 us)
+    const uint32_t rest = (uint32_t)(tiles % kCUs);
+    if ((cfg == GEMM_CFG_256x256 || cfg == GEMM_CFG_256x192) && tiles > kCUs && rest && rest * 2 <= kCUs && !L.qk_cols &&
+        !(three && older > 1)) {
+      const uint32_t ts = std::min({kCUs / rest, 8u, L.k / 512});
+      const uint32_t kc = ts > 1 ? (L.k + ts * BK - 1) / (ts * BK) * BK : 0;
+      if (ts > 1 && (L.k + kc - 1) / kc == ts) {
+        const double sums = (double)ts * rest * cfg_bm(cfg) * cfg_bn(cfg) * 4.0;
+        const double us = c.launch + (double)(tiles / kCUs) * ((L.k + BK - 1) / BK * c.block[cfg] + c.tile[cfg]) +
+                          ((double)(kc / BK) * c.block[cfg] + c.tile[cfg]) + 4.0 + c.reduce_mb * 1e-6 * sums;
+        if (us < best_us) {
+          best_us = us;
+          best = GemmReducePlan{1, kc, (size_t)sums, cfg, ts};
+        }
       }
     }
   }
@@ -279,6 +307,12 @@ hipError_t gemm_fast_launch(const GemmLaunch& L, hipStream_t stream) {
     if (!L.scratch) return hipErrorInvalidValue;
     a.part = (float*)L.scratch;
     a.rsplits = splits;
+  }
+  if (L.tail_splits > 1) {
+    if (!L.scratch || reduce || splits > 1 || L.tail_splits > 8) return hipErrorInvalidValue;
+    a.part = (float*)L.scratch;
+    a.tail_splits = L.tail_splits;
+    a.tail_kc = L.rkc;
   }
   const int cfg = launch_cfg_of(L);
   const int rx = L.reduce_xcd;

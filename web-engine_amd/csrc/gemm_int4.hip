@@ -17,9 +17,13 @@ hipError_t launch_tile(const FastArgs& a, uint32_t splits, int cfg, int rx, hipS
   return launch_fast_cfg<64, 64, 2, 2, IS_F16, INT4, 3>(a, splits, rx, s);
 }
 
+// 64 x 64 tiles (three workgroups per CU) where 128 x 128 ones (two, of 4 waves of 128 x 32: each weight is unpacked once
+// per workgroup) would fill at most a quarter of their slots: 400 x 4096 x 2048 32.9 -> 27.2 us, 2048 x 1024 x 1536 35.2 ->
+// 20.8, 128 x 4096 x 4096 25.6 -> 19.4; but 256 x 18944 x 3584 72.5 us with 128 x 128, 89.0 with 64 x 64.
 int pick_cfg(const Int4Launch& L) {
   if (L.cfg == GEMM_CFG_128x128 || L.cfg == GEMM_CFG_64x64) return L.cfg;
-  return L.m <= 64 ? GEMM_CFG_64x64 : GEMM_CFG_128x128;
+  const uint64_t tiles128 = (uint64_t)((L.m + 127) / 128) * ((L.n + 127) / 128);
+  return L.m <= 64 || tiles128 <= 128 ? GEMM_CFG_64x64 : GEMM_CFG_128x128;
 }
 
 }  // namespace
@@ -37,11 +41,11 @@ bool int4_gemm_supported(const Int4Launch& L) {
 }
 
 GemmReducePlan int4_gemm_plan(const Int4Launch& L) {
-  GemmReducePlan p{1, L.k, 0, -1};
+  GemmReducePlan p{1, L.k, 0, -1, 1};
   const int cfg = pick_cfg(L);
   const uint32_t bm = cfg == GEMM_CFG_64x64 ? 64 : 128, bn = bm;
   const uint64_t tiles = (uint64_t)((L.m + bm - 1) / bm) * ((L.n + bn - 1) / bn);
-  const uint64_t slots = kCUs * 3;
+  const uint64_t slots = kCUs * (bm == 64 ? 3 : 2);
   if (tiles * 2 > slots) return p;
   uint32_t rs = (uint32_t)((slots + tiles - 1) / tiles);
   rs = std::min(rs, L.k / 256);  // every slice keeps at least 256 of K
@@ -49,7 +53,7 @@ GemmReducePlan int4_gemm_plan(const Int4Launch& L) {
   const uint32_t kc = (L.k + rs * BK - 1) / (rs * BK) * BK;
   const uint32_t slices = (L.k + kc - 1) / kc;
   if (slices < 2) return p;
-  return GemmReducePlan{slices, kc, (size_t)slices * L.m * L.n * 4, -1};
+  return GemmReducePlan{slices, kc, (size_t)slices * L.m * L.n * 4, -1, 1};
 }
 
 hipError_t int4_gemm_launch(const Int4Launch& L, hipStream_t stream) {

@@ -4,9 +4,10 @@
 // (src/kernels/matmul.ts:118-178).
 //
 // Structure (one workgroup per BM x BN output tile, 64 k per pipeline stage, S stages in LDS):
-//  * Operands move HBM -> LDS with direct-to-LDS buffer loads (buffer_load_dwordx4 ... lds; outside the ping-pong tiles
-//    issued as inline asm: behind the builtin the compiler drains every load in flight before the next LDS read, once
-//    per 64-k block of these tiles; the ping-pong loop has no such waits and ran 1% slower on the asm): each load
+//  * Operands move HBM -> LDS with direct-to-LDS buffer loads (buffer_load_dwordx4 ... lds; in the int4 tiles and those of
+//    at most 64 rows issued as inline asm: behind the builtin the compiler drains every load in flight before the next
+//    LDS read, once per 64-k block there (64 x 3072 x 3072 fp8 11.2 -> 11.0 us); the larger tiles ran 1-2% slower on the
+//    asm): each load
 //    instruction of a wave fills 1 KB of LDS (lane i writes bytes [16 i, 16 i + 16)), no VGPR staging.
 //    The source address of each lane is chosen so that the LDS image is XOR-swizzled: 16-byte chunk c of
 //    row r sits at chunk position c ^ swz(r), which makes the MFMA fragment reads bank-conflict free.
@@ -27,9 +28,10 @@
 //    that wave through an exact recompute that decodes every byte with the shader's formula.
 // Requirements (checked on the host): x / W rows 16-byte aligned, K and the split-K slice multiples of
 // 16, operand extents below 2^31 bytes.
-// f32 activations arrive as three exact bf16 planes along K (x [M, 3K], split by a pass before the GEMM); the kernel
-// walks k over all 3K while the weights are read at k mod K (K a multiple of 64, so no 64-k block spans two
-// planes): one GEMM of exact products, so every epilogue applies to the f32-exact sum.
+// f32 activations arrive as 16-bit planes along K (split by a pass before the GEMM): two f16 planes with a scale per row
+// (x [M, 2K], fp8 weights) or three exact bf16 planes (x [M, 3K], bf16 weights). The kernel walks k over all planes while
+// the weights are read at k mod K (K a multiple of 64, so no 64-k block spans two planes), so every epilogue applies to the
+// whole sum. The CONV kernels read x as an f16 image and gather each tap's pixels by the loads' addresses (gemm_conv.hip).
 #pragma once
 #include "common.h"
 #include "internal.h"
@@ -79,6 +81,9 @@ struct FastArgs {
   // the lo plane, the others with the hi plane. conv_magic = ceil(2^32 / conv_cin)
   uint32_t conv_width, conv_cin, conv_kp, conv_magic;
   const uint32_t* skip_if;  // CONV kernels and their reduce pass: nothing to do where this word is not 0
+  // A split last round (tail_tiles > 0; GemmReducePlan::tail_splits): the tiles from tail_first on, a multiple of the CUs,
+  // run as tail_splits K slices of tail_kc each, whose raw sums go to part as dense tiles, slice-major
+  uint32_t tail_first, tail_tiles, tail_splits, tail_kc;
   uint32_t mul;  // product epilogue with res (GemmLaunch::mul), 0: none
   // fused per-head RMSNorm + RoPE of the q / k columns (GemmLaunch::qk_*), qk_cols 0: none
   uint32_t qk_cols, q_cols, qk_rope_from;
@@ -108,6 +113,7 @@ constexpr int BK = 64;
 
 constexpr uint32_t kInvalid = 0x80000000u;  // a byte offset past every extent: the load returns 0
 constexpr int kRsrcWord3 = 0x00020000;      // raw buffer, 32-bit data format (gfx9 family)
+constexpr int kCpolNt = 2;                  // buffer-load cache policy: nt (non-temporal)
 
 __device__ __forceinline__ uint32_t xcd_remap_f(uint32_t pid, uint32_t total) {
   const uint32_t xcd = pid & 7u, idx = pid >> 3;
@@ -224,6 +230,8 @@ __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64) gemm_lds_kernel(FastArg
   // 243 -> 279 us, 2, each group its own share in its compute phase: 247 -> 291 us, up-projection, same box).
   // Other tiles: every wave loads its share in the memory phase.
   constexpr int LM = PP ? (B8 ? 0 : 1) : 0;
+  // Loads as inline asm (file comment): the int4 tiles and the small ones
+  constexpr bool DMA_ASM = B4 || BM <= 64;
   constexpr int NL = LM == 1 ? NW / 2 : NW;                               // waves that issue loads
   static_assert(A_INS % NL == 0 && B_INS % NL == 0, "stage loads split evenly over the loading waves");
   constexpr int A_PW = A_INS / NL, B_PW = B_INS / NL, L = A_PW + B_PW;  // loads per loading wave per stage
@@ -238,7 +246,21 @@ __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64) gemm_lds_kernel(FastArg
   const int lw = wave % NL;  // this wave's share of the loads (LM 1: group 1's waves 0 .. NW / 2 - 1)
   const int h = lane >> 5, l32 = lane & 31;
 
-  uint32_t pid = xcd_remap_f(blockIdx.x, gridDim.x);
+  uint32_t pid, z = blockIdx.y, kc = a.kc;
+  constexpr bool TAIL = PP && !CONV;  // the tile shapes whose last round is split
+  bool tail = false;                         // this workgroup is a slice of a last-round tile
+  if constexpr (!TAIL) {
+    pid = xcd_remap_f(blockIdx.x, gridDim.x);
+  } else if (a.tail_tiles && blockIdx.x >= a.tail_first) {
+    const uint32_t t = xcd_remap_f(blockIdx.x - a.tail_first, a.tail_tiles * a.tail_splits);
+    pid = a.tail_first + t % a.tail_tiles;
+    z = t / a.tail_tiles;
+    kc = a.tail_kc;
+    tail = true;
+  } else {
+    pid = xcd_remap_f(blockIdx.x, a.tail_tiles ? a.tail_first : gridDim.x);
+  }
+  const uint32_t tail_tile = TAIL ? pid - a.tail_first : 0;  // (meaningful in a slice)
   if (a.grp_first && pid >= a.grp_first) {  // a tile of the second GEMM of a paired launch
     pid -= a.grp_first;
     a.x = a.g.x;
@@ -266,9 +288,8 @@ __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64) gemm_lds_kernel(FastArg
   const uint32_t in_group = pid % per_group;
   const uint32_t row0 = (first_m + in_group % gsize) * BM, col0 = (in_group / gsize) * BN;
 
-  const uint32_t z = blockIdx.y;
-  const uint32_t k_begin = z * a.kc;
-  const uint32_t k_end = min(a.k, k_begin + a.kc);
+  const uint32_t k_begin = z * kc;
+  const uint32_t k_end = min(a.k, k_begin + kc);
   const int nk = k_end > k_begin ? (int)((k_end - k_begin + BK - 1) / BK) : 0;
 
   const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void*)a.x, (short)0, (int)a.x_bytes, kRsrcWord3);
@@ -341,20 +362,22 @@ __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64) gemm_lds_kernel(FastArg
       if constexpr (q == 0) conv_block(kb);  // the block's loads are issued in order
       const uint32_t o = taps[q] >> conv_tap & 1u ? offa[q] + (uint32_t)conv_off : kInvalid;
       char* dst = base + (lw + q * NL) * 1024;
-      if constexpr (PP) __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lds_ptr_t*)dst, 16, o, 0, 0, 0);
+      if constexpr (!DMA_ASM) __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lds_ptr_t*)dst, 16, o, 0, 0, 0);
       else dma16s(rx, dst, o, 0u);
     } else if constexpr (q < A_PW) {
       const uint32_t o = (full || kb + ka < k_end) ? offa[q] : kInvalid;
       char* dst = base + (lw + q * NL) * 1024;
-      if constexpr (PP) __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lds_ptr_t*)dst, 16, o, (int)(kb * 2), 0, 0);
+      if constexpr (!DMA_ASM) __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lds_ptr_t*)dst, 16, o, (int)(kb * 2), 0, 0);
       else dma16s(rx, dst, o, kb * 2);
     } else {
       constexpr int j = q - A_PW;
       const uint32_t o = (full || kb + kb8 < k_end) ? offb[j] : kInvalid;
       const uint32_t kbw = kb >= a.kwrap2 ? kb - a.kwrap2 : kb >= a.kwrap ? kb - a.kwrap : kb;  // weights' k
       char* dst = base + A_BYTES + (lw + j * NL) * 1024;
-      if constexpr (PP) __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (lds_ptr_t*)dst, 16, o, (int)wbytes(kbw), 0, 0);
-      else if (w_once) dma16s<true>(rw, dst, o, wbytes(kbw));
+      if constexpr (!DMA_ASM) {
+        if (w_once) __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (lds_ptr_t*)dst, 16, o, (int)wbytes(kbw), 0, kCpolNt);
+        else __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (lds_ptr_t*)dst, 16, o, (int)wbytes(kbw), 0, 0);
+      } else if (w_once) dma16s<true>(rw, dst, o, wbytes(kbw));
       else dma16s(rw, dst, o, wbytes(kbw));
     }
   };
@@ -823,6 +846,14 @@ __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64) gemm_lds_kernel(FastArg
     }
   }
 
+  if (TAIL && tail) {
+    float* t = a.part + ((size_t)z * a.tail_tiles + tail_tile) * (BM * BN) + (wm * WTM + lrow) * BN + wn * WTN + lcol;
+#pragma unroll
+    for (int i = 0; i < RR; i++)
+#pragma unroll
+      for (int rc = 0; rc < RC; rc++) *(f32x4*)(t + i * RS * BN + ccol(rc)) = av(i, rc);
+    return;
+  }
   if (a.rsplits > 1) {
     // ---- split-K slice: raw sums (no scale) to the partial-sum plane of this slice
     const size_t plane = (size_t)a.m * a.n;
@@ -1070,6 +1101,34 @@ __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64) gemm_lds_kernel(FastArg
   }
 }
 
+// The epilogue of 4 summed outputs (row, c0 ..) in a reduce pass.
+template <int YT>
+__device__ __forceinline__ void reduce_epilogue(const FastArgs& a, uint32_t row, uint32_t c0, float (&v)[4]) {
+  const bool full = c0 + 3 < a.n;
+  const bool accum = (a.flags & WE_EPI_ACCUMULATE_BIT) != 0;
+  const bool has_bias = (a.flags & WE_EPI_BIAS_BIT) != 0;
+  const bool gelu = (a.flags & WE_EPI_GELU_BIT) != 0;
+  const void* aux = a.mul ? a.res : nullptr;
+  const void* addend = a.mul ? nullptr : a.res ? a.res : (accum ? a.y : nullptr);
+  const size_t yrow = (size_t)a.y_offset + (size_t)row * a.y_stride;
+#pragma unroll
+  for (int e = 0; e < 4; e++) {
+    float t = v[e] * a.scale;
+    if (has_bias) t += a.bias[c0 + e < a.n ? c0 + e : 0];
+    if (gelu) t = gelu_tanh(t);
+    if (a.gate) t *= a.gate[c0 + e < a.n ? c0 + e : 0];
+    if (aux && c0 + e < a.n) t = mul_epilogue(a.mul, load1<YT>(aux, yrow + c0 + e), t);
+    v[e] = t;
+  }
+  if (a.vec_store && full) {
+    store4<YT>(a, yrow + c0, v, addend);
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+      if (c0 + e < a.n) store1<YT>(a, yrow + c0 + e, v[e], addend);
+  }
+}
+
 // Sum of the split-K partial planes, then the epilogue of the GEMM (scale, bias, GELU, accumulate, output
 // type): one thread per 4 consecutive outputs of a row, slices added in slice order.
 // XCD (BM, BN > 0): the slices of a tile ran on one XCD (workgroups go round-robin over the 8 XCDs, and the slice
@@ -1120,28 +1179,34 @@ __global__ void __launch_bounds__(256) splitk_reduce_kernel(FastArgs a) {
       for (int e = 0; e < 4; e++)
         if (c0 + e < a.n) v[e] += p[e];
   }
-  const bool accum = (a.flags & WE_EPI_ACCUMULATE_BIT) != 0;
-  const bool has_bias = (a.flags & WE_EPI_BIAS_BIT) != 0;
-  const bool gelu = (a.flags & WE_EPI_GELU_BIT) != 0;
-  const void* aux = a.mul ? a.res : nullptr;
-  const void* addend = a.mul ? nullptr : a.res ? a.res : (accum ? a.y : nullptr);
-  const size_t yrow = (size_t)a.y_offset + (size_t)row * a.y_stride;
+  reduce_epilogue<YT>(a, row, c0, v);
+}
+
+// The reduce pass of a split last round: one thread per 4 consecutive outputs of a tail tile, slices in slice order.
+template <int YT, int BM, int BN>
+__global__ void __launch_bounds__(256) tail_reduce_kernel(FastArgs a) {
+  constexpr uint32_t ITEMS = BM * BN / 4, Q = ITEMS / 256;  // workgroups per tile
+  const uint32_t t = blockIdx.x / Q, i = (blockIdx.x % Q) * 256 + threadIdx.x;
+  const uint32_t pid = a.tail_first + t;
+  constexpr uint32_t GROUP_M = 4;
+  const uint32_t per_group = GROUP_M * a.tiles_n, first_m = (pid / per_group) * GROUP_M;
+  const uint32_t gsize = min(a.tiles_m - first_m, GROUP_M), in_group = pid % per_group;
+  const uint32_t row = (first_m + in_group % gsize) * BM + i / (BN / 4);
+  const uint32_t c0 = (in_group / gsize) * BN + (i % (BN / 4)) * 4;
+  if (row >= a.m || c0 >= a.n) return;
+  const float* p = a.part + (size_t)t * (BM * BN) + (size_t)i * 4;
+  const size_t plane = (size_t)a.tail_tiles * (BM * BN);
+  f32x4 s[8];
 #pragma unroll
-  for (int e = 0; e < 4; e++) {
-    float t = v[e] * a.scale;
-    if (has_bias) t += a.bias[c0 + e < a.n ? c0 + e : 0];
-    if (gelu) t = gelu_tanh(t);
-    if (a.gate) t *= a.gate[c0 + e < a.n ? c0 + e : 0];
-    if (aux && c0 + e < a.n) t = mul_epilogue(a.mul, load1<YT>(aux, yrow + c0 + e), t);
-    v[e] = t;
-  }
-  if (a.vec_store && full) {
-    store4<YT>(a, yrow + c0, v, addend);
-  } else {
+  for (uint32_t z = 0; z < 8; z++)
+    if (z < a.tail_splits) s[z] = *(const f32x4*)(p + z * plane);
+  float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int e = 0; e < 4; e++)
-      if (c0 + e < a.n) store1<YT>(a, yrow + c0 + e, v[e], addend);
-  }
+  for (uint32_t z = 0; z < 8; z++)
+    if (z < a.tail_splits)
+#pragma unroll
+      for (int e = 0; e < 4; e++) v[e] += s[z][e];
+  reduce_epilogue<YT>(a, row, c0, v);
 }
 
 // Does the split-K reduce pass read each tile's partial sums from the L2 of the XCD that computed them? With a
@@ -1160,6 +1225,11 @@ static hipError_t launch_fast_cfg(FastArgs a, uint32_t splits, int reduce_xcd, h
     a.g.tiles_m = (a.g.m + BM - 1) / BM;
     a.grp_first = tiles;
     tiles += a.g.tiles_m * a.tiles_n;
+  }
+  if (a.tail_splits > 1) {  // a split last round: no K slices or second GEMM beside it
+    a.tail_first = tiles / 256 * 256;
+    a.tail_tiles = tiles - a.tail_first;
+    tiles = a.tail_first + a.tail_tiles * a.tail_splits;
   }
   const dim3 grid(tiles, splits), block(WM * WN * 64);
   if (a.rsplits > 1) {
@@ -1198,6 +1268,16 @@ static hipError_t launch_fast_cfg(FastArgs a, uint32_t splits, int reduce_xcd, h
     case F32: hipLaunchKernelGGL((gemm_lds_kernel<BM, BN, WM, WN, IS_F16, BT, S, F32, PP, CONV>), grid, block, 0, s, a); break;
     case F16: hipLaunchKernelGGL((gemm_lds_kernel<BM, BN, WM, WN, IS_F16, BT, S, F16, PP, CONV>), grid, block, 0, s, a); break;
     default: hipLaunchKernelGGL((gemm_lds_kernel<BM, BN, WM, WN, IS_F16, BT, S, BF16, PP, CONV>), grid, block, 0, s, a); break;
+  }
+  if (a.tail_tiles) {
+    const hipError_t err = hipGetLastError();
+    if (err != hipSuccess) return err;
+    const dim3 rg(a.tail_tiles * (BM * BN / 4 / 256));
+    switch (a.y_dtype) {
+      case F32: hipLaunchKernelGGL((tail_reduce_kernel<F32, BM, BN>), rg, dim3(256), 0, s, a); break;
+      case F16: hipLaunchKernelGGL((tail_reduce_kernel<F16, BM, BN>), rg, dim3(256), 0, s, a); break;
+      default: hipLaunchKernelGGL((tail_reduce_kernel<BF16, BM, BN>), rg, dim3(256), 0, s, a); break;
+    }
   }
   return hipGetLastError();
 }

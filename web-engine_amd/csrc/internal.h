@@ -79,6 +79,7 @@ struct GemmLaunch {
   // reduce pass that runs the epilogue; rcfg: the tile configuration the slices were sized for (-1: by shape)
   uint32_t rsplits, rkc;
   int rcfg;
+  uint32_t tail_splits;  // GemmReducePlan::tail_splits (rsplits 1), its partial sums in scratch
   void* scratch;
 };
 hipError_t gemm_launch(const GemmLaunch& L, hipStream_t stream);
@@ -93,6 +94,7 @@ struct GemmReducePlan {
   uint32_t rsplits, rkc;
   size_t scratch_bytes;
   int rcfg;  // the tile configuration the slices are sized for, -1: the launch picks by shape
+  uint32_t tail_splits;  // > 1: only the last, partly filled round of tiles runs in K slices, that many, of rkc
 };
 GemmReducePlan gemm_reduce_plan(const GemmLaunch& L, uint32_t force_splits = 0);  // force_splits: sweeps
 // The tile shape and K slices by predicted time (M > 64); gemm_reduce_plan below that and with a forced tile shape. The

@@ -1038,13 +1038,7 @@ int matmul_impl(we_ctx* ctx, const we_matmul_params* p, int x_dtype, const void*
   if (rc) return rc;
   we::GemmLaunch L;
   fill_gemm(L, ctx->tune, p, x_dtype, x, w_dtype, w, y_dtype, y, bias, flags, gate, res, mul, splits, kc);
-  // f32 activations (the reference's own dtype) on the fast path: x is split once into 16-bit planes along K in scratch and
-  // the fast kernel runs one GEMM over all planes with the weights read at k mod K. fp8 weights (exact in f16): two f16
-  // planes [M, 2K] (lo | hi), each row scaled by a power of two of its own, which hold x to 2^-23; bf16 weights, whose
-  // range f16 lacks: three bf16 planes [M, 3K] (hi | mid | lo) that sum to x exactly. A third fewer products and fewer f32
-  // roundings: 1024 x 6144 x 6144 fp8 error against f64 9.1e-7 -> 4.2e-7. Taken when the fast kernel accepts the planes
-  // (fp8 or bf16 weights, K a multiple of 64, aligned rows); otherwise, for the allocation-free entry point and for
-  // split-K partial modes, the general kernel splits x into the same planes tile by tile.
+  // The 3x3 convolution of an f32 image on the fast tiles (gemm_conv.hip) where it applies and its scratch is to be had
   if (L.conv_width && !noalloc) {
     const size_t need = we::conv_fast_scratch(L);
     void* scratch = need ? try_scratch(ctx, need) : nullptr;
@@ -1053,19 +1047,33 @@ int matmul_impl(we_ctx* ctx, const we_matmul_params* p, int x_dtype, const void*
       return e == hipSuccess ? WE_OK : hip_fail(ctx, e, "convolution launch");
     }
   }
+  // f32 activations (the reference's own dtype) on the fast path: x is split once into 16-bit planes along K in scratch and
+  // the fast kernel runs one GEMM over all planes with the weights read at k mod K. fp8 weights (exact in f16): two f16
+  // planes [M, 2K] (lo | hi), each row scaled by a power of two of its own, which hold x to 2^-23: a third fewer products
+  // and fewer f32 roundings than three planes (1024 x 6144 x 6144: error against f64 9.1e-7 -> 4.2e-7). Three bf16 planes
+  // [M, 3K] (hi | mid | lo), exactly x, for bf16 weights, whose range f16 lacks, for M <= 64 and for shapes that three
+  // planes run in more than two K slices: those short sums round less than the f16 planes do (17 x 6144 x 2048 1.1e-7 with
+  // three planes, 1.4e-7 with two; 128 x 2048 x 8192 1.6e-7 and 2.5e-7). Taken when the fast kernel accepts the planes
+  // (fp8 or bf16 weights, K a multiple of 64, aligned rows); otherwise, for the allocation-free entry point and for
+  // split-K partial modes, the general kernel splits x into three bf16 planes tile by tile.
   size_t plane_bytes = 0, scale_at = 0;
   if (x_dtype == WE_F32 && !noalloc && !split && !L.generic && !L.conv_width && p->k % 64 == 0 &&
       (w_dtype == WE_FP8_E4M3 || w_dtype == WE_BF16) && (uintptr_t)x % 16 == 0 &&
       (uint64_t)p->m * p->k * 3 <= (1ull << 30)) {
     we::GemmLaunch P = L;
     P.x = (const void*)(uintptr_t)256;  // placeholder with the scratch's alignment, for the check
-    const uint32_t planes = w_dtype == WE_FP8_E4M3 ? 2 : 3;
-    P.x_dtype = planes == 2 ? WE_F16 : WE_BF16;
-    P.k = planes * p->k;
-    P.kc = P.k;
-    P.k_wrap = p->k;
-    P.x_stride = planes * p->k;
-    P.x_offset = 0;
+    auto set_planes = [&](uint32_t planes) {
+      P.x_dtype = planes == 2 ? WE_F16 : WE_BF16;
+      P.k = planes * p->k;
+      P.kc = P.k;
+      P.k_wrap = p->k;
+      P.x_stride = planes * p->k;
+      P.x_offset = 0;
+    };
+    uint32_t planes = 3;
+    set_planes(3);
+    if (w_dtype == WE_FP8_E4M3 && p->m > 64 && we::gemm_fast_supported(P) && we::gemm_reduce_plan(P).rsplits <= 2)
+      set_planes(planes = 2);
     if (we::gemm_fast_supported(P)) {
       L = P;
       plane_bytes = ((uint64_t)p->m * planes * p->k * 2 + 255) / 256 * 256;
@@ -1087,18 +1095,18 @@ int matmul_impl(we_ctx* ctx, const we_matmul_params* p, int x_dtype, const void*
     L.qk_cos = qk->cos_t;
     L.qk_sin = qk->sin_t;
   }
-  we::GemmReducePlan rp{1, L.k, 0, -1};
+  we::GemmReducePlan rp{1, L.k, 0, -1, 1};
   char* scratch = nullptr;  // the planes of x (plane_bytes), then the split-K partial sums
   if (ctx->tune.gemm_splitk > 0) {  // that many slices (sweeps)
     rp = we::gemm_reduce_plan(L, (uint32_t)ctx->tune.gemm_splitk);
   } else if (ctx->tune.gemm_splitk < 0) {
     rp = noalloc ? we::gemm_reduce_plan(L) : we::gemm_plan(L);
-    if (!noalloc && rp.rsplits > 1) {
+    if (!noalloc && rp.scratch_bytes) {
       scratch = (char*)try_scratch(ctx, plane_bytes + rp.scratch_bytes);
       if (!scratch) rp = we::gemm_reduce_plan(L);
     }
   }
-  const size_t part_bytes = rp.rsplits > 1 ? rp.scratch_bytes : 0;
+  const size_t part_bytes = rp.scratch_bytes;
   if (!scratch && plane_bytes + part_bytes) {
     if (noalloc) {
       // the device's fixed scratch array: no allocation, a hard size limit
@@ -1133,6 +1141,7 @@ int matmul_impl(we_ctx* ctx, const we_matmul_params* p, int x_dtype, const void*
     L.scratch = scratch + plane_bytes;
     L.rsplits = rp.rsplits;
     L.rkc = rp.rkc;
+    L.tail_splits = rp.tail_splits;
   }
   L.rcfg = rp.rcfg;
   const bool qk_fused = has_qk && we::gemm_qk_fusable(L);
