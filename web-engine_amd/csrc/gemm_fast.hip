@@ -186,19 +186,22 @@ GemmReducePlan gemm_plan(const GemmLaunch& L) {
     if (L.qk_cols) us += (slices > 1 || !qk_fusable_cfg(cfg) ? 4.0 : 0.0) + 4.0 * L.m * (double)L.qk_cols / 3e6;
     return us;
   };
-  // The older rules' choice stays unless another is predicted 4% faster (the model's error is of that order: 1500 x 4608 x
-  // 3072 took 55.2 us in the 256 x 128 tiles that it put 2% ahead of the 128 x 128 ones, 54.2 us).
+  // The older rules' choice stays unless another is predicted 6% faster, the model's error: 1500 x 4608 x 3072 took 55.2 us in
+  // the 256 x 128 tiles that it put 2% ahead of the 128 x 128 ones (54.2 us), 700 x 12288 x 4096 with the q / k pass 93.3 us in
+  // 256 x 192 tiles, 5% ahead of the 256 x 256 ones (91.5 us).
   GemmReducePlan best = gemm_reduce_plan(L);
   const uint32_t older = best.rsplits;
   best.rcfg = best.rcfg >= 0 ? best.rcfg : pick_fast_cfg(L.m, L.n, best.rsplits, w8);
-  double best_us = 0.96 * predict(best.rcfg, best.rsplits, best.rsplits > 1 ? best.rkc : L.k);
+  double best_us = 0.94 * predict(best.rcfg, best.rsplits, best.rsplits > 1 ? best.rkc : L.k);
   for (const int cfg : {GEMM_CFG_256x256, GEMM_CFG_256x192, GEMM_CFG_256x128, GEMM_CFG_128x128, GEMM_CFG_64x64}) {
     if (cfg_bm(cfg) == 256 && L.m < 256) continue;
     const uint64_t tiles = (uint64_t)((L.m + cfg_bm(cfg) - 1) / cfg_bm(cfg)) * ((L.n + cfg_bn(cfg) - 1) / cfg_bn(cfg));
     // slices only where the tiles fill at most half of the CUs (128 x 128: twice that), as swept
     const uint32_t most = tiles * 2 <= kCUs * (cfg == GEMM_CFG_128x128 ? 2u : 1u) ? std::min(8u, L.k / 256) : 1u;
-    // three planes of x: no fewer slices than the older plan, whose shorter sums round less (128 x 2048 x 8192 1.6e-7)
-    for (uint32_t rs = three ? older : 1; rs <= most; rs++) {
+    // three planes of x: a multiple of the older plan's slices, whose shorter sums round less and may end with the planes
+    // (800 x 4096 x 8192: error 3.3e-7 in 3 slices, 3.8e-7 in 4)
+    for (uint32_t rs = 1; rs <= most; rs++) {
+      if (three && rs % older) continue;
       const uint32_t kc = (L.k + rs * BK - 1) / (rs * BK) * BK;
       if ((L.k + kc - 1) / kc != rs) continue;
       const double us = predict(cfg, rs, kc);

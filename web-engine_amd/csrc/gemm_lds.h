@@ -1134,9 +1134,10 @@ __device__ __forceinline__ void reduce_epilogue(const FastArgs& a, uint32_t row,
 // XCD (BM, BN > 0): the slices of a tile ran on one XCD (workgroups go round-robin over the 8 XCDs, and the slice
 // index adds a multiple of 8 tiles to the workgroup id), so each reduce workgroup takes a part of a tile of its own
 // XCD and reads the slices there. Otherwise one thread per 4 consecutive outputs in row-major order.
-template <int YT, int BM = 0, int BN = 0>
+template <int YT, int BM = 0, int BN = 0, bool CONV = false>
 __global__ void __launch_bounds__(256) splitk_reduce_kernel(FastArgs a) {
-  if (a.skip_if && *a.skip_if) return;
+  if constexpr (CONV)
+    if (*a.skip_if) return;
   uint32_t row, c0;
   if constexpr (BM > 0) {
     constexpr uint32_t ITEMS = BM * BN / 4, Q = ITEMS / 256;  // reduce workgroups per tile
@@ -1249,18 +1250,18 @@ static hipError_t launch_fast_cfg(FastArgs a, uint32_t splits, int reduce_xcd, h
     if (reduce_in_l2(tiles, a.w_bytes, reduce_xcd)) {
       const dim3 rg(tiles * (BM * BN / 4 / 256));
       switch (a.y_dtype) {
-        case F32: hipLaunchKernelGGL((splitk_reduce_kernel<F32, BM, BN>), rg, dim3(256), 0, s, a); break;
-        case F16: hipLaunchKernelGGL((splitk_reduce_kernel<F16, BM, BN>), rg, dim3(256), 0, s, a); break;
-        default: hipLaunchKernelGGL((splitk_reduce_kernel<BF16, BM, BN>), rg, dim3(256), 0, s, a); break;
+        case F32: hipLaunchKernelGGL((splitk_reduce_kernel<F32, BM, BN, CONV>), rg, dim3(256), 0, s, a); break;
+        case F16: hipLaunchKernelGGL((splitk_reduce_kernel<F16, BM, BN, CONV>), rg, dim3(256), 0, s, a); break;
+        default: hipLaunchKernelGGL((splitk_reduce_kernel<BF16, BM, BN, CONV>), rg, dim3(256), 0, s, a); break;
       }
       return hipGetLastError();
     }
     const size_t threads = (size_t)a.m * ((a.n + 3) / 4);
     const dim3 rg((unsigned)((threads + 255) / 256));
     switch (a.y_dtype) {
-      case F32: hipLaunchKernelGGL(splitk_reduce_kernel<F32>, rg, dim3(256), 0, s, a); break;
-      case F16: hipLaunchKernelGGL(splitk_reduce_kernel<F16>, rg, dim3(256), 0, s, a); break;
-      default: hipLaunchKernelGGL(splitk_reduce_kernel<BF16>, rg, dim3(256), 0, s, a); break;
+      case F32: hipLaunchKernelGGL((splitk_reduce_kernel<F32, 0, 0, CONV>), rg, dim3(256), 0, s, a); break;
+      case F16: hipLaunchKernelGGL((splitk_reduce_kernel<F16, 0, 0, CONV>), rg, dim3(256), 0, s, a); break;
+      default: hipLaunchKernelGGL((splitk_reduce_kernel<BF16, 0, 0, CONV>), rg, dim3(256), 0, s, a); break;
     }
     return hipGetLastError();
   }
