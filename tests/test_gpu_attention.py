@@ -233,3 +233,24 @@ def test_f32_planes_leave_wide_heads_to_the_f32_kernel(graph, tune):
     assert np.array_equal(got[:, :6], f32[:, :6], equal_nan=True)
     assert np.abs(got[:-1, 2:4] - clean[:-1, 2:4]).max() < 1e-5  # every query but the last sees none of the padding
     assert np.abs(got[:, 6:] - clean[:, 6:]).max() < 1e-5
+
+
+@pytest.mark.parametrize("tokens,dim,causal", [(200, 128, True), (200, 128, False), (321, 64, True), (321, 64, False)])
+@pytest.mark.parametrize("what", ["zero q rows", "zero k head", "both zero", "tiny"])
+def test_f32_planes_of_zero_and_tiny_operands(graph, what, tokens, dim, causal):
+    """Scores of 0 (an all-zero query row, an all-zero head of K, both) and scores too small for a normal f32, with masked
+    keys (the causal diagonal, the ragged last tile): the mean of the visible V rows, as softmax of equal scores gives."""
+    heads, kv_heads = 2, 1
+    q, k, v = lcg_random(tokens, [tokens * heads * dim, tokens * kv_heads * dim, tokens * kv_heads * dim])
+    if what == "zero q rows":
+        q.reshape(tokens, -1)[::3] = 0
+        k *= np.float32(2.0 ** -9)
+    elif what == "tiny":
+        q *= np.float32(2.0 ** -100)
+        k *= np.float32(2.0 ** -100)
+    else:
+        k[:] = 0
+        q *= np.float32(2.0 ** -9) if what == "zero k head" else np.float32(0)
+    got = run(graph, q, k, v, we.AttentionShape(tokens, heads, kv_heads, dim, causal=causal), we.F32)
+    want = O.attention(q, k, v, tokens, heads, kv_heads, dim, causal)
+    assert np.abs(got - want).max() < 1e-5

@@ -1306,7 +1306,10 @@ __global__ void __launch_bounds__(64 * NW, 1) attn_planes_kernel(AttnArgs a, con
     const uint32_t se = attn_plane_exp(m);
     const float s = __uint_as_float(se << 23);
     static_for<0, DP / 16>([&](auto S) { attn_split8(v[S], s, qh[S], ql[S]); });
+    // a normal, finite factor: a masked score is -inf times it, and 0 (tiny or zero Q rows against a tiny or zero K head)
+    // would make that a NaN. Where the product of the scales leaves the range, scores round to 0 with the clamped one too.
     sc = a.scale_log2 * __uint_as_float((254u - se) << 23) * a.plane_inv[g];
+    sc = fminf(fmaxf(sc, 1.17549435e-38f), 3.40282347e38f);
   }
   const VtrLane vl = vtr_lane(lane);
   // V^T fragment: dims 32 db + c, the lane's 8 keys of 16 s .. (rows of ROWB bytes). The chunk index (4 db + cc) ^ swz(key)
@@ -1366,7 +1369,7 @@ __global__ void __launch_bounds__(64 * NW, 1) attn_planes_kernel(AttnArgs a, con
     }
     float tmax = sacc[0][0];
     static_for<1, 32>([&](auto I) { tmax = fmaxf(tmax, sacc[I / 16][I % 16]); });
-    tmax = halves_max(tmax) * sc;  // sc > 0
+    tmax = halves_max(tmax) * sc;
     const float mn = fmaxf(m, tmax);
     // the max moves when some query's rises by more than 1 (log2 units): p 2^14 stays below 2^15, in f16's range
     const bool rescale = __any(mn > m + 1.0f);
