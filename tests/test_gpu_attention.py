@@ -254,3 +254,43 @@ def test_f32_planes_of_zero_and_tiny_operands(graph, what, tokens, dim, causal):
     got = run(graph, q, k, v, we.AttentionShape(tokens, heads, kv_heads, dim, causal=causal), we.F32)
     want = O.attention(q, k, v, tokens, heads, kv_heads, dim, causal)
     assert np.abs(got - want).max() < 1e-5
+
+
+@pytest.mark.parametrize("e", [24, 30, 40])
+@pytest.mark.parametrize("tokens,dim", [(200, 128), (330, 64)])
+def test_f32_planes_of_unequal_channels(graph, tokens, dim, e):
+    """Channels of K and V far below or above the others: a small V channel to 1e-5 of its own largest output; a K channel
+    2^e above the others that no query reads; a K channel 2^e below the others that the queries read 2^e times as
+    strongly. Each against the oracle at f32's precision."""
+    heads, kv_heads = 2, 1
+    q, k, v = lcg_random(tokens + e, [tokens * heads * dim, tokens * kv_heads * dim, tokens * kv_heads * dim])
+    q2, k2, v2 = q.reshape(tokens, heads, dim), k.reshape(tokens, dim), v.reshape(tokens, dim)
+    v2[:, 3] *= np.float32(2.0 ** -e)
+    k2[:, 5] *= np.float32(2.0 ** e)
+    q2[:, :, 5] = 0
+    k2[:, 7] *= np.float32(2.0 ** -e)
+    q2[:, :, 7] *= np.float32(2.0 ** e)
+    for causal in (False, True):
+        got = run(graph, q, k, v, we.AttentionShape(tokens, heads, kv_heads, dim, causal=causal), we.F32)
+        got = got.reshape(-1, dim)
+        want = O.attention(q, k, v, tokens, heads, kv_heads, dim, causal).reshape(-1, dim)
+        assert np.abs(got - want).max() < 1e-5
+        assert O.rel_error(got[:, 3], want[:, 3]) < 1e-5
+
+
+@pytest.mark.parametrize("e", [24, 30, 40])
+def test_f32_planes_of_one_large_value(graph, tune, e):
+    """One value of V, of K or of a query 2^e above the rest of its channel or row, which the other queries' results do not
+    contain (causal, at the last token): every one of those to f32's precision, and the query's own scores too."""
+    tokens, heads, kv_heads, dim = 300, 6, 3, 128
+    q, k, v = lcg_random(e, [tokens * heads * dim, tokens * kv_heads * dim, tokens * kv_heads * dim])
+    q3, k3, v3 = q.reshape(tokens, heads, dim), k.reshape(tokens, kv_heads, dim), v.reshape(tokens, kv_heads, dim)
+    v3[-1, 0, 9] = 2.0 ** e
+    k3[-1, 1, 9] = 2.0 ** e
+    k3[:, 2, 9] = 0
+    q3[100, 4, 9] = 2.0 ** e  # meets only zeros
+    got = run(graph, q, k, v, we.AttentionShape(tokens, heads, kv_heads, dim, causal=True), we.F32)
+    want = O.attention(q, k, v, tokens, heads, kv_heads, dim, True)
+    got, want = got.reshape(tokens, heads, dim), want.reshape(tokens, heads, dim)
+    assert np.abs(got[:-1] - want[:-1]).max() < 1e-5
+    assert np.abs(got[:-1, :2, 9] - want[:-1, :2, 9]).max() < 1e-5

@@ -55,10 +55,12 @@ struct AttnArgs {
   uint32_t nqb;                        // query blocks per head
   float scale_log2;                    // log2(e) / sqrt(dim)
   int causal;
-  // f32 through f16 planes (attn_planes_kernel): per kv head, then again for V, the inverse scale of its planes and
-  // whether its values are too far apart for them (the f32 MFMA kernel computes those heads). NULL: no planes
+  // f32 through f16 planes (attn_planes_kernel), NULL: no planes. plane_inv: the inverse scales of K's channels
+  // [kv_heads, dim], then V's. What the planes cannot hold goes to the f32 MFMA kernel: plane_head[g] != 0, kv head g
+  // with its queries; plane_rows[h * (blocks of 128 queries) + block] != 0, that block of head h
   const float* plane_inv;
-  const uint32_t* plane_flag;
+  uint32_t* plane_head;
+  uint32_t* plane_rows;
   uint32_t kv_heads;
 };
 
@@ -1034,7 +1036,7 @@ __global__ void __launch_bounds__(ATT_NT, 1) attn32_kernel(AttnArgs a) {
   uint32_t qb, h;
   block_coords(a, qb, h);
   const uint32_t g = h / a.group;
-  if (a.plane_flag && !(a.plane_flag[g] | a.plane_flag[a.kv_heads + g])) return;  // attn_planes_kernel has this head
+  if (a.plane_head && !a.plane_head[g] && !a.plane_rows[h * a.nqb + qb]) return;  // attn_planes_kernel has these queries
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 31, hf = lane >> 5;
@@ -1149,49 +1151,54 @@ __global__ void __launch_bounds__(ATT_NT, 1) attn32_kernel(AttnArgs a) {
 // ------------------------------------------------------------------------------------ f32 through f16 planes
 // Head dim 64 or 128. Every f32 operand is a power of two times the sum of two f16 planes, hi = f16(v 2^e) and
 // lo = f16(v 2^e - hi) (v to 2^-23 of itself), and each product runs as lo x hi + hi x lo + hi x hi on the 32x32x16 f16
-// MFMA with f32 sums: 3/16 of the cycles of the f32 MFMA. K and V are split once per call into scratch, with one scale per kv head;
-// Q rows and P are split in registers. The planes hold a value to 2^-40 of its head's largest, so a head where some
-// row's largest value lies below 2^-16 of the head's largest, or with an inf or NaN, is flagged and left to the f32
-// MFMA kernel, which is launched behind this one and returns at once for the other heads.
-// below, the two passes over K and V and the third launch cost what the products gain (24 heads of 128, 128 tokens: 23.7 us
-// here, 24.4 us on the f32 MFMA; 16 heads, 64 tokens 17.0 and 13.1, 200 tokens causal 27.1 and 41.8)
-// (head dim 64: twice that; 170 tokens causal gained 5% and its error rose from 2.2e-7 to 2.3e-7)
+// MFMA with f32 sums: 3/16 of the cycles of the f32 MFMA. K and V are split once per call into scratch, Q rows and P in
+// registers. The scales: one per channel of a kv head for K, whose inverse goes into Q, and for V, undone in the outputs;
+// one per row of Q; 2^14 for P. So a channel that is small or large everywhere costs no bits.
+// Below 2^-18 of its scale's largest a value loses bits, below 2^-40 it is 0. Few such values are left as they are (a
+// channel of 1103 normal ones holds 0.01 in the mean); the f32 MFMA kernel, which is launched behind and otherwise returns
+// at once, computes
+//  * kv heads with more than 2 + tokens / 256 of them in a channel, with a token whose values all lie below 2^-16 of their
+//    channels' largest, with an inf or NaN, or with a K value of 2^96 or more (its inverse scale could take Q out of range),
+//  * blocks of 128 queries with a Q row that holds more than 2, or more than one to 32 others.
+// With fewer tokens than PLANES_MIN_TOKENS (head dim 64: than twice that) the two passes over K and V and the third launch
+// cost what the products gain: 24 heads of 128, 128 tokens 23.7 us here and 24.4 us on the f32 MFMA; 16 heads, 64 tokens
+// 17.0 and 13.1, 200 tokens causal 27.1 and 41.8; head dim 64, 170 tokens causal 5% less time at an error of 2.3e-7 for 2.2e-7.
 constexpr uint32_t PLANES_MIN_TOKENS = 160;
 constexpr uint32_t PLANE_BLOCKS = 16;  // workgroups per kv head of the scan for the largest values
+constexpr uint32_t PLANE_TINY = 123u << 23;  // 2^-4, 2^-18 of the largest scaled value's power of two
 
-// The per-workgroup largest row maximum and smallest nonzero one (0: an inf or NaN) of a kv head's rows: K (z 0), V (1).
+// The per-workgroup largest |value| (its bits; an inf or NaN is larger than any) of each channel of a kv head: K (z 0),
+// V (1). Clears the split's counts and flags.
 template <int DP>
-__global__ void __launch_bounds__(256) attn_amax_kernel(AttnArgs a, uint32_t* __restrict__ part) {
+__global__ void __launch_bounds__(256) attn_amax_kernel(AttnArgs a, uint32_t* __restrict__ part,
+                                                        uint32_t* __restrict__ count) {
   constexpr int LPR = DP / 8;  // lanes per row
-  __shared__ uint32_t rmax[4], rmin[4];
-  const uint32_t g = blockIdx.y, z = blockIdx.z;
+  __shared__ uint32_t red[4][DP];
+  const uint32_t g = blockIdx.y, z = blockIdx.z, head = z * a.kv_heads + g;
   const float* src = (const float*)(z ? a.v : a.k) + (size_t)g * DP;
   const size_t stride = z ? a.vs : a.ks;
-  const uint32_t sub = threadIdx.x % LPR, r0 = threadIdx.x / LPR;
-  uint32_t big = 0, small = 0xffffffffu;
+  const uint32_t t = threadIdx.x, sub = t % LPR, r0 = t / LPR;
+  if (blockIdx.x == 0) {
+    if (t < DP) count[head * DP + t] = 0;
+    if (t == 0 && z == 0) a.plane_head[g] = 0;
+  }
+  uint32_t m[8] = {};
   for (uint32_t r = blockIdx.x * (256 / LPR) + r0; r < a.tokens; r += PLANE_BLOCKS * (256 / LPR)) {
     const float* p = src + r * stride + sub * 8;
     const u32x4 v0 = *(const u32x4*)p, v1 = *(const u32x4*)(p + 4);
-    uint32_t m = 0;
 #pragma unroll
-    for (int e = 0; e < 4; e++) m = max(m, max(v0[e] & 0x7fffffffu, v1[e] & 0x7fffffffu));
-#pragma unroll
-    for (int d = LPR / 2; d >= 1; d >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, d, LPR));
-    if (m >= 0x7f800000u) small = 0;
-    else if (m) big = max(big, m), small = min(small, m);
+    for (int e = 0; e < 4; e++) m[e] = max(m[e], v0[e] & 0x7fffffffu), m[4 + e] = max(m[4 + e], v1[e] & 0x7fffffffu);
   }
 #pragma unroll
-  for (int d = 32; d >= 1; d >>= 1) {
-    big = max(big, (uint32_t)__shfl_xor((int)big, d, 64));
-    small = min(small, (uint32_t)__shfl_xor((int)small, d, 64));
+  for (int d = LPR; d < 64; d <<= 1)
+#pragma unroll
+    for (int e = 0; e < 8; e++) m[e] = max(m[e], (uint32_t)__shfl_xor((int)m[e], d, 64));
+  if ((t & 63) < LPR) {
+#pragma unroll
+    for (int e = 0; e < 8; e++) red[t >> 6][sub * 8 + e] = m[e];
   }
-  if ((threadIdx.x & 63) == 0) rmax[threadIdx.x >> 6] = big, rmin[threadIdx.x >> 6] = small;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    uint32_t* p = part + ((z * a.kv_heads + g) * PLANE_BLOCKS + blockIdx.x) * 2;
-    p[0] = max(max(rmax[0], rmax[1]), max(rmax[2], rmax[3]));
-    p[1] = min(min(rmin[0], rmin[1]), min(rmin[2], rmin[3]));
-  }
+  if (t < DP) part[(head * PLANE_BLOCKS + blockIdx.x) * DP + t] = max(max(red[0][t], red[1][t]), max(red[2][t], red[3][t]));
 }
 
 // biased exponent of the power of two that brings the largest value (its bits) into [2^14, 2^15)
@@ -1200,40 +1207,65 @@ __device__ __forceinline__ uint32_t attn_plane_exp(uint32_t bits) {
   return e < 253u ? e : 253u;
 }
 
-// 8 f32 values times s -> their f16 planes
-__device__ __forceinline__ void attn_split8(const float (&v)[8], float s, u32x4& hi, u32x4& lo) {
+// 8 f32 values -> their f16 planes
+__device__ __forceinline__ void attn_split8(const float (&v)[8], u32x4& hi, u32x4& lo) {
   const std::true_type f16{};
 #pragma unroll
   for (int i = 0; i < 4; i++) {
-    const float x = v[2 * i] * s, y = v[2 * i + 1] * s;
+    const float x = v[2 * i], y = v[2 * i + 1];
     hi[i] = pack2(x, y, f16);
     lo[i] = pack2(x - f16_to_f32((uint16_t)(hi[i] & 0xffffu)), y - f16_to_f32((uint16_t)(hi[i] >> 16)), f16);
   }
 }
 
-// K (z 0) and V (1) -> f16 [tokens, kv_heads, hi | lo, DP], with each head's inverse scale and flag.
+// K (z 0) and V (1) -> f16 [tokens, kv_heads, hi | lo, DP], the channels' inverse scales and the heads' flags.
 template <int DP>
 __global__ void __launch_bounds__(256) attn_split_kernel(AttnArgs a, const uint32_t* __restrict__ part,
-                                                         uint16_t* __restrict__ kp, uint16_t* __restrict__ vp,
-                                                         float* __restrict__ inv, uint32_t* __restrict__ flag) {
+                                                         uint32_t* __restrict__ count, uint16_t* __restrict__ kp,
+                                                         uint16_t* __restrict__ vp, float* __restrict__ inv) {
   constexpr int LPR = DP / 8;
-  const uint32_t g = blockIdx.y, z = blockIdx.z;
-  const uint32_t* p = part + (z * a.kv_heads + g) * PLANE_BLOCKS * 2;
-  uint32_t big = 0, small = 0xffffffffu;
+  __shared__ __attribute__((aligned(16))) float scale[DP];
+  const uint32_t g = blockIdx.y, z = blockIdx.z, head = z * a.kv_heads + g, t = threadIdx.x;
+  if (t < DP) {
+    const uint32_t* p = part + head * PLANE_BLOCKS * DP + t;
+    uint32_t big = 0;
 #pragma unroll
-  for (uint32_t i = 0; i < PLANE_BLOCKS; i++) big = max(big, p[2 * i]), small = min(small, p[2 * i + 1]);
-  const uint32_t se = attn_plane_exp(big);
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    inv[z * a.kv_heads + g] = __uint_as_float((254u - se) << 23);
-    flag[z * a.kv_heads + g] = small == 0u || (big >> 23) > (small >> 23) + 16u ? 1u : 0u;
+    for (uint32_t i = 0; i < PLANE_BLOCKS; i++) big = max(big, p[i * DP]);
+    const uint32_t se = attn_plane_exp(big);
+    scale[t] = __uint_as_float(se << 23);
+    if (blockIdx.x == 0) {
+      inv[head * DP + t] = __uint_as_float((254u - se) << 23);
+      if (big >= (z ? 255u : 127u + 96u) << 23) atomicOr(&a.plane_head[g], 1u);
+    }
   }
-  const uint32_t r = blockIdx.x * (256 / LPR) + threadIdx.x / LPR, d = threadIdx.x % LPR * 8;
+  __syncthreads();
+  const uint32_t r = blockIdx.x * (256 / LPR) + t / LPR, d = t % LPR * 8;
+  float v[8] = {};
+  uint32_t m = 0, tiny = 0;
+  if (r < a.tokens) {
+    const float* src = (const float*)(z ? a.v : a.k) + r * (size_t)(z ? a.vs : a.ks) + (size_t)g * DP + d;
+    const f32x4 v0 = *(const f32x4*)src, v1 = *(const f32x4*)(src + 4);
+    const f32x4 s0 = *(const f32x4*)(scale + d), s1 = *(const f32x4*)(scale + d + 4);
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+      v[e] = e < 4 ? v0[e & 3] * s0[e & 3] : v1[e & 3] * s1[e & 3];
+      const uint32_t b = __float_as_uint(v[e]) & 0x7fffffffu;
+      m = max(m, b);
+      if (b && b < PLANE_TINY) tiny |= 1u << e;
+    }
+  }
+#pragma unroll
+  for (int x = LPR / 2; x >= 1; x >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, x, LPR));
+  if (m && m < 125u << 23) atomicOr(&a.plane_head[g], 1u);  // the whole token below 2^-2
+  if (tiny && !__hip_atomic_load(&a.plane_head[g], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+#pragma unroll
+    for (int e = 0; e < 8; e++)
+      if ((tiny >> e & 1u) && atomicAdd(&count[head * DP + d + e], 1u) >= 2u + a.tokens / 256u)
+        atomicOr(&a.plane_head[g], 1u);
+  }
   if (r >= a.tokens) return;
-  const float* src = (const float*)(z ? a.v : a.k) + r * (size_t)(z ? a.vs : a.ks) + (size_t)g * DP + d;
-  const f32x4 v0 = *(const f32x4*)src, v1 = *(const f32x4*)(src + 4);
-  const float v[8] = {v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
   u32x4 hi, lo;
-  attn_split8(v, __uint_as_float(se << 23), hi, lo);
+  attn_split8(v, hi, lo);
   uint16_t* o = (z ? vp : kp) + ((size_t)r * a.kv_heads + g) * 2 * DP + d;
   *(u32x4*)o = hi;
   *(u32x4*)(o + DP) = lo;
@@ -1255,7 +1287,7 @@ __global__ void __launch_bounds__(64 * NW, 1) attn_planes_kernel(AttnArgs a, con
   uint32_t qb, h;
   block_coords(a, qb, h);
   const uint32_t g = h / a.group;
-  if (a.plane_flag[g] | a.plane_flag[a.kv_heads + g]) return;
+  if (a.plane_head[g]) return;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 31, hf = lane >> 5;
@@ -1284,16 +1316,19 @@ __global__ void __launch_bounds__(64 * NW, 1) attn_planes_kernel(AttnArgs a, con
   };
   if (nt > 0) issue(0, 0);
 
-  // Q planes: query qi, dims 16 s + 8 hf .. + 7, scaled by the row's own power of two
+  // Q planes: query qi, dims 16 s + 8 hf .. + 7, times K's inverse scales, scaled by the row's own power of two
   u32x4 qh[DP / 16], ql[DP / 16];
   float sc;  // scores -> log2 units
   {
     float v[DP / 16][8];
-    uint32_t m = 0;
+    uint32_t m = 0, tiny = 0, others = 0;
+    const float* kinv = a.plane_inv + g * DP + 8 * hf;
     static_for<0, DP / 16>([&](auto S) {
       const float* p = (const float*)a.q + (size_t)qi * a.qs + (size_t)h * DP + 16 * S + 8 * hf;
       f32x4 v0 = {0, 0, 0, 0}, v1 = {0, 0, 0, 0};
       if (qi < a.tokens) v0 = *(const f32x4*)p, v1 = *(const f32x4*)(p + 4);
+      v0 *= *(const f32x4*)(kinv + 16 * S);
+      v1 *= *(const f32x4*)(kinv + 16 * S + 4);
       static_for<0, 4>([&](auto E) {
         constexpr int e = E;
         v[S][e] = v0[e];
@@ -1305,11 +1340,27 @@ __global__ void __launch_bounds__(64 * NW, 1) attn_planes_kernel(AttnArgs a, con
     m = max(m, (uint32_t)__shfl_xor((int)m, 32, 64));
     const uint32_t se = attn_plane_exp(m);
     const float s = __uint_as_float(se << 23);
-    static_for<0, DP / 16>([&](auto S) { attn_split8(v[S], s, qh[S], ql[S]); });
-    // a normal, finite factor: a masked score is -inf times it, and 0 (tiny or zero Q rows against a tiny or zero K head)
-    // would make that a NaN. Where the product of the scales leaves the range, scores round to 0 with the clamped one too.
-    sc = a.scale_log2 * __uint_as_float((254u - se) << 23) * a.plane_inv[g];
-    sc = fminf(fmaxf(sc, 1.17549435e-38f), 3.40282347e38f);
+    static_for<0, DP / 16>([&](auto S) {
+      static_for<0, 8>([&](auto E) {
+        v[S][E] *= s;
+        const uint32_t b = __float_as_uint(v[S][E]) & 0x7fffffffu;
+        tiny += b && b < PLANE_TINY ? 1u : 0u;
+        others += b >= PLANE_TINY ? 1u : 0u;
+      });
+      attn_split8(v[S], qh[S], ql[S]);
+    });
+    tiny += (uint32_t)__shfl_xor((int)tiny, 32, 64);
+    others += (uint32_t)__shfl_xor((int)others, 32, 64);
+    const int wide = __syncthreads_or(qi < a.tokens && (tiny > 2u || 32u * tiny > others));
+    const uint32_t nb = (a.tokens + ATT_BM - 1) / ATT_BM, b0 = q0 / ATT_BM;  // blocks of the f32 MFMA kernel
+    if (tid < NW / 4 && b0 + tid < nb) a.plane_rows[h * nb + b0 + tid] = wide ? 1u : 0u;
+    if (wide) {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the first tile's loads write LDS
+      return;
+    }
+    // a normal, finite factor: a masked score is -inf times it, and 0 (tiny or zero Q rows) would make that a NaN. Where
+    // the scale leaves the range, scores round to 0 with the clamped one too.
+    sc = fminf(fmaxf(a.scale_log2 * __uint_as_float((254u - se) << 23), 1.17549435e-38f), 3.40282347e38f);
   }
   const VtrLane vl = vtr_lane(lane);
   // V^T fragment: dims 32 db + c, the lane's 8 keys of 16 s .. (rows of ROWB bytes). The chunk index (4 db + cc) ^ swz(key)
@@ -1414,15 +1465,16 @@ __global__ void __launch_bounds__(64 * NW, 1) attn_planes_kernel(AttnArgs a, con
     });
   }
 
-  const float inv = a.plane_inv[a.kv_heads + g] / halves_sum(l);
+  const float inv = 1.0f / halves_sum(l);
   if (qi < a.tokens) {
+    const float* vinv = a.plane_inv + (a.kv_heads + g) * DP + 4 * hf;
     float* O = (float*)a.o + (size_t)qi * a.os + (size_t)h * DP;
     static_for<0, DP / 32>([&](auto D) {
       constexpr int db = D;
       static_for<0, 4>([&](auto G) {
         constexpr int g4 = G;
-        *(f32x4*)(O + 32 * db + 8 * g4 + 4 * hf) = f32x4{o[db][4 * g4] * inv, o[db][4 * g4 + 1] * inv,
-                                                        o[db][4 * g4 + 2] * inv, o[db][4 * g4 + 3] * inv};
+        const f32x4 r = f32x4{o[db][4 * g4], o[db][4 * g4 + 1], o[db][4 * g4 + 2], o[db][4 * g4 + 3]} * inv;
+        *(f32x4*)(O + 32 * db + 8 * g4 + 4 * hf) = r * *(const f32x4*)(vinv + 32 * db + 8 * g4);
       });
     });
   }
@@ -1449,7 +1501,7 @@ bool attn_ring_path(const AttnLaunch& L) { return L.path == 2; }
 
 // f32 through f16 planes: scratch layout (bytes), 0 where the path does not apply
 struct PlanesLayout {
-  size_t vp, part, inv, flag, bytes;
+  size_t vp, part, count, inv, head, rows, bytes;
 };
 bool attn_planes_ok(const AttnLaunch& L, PlanesLayout& p) {
   if (L.dtype != F32 || (L.dim != 64 && L.dim != 128) || L.path != 0 || L.heads == 0 ||
@@ -1458,10 +1510,13 @@ bool attn_planes_ok(const AttnLaunch& L, PlanesLayout& p) {
   const uint64_t plane = (uint64_t)L.tokens * L.kv_heads * 2 * L.dim * 2;
   if (plane >= kAttInvalid || L.kv_heads > 65535) return false;
   p.vp = (plane + 255) / 256 * 256;
+  const size_t words = ((size_t)2 * L.kv_heads * L.dim * 4 + 255) / 256 * 256;  // one per channel of K and V
   p.part = 2 * p.vp;
-  p.inv = p.part + ((size_t)2 * L.kv_heads * PLANE_BLOCKS * 8 + 255) / 256 * 256;
-  p.flag = p.inv + ((size_t)2 * L.kv_heads * 4 + 255) / 256 * 256;
-  p.bytes = p.flag + (size_t)2 * L.kv_heads * 4;
+  p.count = p.part + PLANE_BLOCKS * words;
+  p.inv = p.count + words;
+  p.head = p.inv + words;
+  p.rows = p.head + ((size_t)L.kv_heads * 4 + 255) / 256 * 256;
+  p.bytes = p.rows + (size_t)((L.tokens + ATT_BM - 1) / ATT_BM) * L.heads * 4;
   return true;
 }
 
@@ -1469,13 +1524,14 @@ template <int DP>
 hipError_t launch_planes(AttnArgs a, const AttnLaunch& L, const PlanesLayout& p, hipStream_t s) {
   char* base = (char*)L.scratch;
   uint16_t *kp = (uint16_t*)base, *vp = (uint16_t*)(base + p.vp);
-  uint32_t* part = (uint32_t*)(base + p.part);
+  uint32_t *part = (uint32_t*)(base + p.part), *count = (uint32_t*)(base + p.count);
   a.plane_inv = (const float*)(base + p.inv);
-  a.plane_flag = (const uint32_t*)(base + p.flag);
+  a.plane_head = (uint32_t*)(base + p.head);
+  a.plane_rows = (uint32_t*)(base + p.rows);
   constexpr uint32_t rows = 256 / (DP / 8);
-  hipLaunchKernelGGL(attn_amax_kernel<DP>, dim3(PLANE_BLOCKS, L.kv_heads, 2), dim3(256), 0, s, a, part);
+  hipLaunchKernelGGL(attn_amax_kernel<DP>, dim3(PLANE_BLOCKS, L.kv_heads, 2), dim3(256), 0, s, a, part, count);
   hipLaunchKernelGGL(attn_split_kernel<DP>, dim3((L.tokens + rows - 1) / rows, L.kv_heads, 2), dim3(256), 0, s, a, part,
-                     kp, vp, (float*)(base + p.inv), (uint32_t*)(base + p.flag));
+                     count, kp, vp, (float*)(base + p.inv));
   // 4 waves (128 queries) per workgroup while the workgroups then still fit one round of the CUs, else 8
   const uint32_t n4 = (L.tokens + 127) / 128;
   if ((uint64_t)n4 * L.heads <= 256) {
@@ -1486,7 +1542,7 @@ hipError_t launch_planes(AttnArgs a, const AttnLaunch& L, const PlanesLayout& p,
     hipLaunchKernelGGL((attn_planes_kernel<DP, 8>), dim3(a.nqb * L.heads), dim3(512), 0, s, a, kp, vp);
   }
   a.nqb = (L.tokens + ATT_BM - 1) / ATT_BM;
-  return launch_attn(attn32_kernel<DP>, a, s);  // the flagged heads
+  return launch_attn(attn32_kernel<DP>, a, s);  // the flagged heads and blocks
 }
 }  // namespace
 
@@ -1518,7 +1574,8 @@ hipError_t attention_launch(const AttnLaunch& L, hipStream_t s) {
   a.scale_log2 = 1.4426950408889634f / sqrtf((float)L.dim);
   a.causal = L.causal;
   a.plane_inv = nullptr;
-  a.plane_flag = nullptr;
+  a.plane_head = nullptr;
+  a.plane_rows = nullptr;
   a.kv_heads = L.kv_heads;
   PlanesLayout p;
   if (L.scratch && attn_planes_ok(L, p)) return L.dim == 64 ? launch_planes<64>(a, L, p, s) : launch_planes<128>(a, L, p, s);
