@@ -744,6 +744,25 @@ def test_conv3x3_planes_leave_wide_images_to_the_general_kernel(graph, tune):
     assert O.rel_error(inf[ok], general[ok]) < 4e-6
 
 
+def _conv(graph, h, w, cin, cout, x, wt, w_dt=we.F32):
+    w_store, ow = (O.bf16_rne(wt.reshape(-1)), O.BF16) if w_dt == we.BF16 else (wt.reshape(-1), O.F32)
+    got = run(graph, we.conv3x3_params(h, w, cin, cout, graph=graph), x.reshape(-1), we.F32, w_store, w_dt, we.F32)
+    want = O.matmul(O.conv3x3_params(h, w, cin, cout), O.F32, x.reshape(-1), ow, w_store)
+    return got.reshape(-1, cout), want.reshape(-1, cout)
+
+
+@pytest.mark.parametrize("ex,ew", [(110, -100), (-110, 100), (60, -100)])
+def test_conv3x3_planes_of_large_and_small_operands(graph, ex, ew):
+    """An image at 2^ex against weights at 2^ew: the results fit f32 well, so no product of a sum with one of the planes' two
+    scales alone may leave its range."""
+    h, w, cin, cout = 12, 17, 64, 48
+    rng = np.random.default_rng(1)
+    x = rng.standard_normal((h * w, cin)).astype(np.float32) * np.float32(2.0 ** ex)
+    wt = rng.standard_normal((cout, 9 * cin)).astype(np.float32) * np.float32(2.0) ** np.float32(ew)
+    got, want = _conv(graph, h, w, cin, cout, x, wt)
+    assert O.rel_error(got, want) < 1e-5
+
+
 @pytest.mark.parametrize("k", [128, 1024])  # two f16 planes; three bf16 planes (a K-sliced plan)
 def test_f32_rows_of_any_scale(graph, k):
     """The two f16 planes of an f32 row carry a power of two of the row's own: rows at 2^100, 2^-100, all zeros and with one

@@ -125,7 +125,6 @@ hipError_t conv_fast_launch(const GemmLaunch& L, void* scratch, hipStream_t s) {
   a.y_dtype = (uint32_t)L.y_dtype;
   a.vec_store = ((uintptr_t)L.y % (4 * yb) == 0 && L.y_offset % 4 == 0 && L.y_stride % 4 == 0) ? 1u : 0u;
   a.row_scale = inv;
-  a.row_scale_step = 0;
   a.col_scale = col_scale;
   a.conv_width = L.conv_width;
   a.conv_cin = L.conv_cin;

@@ -276,7 +276,6 @@ FastArgs fast_args(const GemmLaunch& L, uint32_t kc) {
   a.kwrap = L.k_wrap ? L.k_wrap : 0xffffffffu;
   a.kwrap2 = L.k_wrap ? 2 * L.k_wrap : 0xffffffffu;
   a.row_scale = L.row_scale;
-  a.row_scale_step = 1;
   a.scale = L.scale;
   a.x_stride = L.x_stride;
   a.w_stride = L.w_stride;

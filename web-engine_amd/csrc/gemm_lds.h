@@ -71,11 +71,10 @@ struct FastArgs {
   // int4 weights (w: u32 [N, K / 8], rows contiguous): f16 scales [N, sc_groups], one per sc_blocks 64-k blocks
   const uint16_t* sc;
   uint32_t sc_groups, sc_blocks;
-  // f32 operands as two f16 planes (split_f32_f16x2_kernel): the sums of row r times row_scale[r * row_scale_step] (and,
-  // convolution, of column c times col_scale[c]), the powers of two that the planes were scaled by. NULL: none
+  // f32 operands as two f16 planes (split_f32_f16x2_kernel): the sums of row r times row_scale[r] (convolution: of column
+  // c times row_scale[0] and col_scale[c]), the powers of two that the planes were scaled by. NULL: none
   const float* row_scale;
   const float* col_scale;
-  uint32_t row_scale_step;
   // 3x3 convolution input (CONV kernels): x holds an f16 image [m / conv_width, conv_width, 2 conv_cin], the lo and hi
   // plane of each pixel; k runs over segments of conv_kp (9 conv_cin rounded up to 64; tap, channel), the first with
   // the lo plane, the others with the hi plane. conv_magic = ceil(2^32 / conv_cin)
@@ -819,30 +818,32 @@ __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64) gemm_lds_kernel(FastArg
     }
   };
 
-  if constexpr (IS_F16 && (B8 || CONV)) {
-    // two-plane f32 operands: undo the planes' scaling (powers of two)
+  if constexpr (CONV) {
+    // undo the planes' scaling, the image's and the column's powers of two together: one after the other could leave
+    // f32's range where the sum's own size does not (an image at 2^110 against weights at 2^-100)
+    const int re = (int)(__float_as_uint(*a.row_scale) >> 23) - 254;
+#pragma unroll
+    for (int rc = 0; rc < RC; rc++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const uint32_t c = col0 + wn * WTN + ccol(rc) + lcol + e;
+        const int ce = re + (int)(__float_as_uint(a.col_scale[c < a.n ? c : 0u]) >> 23);
+#pragma unroll
+        for (int i = 0; i < RR; i++) {
+          if constexpr (PP) acc[i][rc][e] = ldexpf(acc[i][rc][e], ce);
+          else acc[i][rc >> 2][4 * (rc & 3) + e] = ldexpf(acc[i][rc >> 2][4 * (rc & 3) + e], ce);
+        }
+      }
+  } else if constexpr (IS_F16 && B8) {
+    // two-plane f32 rows: undo the planes' scaling (powers of two)
     if (a.row_scale) {
 #pragma unroll
       for (int i = 0; i < RR; i++) {
         const uint32_t row = row0 + wm * WTM + i * RS + lrow;
-        const float rs = a.row_scale[(row < a.m ? row : 0u) * a.row_scale_step];
+        const float rs = a.row_scale[row < a.m ? row : 0u];
 #pragma unroll
         for (int j = 0; j < (PP ? TN16 : TN); j++) acc[i][j] *= rs;
       }
-    }
-    if constexpr (CONV) {
-#pragma unroll
-      for (int rc = 0; rc < RC; rc++)
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-          const uint32_t c = col0 + wn * WTN + ccol(rc) + lcol + e;
-          const float cs = a.col_scale[c < a.n ? c : 0u];
-#pragma unroll
-          for (int i = 0; i < RR; i++) {
-            if constexpr (PP) acc[i][rc][e] *= cs;
-            else acc[i][rc >> 2][4 * (rc & 3) + e] *= cs;
-          }
-        }
     }
   }
 
