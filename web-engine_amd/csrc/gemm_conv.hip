@@ -1,7 +1,7 @@
 // The 3x3 convolution of an f32 channel-last image (src/kernels/matmul.ts:74-83) on the tiles of gemm_lds.h. The image
 // and f32 weights are split into two f16 planes each in scratch (kernels_misc.hip), bf16 weights into one, and one GEMM
 // runs over the plane products lo x hi, hi x lo, hi x hi (bf16 weights: lo x w, hi x w) along K, with the pixels of each
-// tap gathered by the direct-to-LDS loads' addresses. 128 x 128 pixels, 384 -> 384 channels: 3 x 43.5 GFLOP of MFMA.
+// tap gathered by the direct-to-LDS loads' addresses; lo planes carry another 2^12, which the sums lose before hi x hi. 128 x 128 pixels, 384 -> 384 channels: 3 x 43.5 GFLOP of MFMA.
 #include <algorithm>
 
 #include "gemm_lds.h"
@@ -92,14 +92,15 @@ hipError_t conv_fast_launch(const GemmLaunch& L, void* scratch, hipStream_t s) {
   uint16_t* weights = (uint16_t*)(base + p.weights);
   float* col_scale = (float*)(base + p.col_scale);
   float* inv = (float*)(base + p.misc);
-  uint32_t* flag = (uint32_t*)(base + p.misc + 128);
+  uint32_t* range = (uint32_t*)(base + p.misc + 128);
   hipError_t e =
-      launch_image_f16x2((const float*)L.x, L.m, L.conv_cin, (uint32_t*)(base + p.misc + 256), image, inv, flag, s);
+      launch_image_f16x2((const float*)L.x, L.m, L.conv_cin, (uint32_t*)(base + p.misc + 256), image, inv, range, s);
   if (e != hipSuccess) return e;
   const int wb = L.w_dtype == F32 ? 4 : 2, wplanes = (int)p.segments - 1;
-  // weight rows hi | lo (f32) or hi (bf16: 8 significant bits, exact in f16 down to 2^-31 of the row's largest)
+  // weight rows hi | lo (f32) or hi (bf16: 8 significant bits, exact in f16 down to 2^-31 of the row's largest: tiny ones are
+  // those below, too)
   e = launch_split_f32_f16x2((const char*)L.w + (uint64_t)L.w_offset * wb, L.w_dtype, L.n, L.k, L.w_stride, weights, p.kp,
-                             wplanes, wplanes == 2 ? 1 : -1, 0, col_scale, s);
+                             wplanes, wplanes == 2 ? 1 : -1, 0, col_scale, range, s);
   if (e != hipSuccess) return e;
   const int yb = L.y_dtype == F32 ? 4 : 2;
   FastArgs a{};
@@ -129,6 +130,7 @@ hipError_t conv_fast_launch(const GemmLaunch& L, void* scratch, hipStream_t s) {
   a.conv_width = L.conv_width;
   a.conv_cin = L.conv_cin;
   a.conv_kp = p.kp;
+  a.conv_hi = a.k - p.kp;
   a.conv_magic = (uint32_t)(((1ull << 32) + L.conv_cin - 1) / L.conv_cin);
   uint32_t splits = 1;
   if (p.rsplits > 1) {
@@ -136,15 +138,15 @@ hipError_t conv_fast_launch(const GemmLaunch& L, void* scratch, hipStream_t s) {
     a.rsplits = splits = p.rsplits;
     a.kc = p.rkc;
   }
-  a.skip_if = flag;
+  a.skip_if = range;
   switch (p.cfg) {
     case GEMM_CFG_256x192: e = launch_fast_cfg<256, 192, 4, 2, true, F16, 2, true, true>(a, splits, L.reduce_xcd, s); break;
     case GEMM_CFG_128x128: e = launch_fast_cfg<128, 128, 2, 2, true, F16, 2, false, true>(a, splits, L.reduce_xcd, s); break;
     default: e = launch_fast_cfg<64, 64, 2, 2, true, F16, 3, false, true>(a, splits, L.reduce_xcd, s); break;
   }
   if (e != hipSuccess) return e;
-  GemmLaunch G = L;  // a flagged image: the general kernel (its workgroups return at once for any other)
-  G.only_if = flag;
+  GemmLaunch G = L;  // flagged operands: the general kernel (its workgroups return at once for any others)
+  G.only_if = range;
   return gemm_launch(G, s);
 }
 

@@ -79,6 +79,7 @@ struct FastArgs {
   // plane of each pixel; k runs over segments of conv_kp (9 conv_cin rounded up to 64; tap, channel), the first with
   // the lo plane, the others with the hi plane. conv_magic = ceil(2^32 / conv_cin)
   uint32_t conv_width, conv_cin, conv_kp, conv_magic;
+  uint32_t conv_hi;  // the k of the last segment: the sums before it, of products with a lo plane, are 2^12 times too large
   const uint32_t* skip_if;  // CONV kernels and their reduce pass: nothing to do where this word is not 0
   // A split last round (tail_tiles > 0; GemmReducePlan::tail_splits): the tiles from tail_first on, a multiple of the CUs,
   // run as tail_splits K slices of tail_kc each, whose raw sums go to part as dense tiles, slice-major
@@ -425,6 +426,14 @@ __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64) gemm_lds_kernel(FastArg
 #pragma unroll
     for (int j = 0; j < (PP ? TN16 : TN); j++) acc[i][j] = AccT{};
 
+  // CONV: past the products with lo planes
+  auto lose_lo_scale = [&]() {
+#pragma unroll
+    for (int i = 0; i < RR; i++)
+#pragma unroll
+      for (int j = 0; j < (PP ? TN16 : TN); j++) acc[i][j] *= 0x1p-12f;
+  };
+
   // int4: the f16 scales of the tile's columns as f32, NSB 64-k blocks at a time in two LDS buffers. The values of the
   // next NSB blocks are loaded to registers at the first block of a buffer and stored half a buffer later.
   constexpr int NSB = 8;
@@ -569,6 +578,7 @@ __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64) gemm_lds_kernel(FastArg
           else wait_vmcnt<0>();
         }
         pp_barrier();
+        if (CONV && k_begin + (uint32_t)t * BK == a.conv_hi) lose_lo_scale();
         compute_block(grp == 1 && t + S < nk, k_begin + (uint32_t)(t + S) * BK, cur);
         if (!(grp == 1 && t + 1 == nk)) pp_barrier();  // both groups pass the same number of barriers
         cur = cur + 1 == S ? 0 : cur + 1;
@@ -691,6 +701,7 @@ __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64) gemm_lds_kernel(FastArg
 
     int cur = 0;
     for (int it = 0; it < nk; ++it) {
+      if (CONV && k_begin + (uint32_t)it * BK == a.conv_hi) lose_lo_scale();
       const uint32_t cur_off = (uint32_t)(cur * STAGE);
       const int nxt = cur + 1 == S ? 0 : cur + 1;
       const uint32_t nxt_off = (uint32_t)(nxt * STAGE);
@@ -819,6 +830,7 @@ __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64) gemm_lds_kernel(FastArg
   };
 
   if constexpr (CONV) {
+    if (k_end <= a.conv_hi) lose_lo_scale();  // a slice that ended before
     // undo the planes' scaling, the image's and the column's powers of two together: one after the other could leave
     // f32's range where the sum's own size does not (an image at 2^110 against weights at 2^-100)
     const int re = (int)(__float_as_uint(*a.row_scale) >> 23) - 254;

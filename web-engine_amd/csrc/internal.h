@@ -184,14 +184,16 @@ hipError_t launch_unpack_fp8(const void* packed, size_t n, const float* scale, f
 hipError_t launch_split_f32_planes(const float* x, uint32_t m, uint32_t k, uint32_t x_stride, uint16_t* out,
                                    hipStream_t s);
 // Rows of f32 or bf16 [m, k] (16-byte aligned, k % 8 == 0) -> `planes` f16 planes of kp values (zeros past k) per row,
-// scaled by a power of two of the row's own; inverse scales to inv[m]. lo_at < 0: the hi plane alone.
+// scaled by a power of two of the row's own; inverse scales to inv[m]. lo_at < 0: the hi plane alone. range (cleared): lo is
+// scaled up by another 2^12, and range[0] is set where the rows hold values too far apart for planes.
 hipError_t launch_split_f32_f16x2(const void* x, int dtype, uint32_t m, uint32_t k, uint32_t x_stride, uint16_t* out,
-                                  uint32_t kp, int planes, int lo_at, int hi_at, float* inv, hipStream_t s);
-// An f32 image [pixels, cin] -> f16 [pixels, 2, cin] (lo, hi) with one scale: its inverse to *inv, and 1 to *flag (else 0)
-// where the pixels' values lie too far apart for one scale; part: 2 kImageParts words
+                                  uint32_t kp, int planes, int lo_at, int hi_at, float* inv, uint32_t* range,
+                                  hipStream_t s);
+// An f32 image [pixels, cin] -> f16 [pixels, 2, cin] (lo, scaled up by another 2^12, and hi) with one scale: its inverse to
+// *inv. range: 3 words, cleared first; range[0] is set where the values lie too far apart. part: 2 kImageParts words
 constexpr uint32_t kImageParts = 512;
 hipError_t launch_image_f16x2(const float* x, uint32_t pixels, uint32_t cin, uint32_t* part, uint16_t* out, float* inv,
-                              uint32_t* flag, hipStream_t s);
+                              uint32_t* range, hipStream_t s);
 hipError_t launch_dequant_int4(const uint32_t* w, const uint16_t* sc, uint32_t rows, uint32_t k, uint32_t group,
                                float* out, hipStream_t s);
 hipError_t launch_elementwise(int op, size_t n, size_t d, int dtype, const void* a, const void* b, const void* c,

@@ -62,10 +62,16 @@ __global__ void __launch_bounds__(256) split_f32_planes_kernel(const float* __re
 }
 
 // ------------------------------------------------------------------ f32 operands as two f16 planes
-// v = 2^-e (hi + lo): with the row scaled by 2^e so that its largest finite |v| lies in [2^14, 2^15), hi = f16(v 2^e) and
-// lo = f16(v 2^e - hi) hold v to 2^-23 of itself down to 2^-18 of the row's largest, and to 2^-40 of that largest below.
-// The rounding of the sums in f32 is larger than that (rel. error of 1024 x 6144 x 6144 against f64: see the GEMM's
-// dispatch). inf stays inf with a NaN beside it, as in the three bf16 planes.
+// v = 2^-e (hi + lo / L), L = 2^12 (kPlaneLo) or 1: with the row scaled by 2^e so that its largest finite |v| lies in
+// [2^14, 2^15), hi = f16(v 2^e) and lo = f16((v 2^e - hi) L) hold v to 2^-23 of itself, down to 2^-29 of the row's largest
+// with L = 2^12 (the remainder of that largest, at most 2^3, still fits), to 2^-20 of itself down to 2^-31, and to 2^-52 of
+// that largest below. The rounding of the sums in f32 is larger than the first of these (rel. error of 1024 x 6144 x 6144
+// against f64: see the GEMM's dispatch). Values below 2^-31 of the largest, but 0, are counted as tiny: with more than one of
+// them to 64 others in a row, or more than 8 + 2^-20 of all in the operand, the operand is not for planes, and the general
+// kernel runs in its place. (Normal data holds 1e-9 of them, products like silu(a) b 1e-7; an outlier with nothing else near it,
+// or a channel far below the others, many.) inf stays inf with a NaN beside it, as in the three bf16 planes.
+constexpr float kPlaneLo = 4096.0f;
+constexpr uint32_t kPlaneTiny = 110u << 23;  // 2^-17, 2^-31 of the largest scaled value's power of two
 // The biased exponent of the scale for the largest finite |v| (its bits), and the inverse scale.
 __device__ __forceinline__ uint32_t plane_scale_exp(uint32_t amax_bits) {
   const uint32_t e = 127u + 14u + 127u - (amax_bits >> 23);  // 2^(14 - (exponent - 127)), subnormals as exponent 0
@@ -94,31 +100,48 @@ __device__ __forceinline__ void load8(const void* p, size_t i, float (&v)[8]) {
     for (int e = 0; e < 8; e++) v[e] = bf16_to_f32((uint16_t)(a[e / 2] >> (16 * (e & 1))));
   }
 }
-__device__ __forceinline__ void split_f16x2(const float (&v)[8], float s, u32x4& lo, u32x4& hi) {
+__device__ __forceinline__ uint32_t block_sum256(uint32_t v, uint32_t* red) {
+#pragma unroll
+  for (int d = 32; d >= 1; d >>= 1) v += (uint32_t)__shfl_xor((int)v, d, 64);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  __syncthreads();
+  return red[0] + red[1] + red[2] + red[3];
+}
+// The planes of 8 values times s; counts the tiny ones.
+__device__ __forceinline__ void split_f16x2(const float (&v)[8], float s, float lo_scale, u32x4& lo, u32x4& hi,
+                                            uint32_t& tiny) {
 #pragma unroll
   for (int i = 0; i < 4; i++) {
     const float a = v[2 * i] * s, b = v[2 * i + 1] * s;
+    const uint32_t ba = __float_as_uint(a) & 0x7fffffffu, bb = __float_as_uint(b) & 0x7fffffffu;
+    tiny += (ba && ba < kPlaneTiny ? 1u : 0u) + (bb && bb < kPlaneTiny ? 1u : 0u);
     const uint32_t ha = f32_to_f16(a), hb = f32_to_f16(b);
     hi[i] = ha | (hb << 16);
-    lo[i] = (uint32_t)f32_to_f16(a - f16_to_f32((uint16_t)ha)) | ((uint32_t)f32_to_f16(b - f16_to_f32((uint16_t)hb)) << 16);
+    lo[i] = (uint32_t)f32_to_f16((a - f16_to_f32((uint16_t)ha)) * lo_scale) |
+            ((uint32_t)f32_to_f16((b - f16_to_f32((uint16_t)hb)) * lo_scale) << 16);
   }
 }
 
 // One workgroup per row [k values at src + row * stride] -> f16 planes at out + row * planes * kp, zeros past k: plane
 // lo_at holds lo, plane hi_at hi (lo_at < 0: hi alone). The row's inverse scale goes to inv[row]. Two reads of the row
-// (the second from L2): k % 8 == 0, rows and out 16-byte aligned.
+// (the second from L2): k % 8 == 0, rows and out 16-byte aligned. range: the tiny values of all rows are added up in its
+// second word, and its first is set where they are too many (of a row, or more than `most` of all).
 template <int DT>
 __global__ void __launch_bounds__(256) split_f32_f16x2_kernel(const void* __restrict__ src, uint32_t k, uint32_t stride,
                                                               uint16_t* __restrict__ out, uint32_t kp, int planes,
-                                                              int lo_at, int hi_at, float* __restrict__ inv) {
-  __shared__ uint32_t red[4];
+                                                              int lo_at, int hi_at, float lo_scale, float* __restrict__ inv,
+                                                              uint32_t* __restrict__ range, uint32_t most) {
+  __shared__ uint32_t red[4], red2[4], red3[4];
   const size_t row = blockIdx.x, base = row * stride;
-  uint32_t m = 0;
+  uint32_t m = 0, tiny = 0, nonzero = 0;
   for (uint32_t i = threadIdx.x * 8; i < k; i += 2048) {
     float v[8];
     load8<DT>(src, base + i, v);
 #pragma unroll
-    for (int e = 0; e < 8; e++) m = max(m, finite_bits(v[e]));
+    for (int e = 0; e < 8; e++) {
+      m = max(m, finite_bits(v[e]));
+      nonzero += v[e] != 0.0f ? 1u : 0u;
+    }
   }
   const uint32_t se = plane_scale_exp(block_max256(m, red));
   const float s = __uint_as_float(se << 23);
@@ -128,80 +151,86 @@ __global__ void __launch_bounds__(256) split_f32_f16x2_kernel(const void* __rest
     float v[8] = {};
     if (i < k) load8<DT>(src, base + i, v);
     u32x4 lo, hi;
-    split_f16x2(v, s, lo, hi);
+    split_f16x2(v, s, lo_scale, lo, hi, tiny);
     *(u32x4*)(dst + (size_t)hi_at * kp + i) = hi;
     if (lo_at >= 0) *(u32x4*)(dst + (size_t)lo_at * kp + i) = lo;
+  }
+  if (range && __syncthreads_or(tiny != 0)) {
+    const uint32_t t = block_sum256(tiny, red2), n = block_sum256(nonzero, red3);
+    if (threadIdx.x == 0 && (64u * t > n - t || atomicAdd(range + 1, t) + t > most)) atomicOr(range, 1u);
   }
 }
 
 hipError_t launch_split_f32_f16x2(const void* x, int dtype, uint32_t m, uint32_t k, uint32_t x_stride, uint16_t* out,
-                                  uint32_t kp, int planes, int lo_at, int hi_at, float* inv, hipStream_t s) {
+                                  uint32_t kp, int planes, int lo_at, int hi_at, float* inv, uint32_t* range,
+                                  hipStream_t s) {
   if (m == 0) return hipSuccess;
   const auto kern = dtype == F32 ? split_f32_f16x2_kernel<F32> : split_f32_f16x2_kernel<BF16>;
-  hipLaunchKernelGGL(kern, dim3(m), dim3(256), 0, s, x, k, x_stride, out, kp, planes, lo_at, hi_at, inv);
+  hipLaunchKernelGGL(kern, dim3(m), dim3(256), 0, s, x, k, x_stride, out, kp, planes, lo_at, hi_at, range ? kPlaneLo : 1.0f,
+                     inv, range, (uint32_t)(8 + ((uint64_t)m * k >> 20)));
   return hipGetLastError();
 }
 
 // An f32 image (cin values per pixel, cin % 8 == 0) -> per pixel the lo and the hi plane of its cin values, one scale for
-// the whole image (a convolution's sums mix pixels): the largest pixel maximum and the smallest nonzero one per workgroup
-// into part, then the split, whose workgroups each reduce part. The planes hold a value to 2^-40 of the image's largest: an
-// image with a pixel whose largest value lies below 2^-16 of that is flagged, and the general kernel takes it.
-__global__ void __launch_bounds__(256) image_amax_kernel(const float* __restrict__ x, uint32_t pixels, uint32_t cin,
-                                                         uint32_t* __restrict__ part) {
+// the whole image (a convolution's sums mix pixels): the largest value and the number of nonzero ones per workgroup into
+// part, then the split, whose workgroups each reduce part. range[0] is set where the image is not for planes (the rule above,
+// the whole image as one row); range[1], range[2]: counts of the weights and of the image.
+__global__ void __launch_bounds__(256) image_amax_kernel(const float* __restrict__ x, size_t n, uint32_t* __restrict__ part,
+                                                         uint32_t* __restrict__ range) {
   __shared__ uint32_t red[4], red2[4];
-  const uint32_t sub = threadIdx.x & 15u;  // 16 lanes per pixel
-  uint32_t big = 0, inv_small = 0;         // inv_small: the complement of the smallest, so both reduce by max
-  for (uint32_t p = blockIdx.x * 16 + (threadIdx.x >> 4); p < pixels; p += kImageParts * 16) {
-    uint32_t m = 0;
-    for (uint32_t c = sub * 8; c < cin; c += 128) {
-      float v[8];
-      load8<F32>(x, (size_t)p * cin + c, v);
+  if (blockIdx.x == 0 && threadIdx.x < 3) range[threadIdx.x] = 0;
+  uint32_t big = 0, nonzero = 0;
+  for (size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 8; i < n; i += (size_t)kImageParts * 2048) {
+    float v[8];
+    load8<F32>(x, i, v);
 #pragma unroll
-      for (int e = 0; e < 8; e++) m = max(m, finite_bits(v[e]));
+    for (int e = 0; e < 8; e++) {
+      big = max(big, finite_bits(v[e]));
+      nonzero += v[e] != 0.0f ? 1u : 0u;
     }
-#pragma unroll
-    for (int d = 8; d >= 1; d >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, d, 16));
-    if (m) big = max(big, m), inv_small = max(inv_small, ~m);
   }
   big = block_max256(big, red);
-  inv_small = block_max256(inv_small, red2);
+  nonzero = block_sum256(nonzero, red2);
   if (threadIdx.x == 0) {
     part[blockIdx.x] = big;
-    part[kImageParts + blockIdx.x] = inv_small;
+    part[kImageParts + blockIdx.x] = nonzero;
   }
 }
 __global__ void __launch_bounds__(256) image_f16x2_kernel(const float* __restrict__ x, size_t n, uint32_t cin,
                                                           const uint32_t* __restrict__ part, uint16_t* __restrict__ out,
-                                                          float* __restrict__ inv, uint32_t* __restrict__ flag) {
-  __shared__ uint32_t red[4], red2[4];
+                                                          float* __restrict__ inv, uint32_t* __restrict__ range) {
+  __shared__ uint32_t red[4], red2[4], red3[4];
   static_assert(kImageParts == 512, "two parts per thread");
   const uint32_t t = threadIdx.x, big = block_max256(max(part[t], part[256 + t]), red);
-  if (blockIdx.x == 0) {  // workgroup-uniform
-    const uint32_t small = ~block_max256(max(part[kImageParts + t], part[kImageParts + 256 + t]), red2);
-    if (t == 0) *flag = (big >> 23) > (small >> 23) + 16u ? 1u : 0u;
-  }
   const uint32_t se = plane_scale_exp(big);
   const float s = __uint_as_float(se << 23);
   if (blockIdx.x == 0 && t == 0) *inv = __uint_as_float((254u - se) << 23);
   const size_t i = ((size_t)blockIdx.x * 256 + t) * 8;
-  if (i >= n) return;
-  float v[8];
-  load8<F32>(x, i, v);
-  u32x4 lo, hi;
-  split_f16x2(v, s, lo, hi);
-  uint16_t* dst = out + i / cin * 2 * cin + i % cin;
-  *(u32x4*)dst = lo;
-  *(u32x4*)(dst + cin) = hi;
+  uint32_t tiny = 0;
+  if (i < n) {
+    float v[8];
+    load8<F32>(x, i, v);
+    u32x4 lo, hi;
+    split_f16x2(v, s, kPlaneLo, lo, hi, tiny);
+    uint16_t* dst = out + i / cin * 2 * cin + i % cin;
+    *(u32x4*)dst = lo;
+    *(u32x4*)(dst + cin) = hi;
+  }
+  if (__syncthreads_or(tiny != 0)) {
+    const uint32_t count = block_sum256(tiny, red2);
+    const uint32_t nonzero = block_sum256(part[kImageParts + t] + part[kImageParts + 256 + t], red3);
+    if (t == 0 && atomicAdd(range + 2, count) + count > min(8u + (uint32_t)(n >> 20), nonzero / 64u)) atomicOr(range, 1u);
+  }
 }
 
 hipError_t launch_image_f16x2(const float* x, uint32_t pixels, uint32_t cin, uint32_t* part, uint16_t* out, float* inv,
-                              uint32_t* flag, hipStream_t s) {
+                              uint32_t* range, hipStream_t s) {
   const size_t n = (size_t)pixels * cin;
-  hipLaunchKernelGGL(image_amax_kernel, dim3(kImageParts), dim3(256), 0, s, x, pixels, cin, part);
+  hipLaunchKernelGGL(image_amax_kernel, dim3(kImageParts), dim3(256), 0, s, x, n, part, range);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(image_f16x2_kernel, dim3((unsigned)((n / 8 + 255) / 256)), dim3(256), 0, s, x, n, cin, part, out, inv,
-                     flag);
+                     range);
   return hipGetLastError();
 }
 

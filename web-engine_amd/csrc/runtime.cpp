@@ -1131,7 +1131,7 @@ int matmul_impl(we_ctx* ctx, const we_matmul_params* p, int x_dtype, const void*
       float* inv = (float*)(scratch + scale_at);
       L.row_scale = inv;
       e = we::launch_split_f32_f16x2(xs, WE_F32, p->m, p->k, p->x_stride, (uint16_t*)scratch, p->k, 2, 0, 1, inv,
-                                     ctx->compute);
+                                     nullptr, ctx->compute);
     } else {
       e = we::launch_split_f32_planes(xs, p->m, p->k, p->x_stride, (uint16_t*)scratch, ctx->compute);
     }
