@@ -198,10 +198,11 @@ int we_conv3x3_params(we_ctx* ctx, uint32_t height, uint32_t width, uint32_t cin
  * (src/kernels/matmul.ts:118-178) dispatched by linear() (src/model/ops.ts:61-73).
  * x: x_dtype in {F32, F16, BF16}; y: y_dtype in {F32, F16, BF16}; w_scales: int4 only, f16 [N, K/group];
  * bias: f32 [N] with WE_EPI_BIAS. Accumulation is fp32 on bf16/f16 MFMA. f32 operands are split into 16-bit planes that are
- * multiplied plane by plane: three bf16 planes whose sum is the f32 value exactly, or, for f32 x against fp8 weights and for
- * the 3x3 convolution of an f32 image, two f16 planes scaled by a power of two (per row of x or W, per image), which hold a
- * value to 2^-23 of itself down to 2^-18 of its row's or image's largest and to 2^-40 of that largest below; an image whose
- * pixels lie further apart than 2^16 takes the three planes. */
+ * multiplied plane by plane: three bf16 planes whose sum is the f32 value exactly, or, for large products of f32 x with
+ * fp8 weights and for the 3x3 convolution of an f32 image, two f16 planes scaled by powers of two (per row of x or W, per
+ * image). Two planes hold a value to 2^-23 of itself down to 2^-29 of its row's or image's largest and to 2^-20 down to
+ * 2^-31; operands in which more than a few nonzero values lie further below (1 to 64 others in a row or image, 8 and a
+ * millionth of all) are found on the device and take the exact planes. */
 int we_matmul(we_ctx* ctx, const we_matmul_params* p, int x_dtype, const void* x, int w_dtype, const void* w,
               const void* w_scales, uint32_t group, int y_dtype, void* y, const float* bias, uint32_t flags);
 /* we_matmul that allocates nothing. No counterpart in the reference: for callers that cannot allocate device memory

@@ -813,6 +813,64 @@ def test_f32_rows_of_any_scale(graph, k):
         assert O.rel_error(got[r], want[r]) < 1e-5
 
 
+WIDE_ROWS = [(300, 16400, 1088, e, epi) for e in (0, 24, 30, 36, 40, 100) for epi in ("plain", "swiglu in place")] + [
+    (1024, 6144, 3072, 0, "swiglu in place"), (1024, 6144, 3072, 40, "swiglu in place"),  # two K slices
+    (2051, 4100, 512, 40, "plain"), (1030, 16400, 3072, 40, "plain")]  # over 2048 rows; a split last round
+
+
+@pytest.mark.parametrize("m,n,k,e,epi", WIDE_ROWS)
+def test_f32_rows_of_wide_range(graph, m, n, k, e, epi):
+    """f32 x with fp8 weights at shapes for two f16 planes (M > 64, 5 GFLOP and more): rows at 2^100 and 2^-100, the two NaN codes
+    among the weights, and values 2^e apart that do not meet in a result: one value 2^e above the rest of its row in a
+    column whose weights are 0, a row with nothing but such a value and a single 1, and a column 2^-e of the others that
+    output column 3 alone reads. Rows and that column by their own size, whichever planes the device takes."""
+    rng = np.random.default_rng(e)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    w_store, _, ow = make_weights(rng, n, k, we.FP8)
+    w = w_store.reshape(n, k)
+    w[:, 5] = 0
+    w[3] = 0
+    w[3, 7] = 0x38  # 1.0
+    w[100, 50], w[n - 1, 51] = 0x7E, 0xFE  # +-448 for the oracle
+    w_oracle = w_store.copy()
+    w[100, 50], w[n - 1, 51] = 0x7F, 0xFF  # +-480 to the kernels
+    x[:, 5] = 0
+    x[20] *= np.float32(2.0 ** 100)
+    x[21] *= np.float32(2.0 ** -100)
+    if e:
+        x[11, 5] = 2.0 ** e
+        x[200] = 0
+        x[200, 5], x[200, 9] = 2.0 ** e, 1.0
+        x[:, 7] *= np.float32(2.0 ** -e)
+    x[200, 7] = np.float32(2.0 ** -e)
+    x[21, 7] = np.float32(2.0 ** -100)
+    p = we.matmul_params(m, n, k, 0.02, graph=graph)
+    mark = graph.mark()
+    xb, wb = graph.buffer(x.reshape(-1)), graph.buffer(w_store)
+    aux = rng.standard_normal((m, n)).astype(np.float32)
+    y = graph.buffer(aux.reshape(-1)) if epi != "plain" else graph.buffer(m * n * 4)
+    if epi == "plain":
+        graph.matmul(p, we.F32, xb, we.FP8, wb, we.F32, y)
+    else:
+        graph.matmul(p, we.F32, xb, we.FP8, wb, we.F32, y, mul=we.MUL_SWIGLU, aux=y)
+    got = graph.read(y, dtype=np.float32).astype(np.float64).reshape(m, n)
+    graph.release(mark)
+    rows = [0, 11, 20, 21, 64, 200, 256, m - 1]
+    op = O.matmul_params(m, n, k, 0.02)
+    table = O.e4m3_gpu_table().astype(np.float64)
+    col = (x[:, 7].astype(np.float64)) * table[0x38] * 0.02
+
+    def fin(v, a):
+        a = a.astype(np.float64)
+        return v if epi == "plain" else a / (1 + np.exp(-a)) * v
+    for r in rows:
+        want = O.matmul_rows(op, O.F32, x.reshape(-1), ow, w_oracle, r, r + 1)[r * n:(r + 1) * n]
+        want[100] += 32 * 0.02 * float(x[r, 50])
+        want[n - 1] -= 32 * 0.02 * float(x[r, 51])
+        assert O.rel_error(got[r], fin(want, aux[r])) < TOL_F32_OUT, r
+    assert np.abs(got[:, 3] / fin(col, aux[:, 3]) - 1).max() < TOL_F32_OUT
+
+
 @pytest.mark.parametrize("m,n,k,w_dt", [(65, 1040, 2048, we.FP8), (129, 520, 4096, we.BF16), (300, 1028, 1024, we.FP8),
                                         (520, 260, 3072, we.FP8), (700, 400, 512, we.BF16)])
 def test_planned_tiles_and_slices(graph, m, n, k, w_dt):

@@ -76,16 +76,17 @@ __device__ __forceinline__ float e4m3_shader(uint32_t b) {
 
 // Four fp8 bytes of one word -> four 16-bit values (two packed words). The hardware converter decodes
 // OCP e4m3fn and turns the two NaN codes into NaN; the reference shader turns them into +-480, so words
-// holding a NaN code take a slow path that writes +-480 (0x43f0 bf16 / 0x5f80 f16) for those bytes.
+// holding a NaN code take a slow path that writes +-480 (0x43f0 bf16 / 0x5f80 f16) for those bytes. f16: times the power
+// of two `scale` (2^-5 .. 2^7: every code stays a normal f16).
 __device__ __forceinline__ bool has_nan_code(uint32_t w) {
   return (((w & 0x7f7f7f7fu) + 0x01010101u) & 0x80808080u) != 0u;
 }
 template <bool IS_F16>
-__device__ __forceinline__ u32x2 fp8x4_to_16(uint32_t w) {
+__device__ __forceinline__ u32x2 fp8x4_to_16(uint32_t w, float scale = 1.0f) {
   u32x2 r;
   if constexpr (IS_F16) {
-    f16x2 lo = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w, 1.0f, false);
-    f16x2 hi = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w, 1.0f, true);
+    f16x2 lo = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w, scale, false);
+    f16x2 hi = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w, scale, true);
     r.x = __builtin_bit_cast(uint32_t, lo);
     r.y = __builtin_bit_cast(uint32_t, hi);
   } else {
@@ -95,7 +96,7 @@ __device__ __forceinline__ u32x2 fp8x4_to_16(uint32_t w) {
     r.y = __builtin_bit_cast(uint32_t, hi);
   }
   if (__builtin_expect(has_nan_code(w), 0)) {
-    const uint32_t big = IS_F16 ? 0x5f80u : 0x43f0u;
+    const uint32_t big = IS_F16 ? 0x5f80u + ((__float_as_uint(scale) >> 23) - 127u) * 0x400u : 0x43f0u;
     uint32_t h[4];
 #pragma unroll
     for (int i = 0; i < 4; i++) {
@@ -231,6 +232,34 @@ __device__ __forceinline__ void dma16s(const __amdgpu_buffer_rsrc_t& r, void* ds
                  :
                  : "s"((uint32_t)(uintptr_t)(lds_ptr_t*)dst), "v"(voff), "s"(r), "s"(soff)
                  : "memory");
+}
+
+// out[r, p K + k] = plane p of x[r, k]: hi = bf16(x), mid = bf16(x - hi), lo = bf16(x - hi - mid). Each remainder is
+// exact in f32 (at most 16, then 8 significant bits), so hi + mid + lo == x for every normal f32 value and a GEMM
+// over the 3K planes against weights that repeat every K sums exact products of all 24 bits of x. A thread takes 8
+// consecutive values of a row (two 16-byte loads, three 16-byte stores) per step; x rows 16-byte aligned, K % 8 == 0.
+__device__ __forceinline__ void split_planes3(const float* __restrict__ x, uint32_t m, uint32_t k, uint32_t xs,
+                                              uint16_t* __restrict__ out, size_t first, size_t step) {
+  const uint32_t groups = k / 8;
+  for (size_t idx = first; idx < (size_t)m * groups; idx += step) {
+    const uint32_t r = (uint32_t)(idx / groups), g = (uint32_t)(idx % groups);
+    const float* src = x + (size_t)r * xs + (size_t)g * 8;
+    const f32x4 a = *(const f32x4*)src, b = *(const f32x4*)(src + 4);
+    const float v[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+    uint32_t h[3][8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      h[0][i] = f32_to_bf16(v[i]);
+      const float r1 = v[i] - bf16_to_f32((uint16_t)h[0][i]);
+      h[1][i] = f32_to_bf16(r1);
+      h[2][i] = f32_to_bf16(r1 - bf16_to_f32((uint16_t)h[1][i]));
+    }
+    uint16_t* dst = out + (size_t)r * 3 * k + (size_t)g * 8;
+#pragma unroll
+    for (int p = 0; p < 3; p++)
+      *(u32x4*)(dst + (size_t)p * k) = u32x4{h[p][0] | (h[p][1] << 16), h[p][2] | (h[p][3] << 16),
+                                             h[p][4] | (h[p][5] << 16), h[p][6] | (h[p][7] << 16)};
+  }
 }
 
 }  // namespace we

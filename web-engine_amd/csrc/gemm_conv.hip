@@ -100,7 +100,7 @@ hipError_t conv_fast_launch(const GemmLaunch& L, void* scratch, hipStream_t s) {
   // weight rows hi | lo (f32) or hi (bf16: 8 significant bits, exact in f16 down to 2^-31 of the row's largest: tiny ones are
   // those below, too)
   e = launch_split_f32_f16x2((const char*)L.w + (uint64_t)L.w_offset * wb, L.w_dtype, L.n, L.k, L.w_stride, weights, p.kp,
-                             wplanes, wplanes == 2 ? 1 : -1, 0, col_scale, range, s);
+                             wplanes, wplanes == 2 ? 1 : -1, 0, col_scale, false, range, s);
   if (e != hipSuccess) return e;
   const int yb = L.y_dtype == F32 ? 4 : 2;
   FastArgs a{};

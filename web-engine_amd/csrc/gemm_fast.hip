@@ -276,6 +276,15 @@ FastArgs fast_args(const GemmLaunch& L, uint32_t kc) {
   a.kwrap = L.k_wrap ? L.k_wrap : 0xffffffffu;
   a.kwrap2 = L.k_wrap ? 2 * L.k_wrap : 0xffffffffu;
   a.row_scale = L.row_scale;
+  a.cvt_lo = L.row_scale ? 0x1p-5f : 1.0f;
+  a.cvt_hi = L.row_scale ? 0x1p7f : 1.0f;
+  a.only_if = L.only_if;
+  a.range = L.range;
+  a.range_n = L.range_n;
+  a.range_most = L.range_most;
+  a.f32 = L.f32;
+  a.f32_stride = L.f32_stride;
+  a.skip_if = a.skip_out = L.skip_out;
   a.scale = L.scale;
   a.x_stride = L.x_stride;
   a.w_stride = L.w_stride;

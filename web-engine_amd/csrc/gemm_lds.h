@@ -80,7 +80,21 @@ struct FastArgs {
   // the lo plane, the others with the hi plane. conv_magic = ceil(2^32 / conv_cin)
   uint32_t conv_width, conv_cin, conv_kp, conv_magic;
   uint32_t conv_hi;  // the k of the last segment: the sums before it, of products with a lo plane, are 2^12 times too large
-  const uint32_t* skip_if;  // CONV kernels and their reduce pass: nothing to do where this word is not 0
+  // Launches that decide on the device whether they run. skip_if: CONV kernels and reduce passes do nothing where this word
+  // is not 0 (NULL: they run); only_if: fp8 kernels for bf16 x and reduce passes do nothing where it is 0 (NULL: they run).
+  // range_n > 0 (two f16 planes): the tiny values that split_f32_f16x2_kernel counted, by workgroup; more than range_most
+  // of them and the kernel splits the f32 rows (f32, f32_stride) into three bf16 planes in the place of the two and does
+  // nothing else. Its first workgroup leaves in skip_out whether it was so.
+  const uint32_t* skip_if;
+  const uint32_t* only_if;
+  const uint32_t* range;
+  uint32_t range_n, range_most;
+  uint32_t* skip_out;
+  const float* f32;
+  uint32_t f32_stride;
+  // fp8 weights for f16 x: the powers of two that the weights below k = kwrap and from there on are converted with. Two
+  // planes: 2^-5 with the lo plane, which carries 2^12, and 2^7 with the hi plane, all normal f16 values; else 1 and 1
+  float cvt_lo, cvt_hi;
   // A split last round (tail_tiles > 0; GemmReducePlan::tail_splits): the tiles from tail_first on, a multiple of the CUs,
   // run as tail_splits K slices of tail_kc each, whose raw sums go to part as dense tiles, slice-major
   uint32_t tail_first, tail_tiles, tail_splits, tail_kc;
@@ -134,13 +148,13 @@ __device__ __forceinline__ void wait_vmcnt() {
 }
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-// fp8 word -> 4 x 16-bit through the hardware converter
+// fp8 word -> 4 x 16-bit through the hardware converter, f16 times the power of two `scale`
 template <bool IS_F16>
-__device__ __forceinline__ u32x2 cvt_fp8x4(uint32_t w) {
+__device__ __forceinline__ u32x2 cvt_fp8x4(uint32_t w, float scale) {
   u32x2 r;
   if constexpr (IS_F16) {
-    r.x = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w, 1.0f, false));
-    r.y = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w, 1.0f, true));
+    r.x = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w, scale, false));
+    r.y = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w, scale, true));
   } else {
     r.x = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, 1.0f, false));
     r.y = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, 1.0f, true));
@@ -239,12 +253,38 @@ __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64) gemm_lds_kernel(FastArg
   constexpr int B_CPR = B_ROW / 16;                                       // 16-B chunks per weight row
   __shared__ __attribute__((aligned(1024))) char lds[S * STAGE];
 
-  if constexpr (CONV)
-    if (*a.skip_if) return;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WAVES_N, wn = wave % WAVES_N;
   const int lw = wave % NL;  // this wave's share of the loads (LM 1: group 1's waves 0 .. NW / 2 - 1)
   const int h = lane >> 5, l32 = lane & 31;
+  if constexpr (CONV) {
+    if (*a.skip_if) return;
+  } else if constexpr (B8 && IS_F16) {
+    if (a.range_n) {  // every wave adds the counts up by itself, all loads in flight
+      u32x4 c[kRangeWords / 256];
+#pragma unroll
+      for (uint32_t i = 0; i < kRangeWords / 256; i++) {
+        const uint32_t at = i * 256 + lane * 4;  // range_n is a multiple of 4
+        c[i] = at < a.range_n ? *(const u32x4*)(a.range + at) : u32x4{};
+      }
+      uint32_t tiny = 0;
+#pragma unroll
+      for (uint32_t i = 0; i < kRangeWords / 256; i++) tiny += (c[i][0] + c[i][1]) + (c[i][2] + c[i][3]);
+#pragma unroll
+      for (int d = 32; d >= 1; d >>= 1) tiny += (uint32_t)__shfl_xor((int)tiny, d, 64);
+      const bool wide = __builtin_amdgcn_readfirstlane((int)tiny) > (int)a.range_most;
+      const uint32_t wg = blockIdx.y * gridDim.x + blockIdx.x;
+      if (wg == 0 && tid == 0) *a.skip_out = wide ? 1u : 0u;
+      if (wide) {
+        // three planes instead of two, for the launch behind: no workgroup of this one reads the two
+        split_planes3(a.f32, a.m, a.kwrap, a.f32_stride, (uint16_t*)a.x, (size_t)wg * (NW * 64) + tid,
+                      (size_t)gridDim.x * gridDim.y * (NW * 64));
+        return;
+      }
+    }
+  } else if constexpr (B8) {
+    if (a.only_if && *a.only_if == 0) return;
+  }
 
   uint32_t pid, z = blockIdx.y, kc = a.kc;
   constexpr bool TAIL = PP && !CONV;  // the tile shapes whose last round is split
@@ -461,6 +501,12 @@ __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64) gemm_lds_kernel(FastArg
     }
   };
 
+  // f16 x: the factor of the block's fp8 weights (FastArgs::cvt_lo)
+  float wscale = 1.0f;
+  auto block_wscale = [&](uint32_t kb) {
+    if constexpr (B8 && IS_F16) wscale = kb < a.kwrap ? a.cvt_lo : a.cvt_hi;
+  };
+
   u32x4 xf[2][TM];           // x fragments, double-buffered over steps
   u32x4 wr[2][TN];           // fp8: raw 16-B chunks (t = 0, 1); 16-bit: fragments double-buffered over steps
   auto read_x = [&](uint32_t st_off, int s, u32x4 (&d)[TM]) {
@@ -503,7 +549,7 @@ __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64) gemm_lds_kernel(FastArg
     constexpr bool PRE_CVT = PRE > 0;
     u32x4 wcv[PRE_CVT ? PRE : 1][TN16];
     auto unpack = [&](const u32x4& r, int q) {
-      const u32x2 lo = cvt_fp8x4<IS_F16>(r[2 * q]), hi = cvt_fp8x4<IS_F16>(r[2 * q + 1]);
+      const u32x2 lo = cvt_fp8x4<IS_F16>(r[2 * q], wscale), hi = cvt_fp8x4<IS_F16>(r[2 * q + 1], wscale);
       return u32x4{lo.x, lo.y, hi.x, hi.y};
     };
     auto memory_block = [&](uint32_t st_off) {
@@ -593,6 +639,7 @@ __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64) gemm_lds_kernel(FastArg
       if (grp == 1) pp_barrier();  // group 1 sits out interval 0
       int cur = 0;
       for (int t = 0; t < nk; ++t) {
+        block_wscale(k_begin + (uint32_t)t * BK);
         const uint32_t cur_off = (uint32_t)(cur * STAGE);
         const int ahead = cur + S - 1 >= S ? cur - 1 : cur + S - 1;  // stage of block t + S - 1
         if (t + S - 1 < nk) issue(k_begin + (uint32_t)(t + S - 1) * BK, ahead);
@@ -702,6 +749,7 @@ __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64) gemm_lds_kernel(FastArg
     int cur = 0;
     for (int it = 0; it < nk; ++it) {
       if (CONV && k_begin + (uint32_t)it * BK == a.conv_hi) lose_lo_scale();
+      block_wscale(k_begin + (uint32_t)it * BK);
       const uint32_t cur_off = (uint32_t)(cur * STAGE);
       const int nxt = cur + 1 == S ? 0 : cur + 1;
       const uint32_t nxt_off = (uint32_t)(nxt * STAGE);
@@ -730,7 +778,7 @@ __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64) gemm_lds_kernel(FastArg
         for (int j = 0; j < TN; j++) {
           if constexpr (B8) {
             const u32x4 q = wr[s >> 1][j];
-            const u32x2 lo = cvt_fp8x4<IS_F16>(q[(s & 1) * 2]), hi = cvt_fp8x4<IS_F16>(q[(s & 1) * 2 + 1]);
+            const u32x2 lo = cvt_fp8x4<IS_F16>(q[(s & 1) * 2], wscale), hi = cvt_fp8x4<IS_F16>(q[(s & 1) * 2 + 1], wscale);
             wf[j] = u32x4{lo.x, lo.y, hi.x, hi.y};
           } else {
             wf[j] = wr[s & 1][j];
@@ -766,6 +814,7 @@ __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64) gemm_lds_kernel(FastArg
           const uint32_t kk = k0 + 8 * g16;
           const bool in = kk < k_end;
           const uint32_t kkw = kk >= a.kwrap2 ? kk - a.kwrap2 : kk >= a.kwrap ? kk - a.kwrap : kk;  // weights' k
+          block_wscale(kk);
           u32x4 xr[RR];
           u32x4 wv[TN16];
 #pragma unroll
@@ -779,7 +828,7 @@ __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64) gemm_lds_kernel(FastArg
             const uint32_t col = col0 + wn * WTN + j * 16 + r16;
             const uint32_t o = col < a.n && in ? col * a.w_stride + kkw : kInvalid;
             const u32x2 raw = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rw, o, 0, 0));
-            const u32x2 lo = fp8x4_to_16<IS_F16>(raw.x), hi = fp8x4_to_16<IS_F16>(raw.y);
+            const u32x2 lo = fp8x4_to_16<IS_F16>(raw.x, wscale), hi = fp8x4_to_16<IS_F16>(raw.y, wscale);
             wv[j] = u32x4{lo.x, lo.y, hi.x, hi.y};
           }
 #pragma unroll
@@ -791,6 +840,7 @@ __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64) gemm_lds_kernel(FastArg
         for (uint32_t k0 = k_begin; k0 < k_end; k0 += 16) {
           const uint32_t kk = k0 + 8 * h;  // 8 k per lane half; k_end - k0 >= 16 (multiples of 16)
           const uint32_t kkw = kk >= a.kwrap2 ? kk - a.kwrap2 : kk >= a.kwrap ? kk - a.kwrap : kk;  // weights' k
+          block_wscale(kk);
           u32x4 xr[TM];
           u32x4 wv[TN];
 #pragma unroll
@@ -804,7 +854,7 @@ __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64) gemm_lds_kernel(FastArg
             const uint32_t col = col0 + wn * WTN + j * 32 + l32;
             const uint32_t o = col < a.n ? col * a.w_stride + kkw : kInvalid;
             const u32x2 raw = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rw, o, 0, 0));
-            const u32x2 lo = fp8x4_to_16<IS_F16>(raw.x), hi = fp8x4_to_16<IS_F16>(raw.y);
+            const u32x2 lo = fp8x4_to_16<IS_F16>(raw.x, wscale), hi = fp8x4_to_16<IS_F16>(raw.y, wscale);
             wv[j] = u32x4{lo.x, lo.y, hi.x, hi.y};
           }
 #pragma unroll
@@ -847,14 +897,16 @@ __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64) gemm_lds_kernel(FastArg
         }
       }
   } else if constexpr (IS_F16 && B8) {
-    // two-plane f32 rows: undo the planes' scaling (powers of two)
+    // two-plane f32 rows: undo the planes' scaling and the weights' (cvt_lo), powers of two
     if (a.row_scale) {
 #pragma unroll
       for (int i = 0; i < RR; i++) {
         const uint32_t row = row0 + wm * WTM + i * RS + lrow;
-        const float rs = a.row_scale[row < a.m ? row : 0u];
+        const int re = (int)(__float_as_uint(a.row_scale[row < a.m ? row : 0u]) >> 23) - 127 - 7;
 #pragma unroll
-        for (int j = 0; j < (PP ? TN16 : TN); j++) acc[i][j] *= rs;
+        for (int j = 0; j < (PP ? TN16 : TN); j++)
+#pragma unroll
+          for (int e = 0; e < (PP ? 4 : 16); e++) acc[i][j][e] = ldexpf(acc[i][j][e], re);
       }
     }
   }
@@ -1147,10 +1199,9 @@ __device__ __forceinline__ void reduce_epilogue(const FastArgs& a, uint32_t row,
 // XCD (BM, BN > 0): the slices of a tile ran on one XCD (workgroups go round-robin over the 8 XCDs, and the slice
 // index adds a multiple of 8 tiles to the workgroup id), so each reduce workgroup takes a part of a tile of its own
 // XCD and reads the slices there. Otherwise one thread per 4 consecutive outputs in row-major order.
-template <int YT, int BM = 0, int BN = 0, bool CONV = false>
+template <int YT, int BM = 0, int BN = 0>
 __global__ void __launch_bounds__(256) splitk_reduce_kernel(FastArgs a) {
-  if constexpr (CONV)
-    if (*a.skip_if) return;
+  if ((a.skip_if && *a.skip_if) || (a.only_if && !*a.only_if)) return;
   uint32_t row, c0;
   if constexpr (BM > 0) {
     constexpr uint32_t ITEMS = BM * BN / 4, Q = ITEMS / 256;  // reduce workgroups per tile
@@ -1199,6 +1250,7 @@ __global__ void __launch_bounds__(256) splitk_reduce_kernel(FastArgs a) {
 // The reduce pass of a split last round: one thread per 4 consecutive outputs of a tail tile, slices in slice order.
 template <int YT, int BM, int BN>
 __global__ void __launch_bounds__(256) tail_reduce_kernel(FastArgs a) {
+  if ((a.skip_if && *a.skip_if) || (a.only_if && !*a.only_if)) return;
   constexpr uint32_t ITEMS = BM * BN / 4, Q = ITEMS / 256;  // workgroups per tile
   const uint32_t t = blockIdx.x / Q, i = (blockIdx.x % Q) * 256 + threadIdx.x;
   const uint32_t pid = a.tail_first + t;
@@ -1263,18 +1315,18 @@ static hipError_t launch_fast_cfg(FastArgs a, uint32_t splits, int reduce_xcd, h
     if (reduce_in_l2(tiles, a.w_bytes, reduce_xcd)) {
       const dim3 rg(tiles * (BM * BN / 4 / 256));
       switch (a.y_dtype) {
-        case F32: hipLaunchKernelGGL((splitk_reduce_kernel<F32, BM, BN, CONV>), rg, dim3(256), 0, s, a); break;
-        case F16: hipLaunchKernelGGL((splitk_reduce_kernel<F16, BM, BN, CONV>), rg, dim3(256), 0, s, a); break;
-        default: hipLaunchKernelGGL((splitk_reduce_kernel<BF16, BM, BN, CONV>), rg, dim3(256), 0, s, a); break;
+        case F32: hipLaunchKernelGGL((splitk_reduce_kernel<F32, BM, BN>), rg, dim3(256), 0, s, a); break;
+        case F16: hipLaunchKernelGGL((splitk_reduce_kernel<F16, BM, BN>), rg, dim3(256), 0, s, a); break;
+        default: hipLaunchKernelGGL((splitk_reduce_kernel<BF16, BM, BN>), rg, dim3(256), 0, s, a); break;
       }
       return hipGetLastError();
     }
     const size_t threads = (size_t)a.m * ((a.n + 3) / 4);
     const dim3 rg((unsigned)((threads + 255) / 256));
     switch (a.y_dtype) {
-      case F32: hipLaunchKernelGGL((splitk_reduce_kernel<F32, 0, 0, CONV>), rg, dim3(256), 0, s, a); break;
-      case F16: hipLaunchKernelGGL((splitk_reduce_kernel<F16, 0, 0, CONV>), rg, dim3(256), 0, s, a); break;
-      default: hipLaunchKernelGGL((splitk_reduce_kernel<BF16, 0, 0, CONV>), rg, dim3(256), 0, s, a); break;
+      case F32: hipLaunchKernelGGL(splitk_reduce_kernel<F32>, rg, dim3(256), 0, s, a); break;
+      case F16: hipLaunchKernelGGL(splitk_reduce_kernel<F16>, rg, dim3(256), 0, s, a); break;
+      default: hipLaunchKernelGGL(splitk_reduce_kernel<BF16>, rg, dim3(256), 0, s, a); break;
     }
     return hipGetLastError();
   }

@@ -60,7 +60,7 @@ struct GemmLaunch {
   // 3x3 convolution input (conv_width > 0, the general kernel only): x is a channel-last image
   // [m / conv_width, conv_width, conv_cin] and k runs over (tap, channel), K = 9 * conv_cin
   uint32_t conv_width, conv_cin;
-  const uint32_t* only_if;  // general kernel: a device word, 0: the launch does nothing (NULL: it runs)
+  const uint32_t* only_if;  // general kernel, fast kernel for fp8 weights and bf16 x: a device word, 0: the launch does nothing
   int x_dtype, w_dtype, y_dtype;
   uint32_t m, n, k;
   float scale;
@@ -75,6 +75,13 @@ struct GemmLaunch {
   uint32_t k_wrap;
   // k_wrap with two f16 planes: the rows' inverse scales (launch_split_f32_f16x2)
   const float* row_scale;
+  // and their counts of tiny values, range_n words: with more than range_most the launch only writes three bf16
+  // planes of the rows at f32 over the two, and 1 (else 0) to *skip_out
+  const uint32_t* range;
+  uint32_t range_n, range_most;
+  uint32_t* skip_out;
+  const float* f32;
+  uint32_t f32_stride;
   // split-K for small M: K in rsplits slices of rkc, partial sums in scratch (rsplits * m * n f32), then a
   // reduce pass that runs the epilogue; rcfg: the tile configuration the slices were sized for (-1: by shape)
   uint32_t rsplits, rkc;
@@ -184,10 +191,14 @@ hipError_t launch_unpack_fp8(const void* packed, size_t n, const float* scale, f
 hipError_t launch_split_f32_planes(const float* x, uint32_t m, uint32_t k, uint32_t x_stride, uint16_t* out,
                                    hipStream_t s);
 // Rows of f32 or bf16 [m, k] (16-byte aligned, k % 8 == 0) -> `planes` f16 planes of kp values (zeros past k) per row,
-// scaled by a power of two of the row's own; inverse scales to inv[m]. lo_at < 0: the hi plane alone. range (cleared): lo is
-// scaled up by another 2^12, and range[0] is set where the rows hold values too far apart for planes.
+// scaled by a power of two of the row's own, lo by another 2^12; inverse scales to inv[m]. lo_at < 0: the hi plane alone.
+// words (f32 rows): how many values lie too far below their row's largest goes to range, range_words(m) words, more
+// than planes_most_tiny in all where the rows are not for planes; else range[0] (cleared before) is set there.
+constexpr uint32_t kRangeWords = 2048;
+inline uint32_t range_words(uint32_t m) { return m < kRangeWords ? (m + 3) / 4 * 4 : kRangeWords; }
+inline uint32_t planes_most_tiny(uint32_t m, uint32_t k) { return (uint32_t)(8 + ((uint64_t)m * k >> 20)); }
 hipError_t launch_split_f32_f16x2(const void* x, int dtype, uint32_t m, uint32_t k, uint32_t x_stride, uint16_t* out,
-                                  uint32_t kp, int planes, int lo_at, int hi_at, float* inv, uint32_t* range,
+                                  uint32_t kp, int planes, int lo_at, int hi_at, float* inv, bool words, uint32_t* range,
                                   hipStream_t s);
 // An f32 image [pixels, cin] -> f16 [pixels, 2, cin] (lo, scaled up by another 2^12, and hi) with one scale: its inverse to
 // *inv. range: 3 words, cleared first; range[0] is set where the values lie too far apart. part: 2 kImageParts words

@@ -33,43 +33,20 @@ hipError_t launch_fill(void* p, size_t bytes, uint8_t byte, hipStream_t s) {
 hipError_t launch_zero(void* p, size_t bytes, hipStream_t s) { return launch_fill(p, bytes, 0, s); }
 
 // ------------------------------------------------------------------ f32 activations as three bf16 planes
-// out[r, p K + k] = plane p of x[r, k]: hi = bf16(x), mid = bf16(x - hi), lo = bf16(x - hi - mid). Each remainder is
-// exact in f32 (at most 16, then 8 significant bits), so hi + mid + lo == x for every normal f32 value and a GEMM
-// over the 3K planes against weights that repeat every K sums exact products of all 24 bits of x. One thread per 8
-// consecutive values of a row (two 16-byte loads, three 16-byte stores); x rows 16-byte aligned, K % 8 == 0.
 __global__ void __launch_bounds__(256) split_f32_planes_kernel(const float* __restrict__ x, uint32_t m, uint32_t k,
                                                               uint32_t xs, uint16_t* __restrict__ out) {
-  const uint32_t groups = k / 8;
-  const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (idx >= (size_t)m * groups) return;
-  const uint32_t r = (uint32_t)(idx / groups), g = (uint32_t)(idx % groups);
-  const float* src = x + (size_t)r * xs + (size_t)g * 8;
-  const f32x4 a = *(const f32x4*)src, b = *(const f32x4*)(src + 4);
-  const float v[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
-  uint32_t h[3][8];
-#pragma unroll
-  for (int i = 0; i < 8; i++) {
-    h[0][i] = f32_to_bf16(v[i]);
-    const float r1 = v[i] - bf16_to_f32((uint16_t)h[0][i]);
-    h[1][i] = f32_to_bf16(r1);
-    h[2][i] = f32_to_bf16(r1 - bf16_to_f32((uint16_t)h[1][i]));
-  }
-  uint16_t* dst = out + (size_t)r * 3 * k + (size_t)g * 8;
-#pragma unroll
-  for (int p = 0; p < 3; p++)
-    *(u32x4*)(dst + (size_t)p * k) = u32x4{h[p][0] | (h[p][1] << 16), h[p][2] | (h[p][3] << 16),
-                                           h[p][4] | (h[p][5] << 16), h[p][6] | (h[p][7] << 16)};
+  split_planes3(x, m, k, xs, out, (size_t)blockIdx.x * 256 + threadIdx.x, (size_t)gridDim.x * 256);
 }
 
 // ------------------------------------------------------------------ f32 operands as two f16 planes
-// v = 2^-e (hi + lo / L), L = 2^12 (kPlaneLo) or 1: with the row scaled by 2^e so that its largest finite |v| lies in
-// [2^14, 2^15), hi = f16(v 2^e) and lo = f16((v 2^e - hi) L) hold v to 2^-23 of itself, down to 2^-29 of the row's largest
-// with L = 2^12 (the remainder of that largest, at most 2^3, still fits), to 2^-20 of itself down to 2^-31, and to 2^-52 of
-// that largest below. The rounding of the sums in f32 is larger than the first of these (rel. error of 1024 x 6144 x 6144
-// against f64: see the GEMM's dispatch). Values below 2^-31 of the largest, but 0, are counted as tiny: with more than one of
-// them to 64 others in a row, or more than 8 + 2^-20 of all in the operand, the operand is not for planes, and the general
-// kernel runs in its place. (Normal data holds 1e-9 of them, products like silu(a) b 1e-7; an outlier with nothing else near it,
-// or a channel far below the others, many.) inf stays inf with a NaN beside it, as in the three bf16 planes.
+// v = 2^-e (hi + 2^-12 lo): with the row scaled by 2^e so that its largest finite |v| lies in [2^14, 2^15), hi = f16(v 2^e)
+// and lo = f16((v 2^e - hi) 2^12) hold v to 2^-23 of itself down to 2^-29 of the row's largest (whose remainder, at most
+// 2^3, still fits), to 2^-20 of itself down to 2^-31, and to 2^-52 of that largest below. The rounding of the sums in f32
+// is larger than the first of these (rel. error of 1024 x 6144 x 6144 against f64: see the GEMM's dispatch). Values below
+// 2^-31 of the largest, but 0, are counted as tiny: with more than one of them to 64 others in a row, or more than
+// 8 + 2^-20 of all in the operand, the planes are not used: three bf16 planes (GEMM) or the general kernel (convolution) run
+// instead, chosen on the device. (Normal data holds 1e-9 of them, products like silu(a) b 1e-7; a row with an outlier, or
+// a column far below the others, many.) inf stays inf with a NaN beside it, as in the three bf16 planes.
 constexpr float kPlaneLo = 4096.0f;
 constexpr uint32_t kPlaneTiny = 110u << 23;  // 2^-17, 2^-31 of the largest scaled value's power of two
 // The biased exponent of the scale for the largest finite |v| (its bits), and the inverse scale.
@@ -108,8 +85,7 @@ __device__ __forceinline__ uint32_t block_sum256(uint32_t v, uint32_t* red) {
   return red[0] + red[1] + red[2] + red[3];
 }
 // The planes of 8 values times s; counts the tiny ones.
-__device__ __forceinline__ void split_f16x2(const float (&v)[8], float s, float lo_scale, u32x4& lo, u32x4& hi,
-                                            uint32_t& tiny) {
+__device__ __forceinline__ void split_f16x2(const float (&v)[8], float s, u32x4& lo, u32x4& hi, uint32_t& tiny) {
 #pragma unroll
   for (int i = 0; i < 4; i++) {
     const float a = v[2 * i] * s, b = v[2 * i + 1] * s;
@@ -117,57 +93,68 @@ __device__ __forceinline__ void split_f16x2(const float (&v)[8], float s, float 
     tiny += (ba && ba < kPlaneTiny ? 1u : 0u) + (bb && bb < kPlaneTiny ? 1u : 0u);
     const uint32_t ha = f32_to_f16(a), hb = f32_to_f16(b);
     hi[i] = ha | (hb << 16);
-    lo[i] = (uint32_t)f32_to_f16((a - f16_to_f32((uint16_t)ha)) * lo_scale) |
-            ((uint32_t)f32_to_f16((b - f16_to_f32((uint16_t)hb)) * lo_scale) << 16);
+    lo[i] = (uint32_t)f32_to_f16((a - f16_to_f32((uint16_t)ha)) * kPlaneLo) |
+            ((uint32_t)f32_to_f16((b - f16_to_f32((uint16_t)hb)) * kPlaneLo) << 16);
   }
 }
 
-// One workgroup per row [k values at src + row * stride] -> f16 planes at out + row * planes * kp, zeros past k: plane
-// lo_at holds lo, plane hi_at hi (lo_at < 0: hi alone). The row's inverse scale goes to inv[row]. Two reads of the row
-// (the second from L2): k % 8 == 0, rows and out 16-byte aligned. range: the tiny values of all rows are added up in its
-// second word, and its first is set where they are too many (of a row, or more than `most` of all).
-template <int DT>
-__global__ void __launch_bounds__(256) split_f32_f16x2_kernel(const void* __restrict__ src, uint32_t k, uint32_t stride,
-                                                              uint16_t* __restrict__ out, uint32_t kp, int planes,
-                                                              int lo_at, int hi_at, float lo_scale, float* __restrict__ inv,
+// Rows [k values at src + row * stride] -> f16 planes at out + row * planes * kp, zeros past k: plane lo_at holds lo, plane
+// hi_at hi (lo_at < 0: hi alone). The row's inverse scale goes to inv[row]. Two reads of the row (the second from L2):
+// k % 8 == 0, rows and out 16-byte aligned. A workgroup takes the rows from blockIdx.x on in steps of the grid. Tiny values
+// (above; `most` is 8 + 2^-20 of all): WORDS, their number over the workgroup's rows to range[blockIdx.x], most + 1 where they
+// are too many already; else they are added to range[1], and range[0] is set where they are too many.
+template <int DT, bool WORDS>
+__global__ void __launch_bounds__(256) split_f32_f16x2_kernel(const void* __restrict__ src, uint32_t m, uint32_t k,
+                                                              uint32_t stride, uint16_t* __restrict__ out, uint32_t kp,
+                                                              int planes, int lo_at, int hi_at, float* __restrict__ inv,
                                                               uint32_t* __restrict__ range, uint32_t most) {
   __shared__ uint32_t red[4], red2[4], red3[4];
-  const size_t row = blockIdx.x, base = row * stride;
-  uint32_t m = 0, tiny = 0, nonzero = 0;
-  for (uint32_t i = threadIdx.x * 8; i < k; i += 2048) {
-    float v[8];
-    load8<DT>(src, base + i, v);
+  uint32_t total = 0;
+  for (size_t row = blockIdx.x; row < m; row += gridDim.x) {
+    const size_t base = row * stride;
+    uint32_t mx = 0, tiny = 0, nonzero = 0;
+    for (uint32_t i = threadIdx.x * 8; i < k; i += 2048) {
+      float v[8];
+      load8<DT>(src, base + i, v);
 #pragma unroll
-    for (int e = 0; e < 8; e++) {
-      m = max(m, finite_bits(v[e]));
-      nonzero += v[e] != 0.0f ? 1u : 0u;
+      for (int e = 0; e < 8; e++) {
+        mx = max(mx, finite_bits(v[e]));
+        nonzero += v[e] != 0.0f ? 1u : 0u;
+      }
+    }
+    const uint32_t se = plane_scale_exp(block_max256(mx, red));
+    const float s = __uint_as_float(se << 23);
+    if (threadIdx.x == 0) inv[row] = __uint_as_float((254u - se) << 23);
+    uint16_t* dst = out + row * (size_t)planes * kp;
+    for (uint32_t i = threadIdx.x * 8; i < kp; i += 2048) {
+      float v[8] = {};
+      if (i < k) load8<DT>(src, base + i, v);
+      u32x4 lo, hi;
+      split_f16x2(v, s, lo, hi, tiny);
+      *(u32x4*)(dst + (size_t)hi_at * kp + i) = hi;
+      if (lo_at >= 0) *(u32x4*)(dst + (size_t)lo_at * kp + i) = lo;
+    }
+    if (__syncthreads_or(tiny != 0)) {  // also before the next row's maxima
+      const uint32_t t = block_sum256(tiny, red2), n = block_sum256(nonzero, red3);
+      total = 64u * t > n - t ? most + 1 : min(total + t, most + 1);
+      __syncthreads();
     }
   }
-  const uint32_t se = plane_scale_exp(block_max256(m, red));
-  const float s = __uint_as_float(se << 23);
-  if (threadIdx.x == 0) inv[row] = __uint_as_float((254u - se) << 23);
-  uint16_t* dst = out + row * (size_t)planes * kp;
-  for (uint32_t i = threadIdx.x * 8; i < kp; i += 2048) {
-    float v[8] = {};
-    if (i < k) load8<DT>(src, base + i, v);
-    u32x4 lo, hi;
-    split_f16x2(v, s, lo_scale, lo, hi, tiny);
-    *(u32x4*)(dst + (size_t)hi_at * kp + i) = hi;
-    if (lo_at >= 0) *(u32x4*)(dst + (size_t)lo_at * kp + i) = lo;
-  }
-  if (range && __syncthreads_or(tiny != 0)) {
-    const uint32_t t = block_sum256(tiny, red2), n = block_sum256(nonzero, red3);
-    if (threadIdx.x == 0 && (64u * t > n - t || atomicAdd(range + 1, t) + t > most)) atomicOr(range, 1u);
+  if (threadIdx.x == 0) {
+    if constexpr (WORDS) range[blockIdx.x] = total;
+    else if (total && (total > most || atomicAdd(range + 1, total) + total > most)) atomicOr(range, 1u);
   }
 }
 
 hipError_t launch_split_f32_f16x2(const void* x, int dtype, uint32_t m, uint32_t k, uint32_t x_stride, uint16_t* out,
-                                  uint32_t kp, int planes, int lo_at, int hi_at, float* inv, uint32_t* range,
+                                  uint32_t kp, int planes, int lo_at, int hi_at, float* inv, bool words, uint32_t* range,
                                   hipStream_t s) {
   if (m == 0) return hipSuccess;
-  const auto kern = dtype == F32 ? split_f32_f16x2_kernel<F32> : split_f32_f16x2_kernel<BF16>;
-  hipLaunchKernelGGL(kern, dim3(m), dim3(256), 0, s, x, k, x_stride, out, kp, planes, lo_at, hi_at, range ? kPlaneLo : 1.0f,
-                     inv, range, (uint32_t)(8 + ((uint64_t)m * k >> 20)));
+  const auto kern = words            ? split_f32_f16x2_kernel<F32, true>
+                    : dtype == F32 ? split_f32_f16x2_kernel<F32, false>
+                                   : split_f32_f16x2_kernel<BF16, false>;
+  hipLaunchKernelGGL(kern, dim3(words ? range_words(m) : m), dim3(256), 0, s, x, m, k, x_stride, out, kp, planes, lo_at,
+                     hi_at, inv, range, planes_most_tiny(m, k));
   return hipGetLastError();
 }
 
@@ -211,7 +198,7 @@ __global__ void __launch_bounds__(256) image_f16x2_kernel(const float* __restric
     float v[8];
     load8<F32>(x, i, v);
     u32x4 lo, hi;
-    split_f16x2(v, s, kPlaneLo, lo, hi, tiny);
+    split_f16x2(v, s, lo, hi, tiny);
     uint16_t* dst = out + i / cin * 2 * cin + i % cin;
     *(u32x4*)dst = lo;
     *(u32x4*)(dst + cin) = hi;

@@ -6,6 +6,7 @@
 
 #include <atomic>
 #include <cstdarg>
+#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -968,6 +969,12 @@ void fill_gemm(we::GemmLaunch& L, const we::Tuning& t, const we_matmul_params* p
   L.scratch = nullptr;
 }
 
+// From where on two f16 planes of f32 rows pay for the launch behind them (which returns at once): 300 x 16384 x 512
+// (5 GFLOP) 34.7 us against 39.4 with three bf16 planes; 2048 x 4096 x 256 (4.3 GFLOP) 28.3 and 28.7, 4096 x 4096 x 128
+// 31.1 and 28.0, 128 x 3072 x 128 13.9 and 11.9
+constexpr double kTwoPlanesWork = 5e9;
+constexpr uint32_t kTwoPlanesK = 512;
+
 int matmul_impl(we_ctx* ctx, const we_matmul_params* p, int x_dtype, const void* x, int w_dtype, const void* w,
                 const void* w_scales, uint32_t group, int y_dtype, void* y, const float* bias, uint32_t flags,
                 const float* gate, const void* res, bool noalloc, int mul, const QkFuse* qk) {
@@ -1047,42 +1054,6 @@ int matmul_impl(we_ctx* ctx, const we_matmul_params* p, int x_dtype, const void*
       return e == hipSuccess ? WE_OK : hip_fail(ctx, e, "convolution launch");
     }
   }
-  // f32 activations (the reference's own dtype) on the fast path: x is split once into 16-bit planes along K in scratch and
-  // the fast kernel runs one GEMM over all planes with the weights read at k mod K. fp8 weights (exact in f16): two f16
-  // planes [M, 2K] (lo | hi), each row scaled by a power of two of its own, which hold x to 2^-23: a third fewer products
-  // and fewer f32 roundings than three planes (1024 x 6144 x 6144: error against f64 9.1e-7 -> 4.2e-7). Three bf16 planes
-  // [M, 3K] (hi | mid | lo), exactly x, for bf16 weights, whose range f16 lacks, for M <= 64 and for shapes that three
-  // planes run in more than two K slices: those short sums round less than the f16 planes do (17 x 6144 x 2048 1.1e-7 with
-  // three planes, 1.4e-7 with two; 128 x 2048 x 8192 1.6e-7 and 2.5e-7). Taken when the fast kernel accepts the planes
-  // (fp8 or bf16 weights, K a multiple of 64, aligned rows); otherwise, for the allocation-free entry point and for
-  // split-K partial modes, the general kernel splits x into three bf16 planes tile by tile.
-  size_t plane_bytes = 0, scale_at = 0;
-  if (x_dtype == WE_F32 && !noalloc && !split && !L.generic && !L.conv_width && p->k % 64 == 0 &&
-      (w_dtype == WE_FP8_E4M3 || w_dtype == WE_BF16) && (uintptr_t)x % 16 == 0 &&
-      (uint64_t)p->m * p->k * 3 <= (1ull << 30)) {
-    we::GemmLaunch P = L;
-    P.x = (const void*)(uintptr_t)256;  // placeholder with the scratch's alignment, for the check
-    auto set_planes = [&](uint32_t planes) {
-      P.x_dtype = planes == 2 ? WE_F16 : WE_BF16;
-      P.k = planes * p->k;
-      P.kc = P.k;
-      P.k_wrap = p->k;
-      P.x_stride = planes * p->k;
-      P.x_offset = 0;
-    };
-    uint32_t planes = 3;
-    set_planes(3);
-    if (w_dtype == WE_FP8_E4M3 && p->m > 64 && we::gemm_fast_supported(P) && we::gemm_reduce_plan(P).rsplits <= 2)
-      set_planes(planes = 2);
-    if (we::gemm_fast_supported(P)) {
-      L = P;
-      plane_bytes = ((uint64_t)p->m * planes * p->k * 2 + 255) / 256 * 256;
-      if (planes == 2) {
-        scale_at = plane_bytes;
-        plane_bytes += ((uint64_t)p->m * 4 + 255) / 256 * 256;
-      }
-    }
-  }
   const bool has_qk = qk && qk->q_heads + qk->k_heads;
   if (has_qk) {
     L.qk_cols = (qk->q_heads + qk->k_heads) * 128;
@@ -1095,59 +1066,121 @@ int matmul_impl(we_ctx* ctx, const we_matmul_params* p, int x_dtype, const void*
     L.qk_cos = qk->cos_t;
     L.qk_sin = qk->sin_t;
   }
-  we::GemmReducePlan rp{1, L.k, 0, -1, 1};
-  char* scratch = nullptr;  // the planes of x (plane_bytes), then the split-K partial sums
-  if (ctx->tune.gemm_splitk > 0) {  // that many slices (sweeps)
-    rp = we::gemm_reduce_plan(L, (uint32_t)ctx->tune.gemm_splitk);
-  } else if (ctx->tune.gemm_splitk < 0) {
-    rp = noalloc ? we::gemm_reduce_plan(L) : we::gemm_plan(L);
-    if (!noalloc && rp.scratch_bytes) {
+  // f32 activations (the reference's own dtype) on the fast path: x is split once into 16-bit planes along K in scratch and
+  // the fast kernel runs one GEMM over all planes with the weights read at k mod K. Taken when the fast kernel accepts the
+  // planes (fp8 or bf16 weights, K a multiple of 64, aligned rows); otherwise, for the allocation-free entry point and for
+  // split-K partial modes, the general kernel splits x into three bf16 planes tile by tile.
+  uint32_t planes = 0;
+  const float* xs = (const float*)x + p->x_offset;
+  auto planes_launch = [&](uint32_t n) {
+    we::GemmLaunch P = L;
+    P.x = (const void*)(uintptr_t)256;  // placeholder with the scratch's alignment, for the checks
+    P.x_dtype = n == 2 ? WE_F16 : WE_BF16;
+    P.k = n * p->k;
+    P.kc = P.k;
+    P.k_wrap = p->k;
+    P.x_stride = n * p->k;
+    P.x_offset = 0;
+    return P;
+  };
+  if (x_dtype == WE_F32 && !noalloc && !split && !L.generic && !L.conv_width && p->k % 64 == 0 &&
+      (w_dtype == WE_FP8_E4M3 || w_dtype == WE_BF16) && (uintptr_t)x % 16 == 0 &&
+      (uint64_t)p->m * p->k * 3 <= (1ull << 30) && we::gemm_fast_supported(planes_launch(3)))
+    planes = 3;
+  // the tile shape and K slices of a launch; a negative switch: the plan, 0: no slices, n: n slices (sweeps)
+  auto plan_of = [&](const we::GemmLaunch& G) {
+    if (ctx->tune.gemm_splitk > 0) return we::gemm_reduce_plan(G, (uint32_t)ctx->tune.gemm_splitk);
+    if (ctx->tune.gemm_splitk == 0) return we::GemmReducePlan{1, G.k, 0, -1, 1};
+    return noalloc ? we::gemm_reduce_plan(G) : we::gemm_plan(G);
+  };
+  auto launch_planned = [&](we::GemmLaunch& G, const we::GemmReducePlan& rp, void* part) {
+    if (rp.scratch_bytes) {
+      G.scratch = part;
+      G.rsplits = rp.rsplits;
+      G.rkc = rp.rkc;
+      G.tail_splits = rp.tail_splits;
+    }
+    G.rcfg = rp.rcfg;
+    if (!we::gemm_qk_fusable(G)) G.qk_cols = G.q_cols = 0;  // the plain GEMM, then the q/k pass below
+    return we::gemm_launch(G, ctx->compute);
+  };
+  bool launched = false, qk_fused = false;
+  // Two f16 planes [M, 2K] (lo | hi) for fp8 weights (exact in f16), each row scaled by a power of two of its own: a third
+  // fewer products and fewer f32 roundings than three bf16 planes (1024 x 6144 x 6144: error against f64 9.1e-7 -> 4.2e-7).
+  // Rows with values too far apart for them (kernels_misc.hip) are found on the device: then the launch writes the three
+  // exact planes [M, 3K] over the two, and the GEMM over them runs behind, which otherwise returns at once. Not for M <= 64 and shapes that three planes run in more
+  // than two K slices: those short sums round less than the f16 planes do (17 x 6144 x 2048 1.1e-7 with three planes,
+  // 1.4e-7 with two; 128 x 2048 x 8192 1.6e-7 and 2.5e-7); nor where the products are too few to pay for the launches.
+  if (planes && w_dtype == WE_FP8_E4M3 && p->m > 64 && !(has_qk && y_dtype != WE_F32) &&
+      2.0 * p->m * p->n * p->k >= kTwoPlanesWork && p->k >= kTwoPlanesK &&
+      we::gemm_reduce_plan(planes_launch(3)).rsplits <= 2 &&
+      we::gemm_fast_supported(planes_launch(2))) {
+    we::GemmLaunch two = planes_launch(2), three = planes_launch(3);
+    const we::GemmReducePlan rp2 = plan_of(two), rp3 = we::gemm_reduce_plan(three);  // three: as few launches as can be
+    auto round256 = [](uint64_t n) { return (size_t)((n + 255) / 256 * 256); };
+    const size_t scale_at = round256((uint64_t)p->m * 3 * p->k * 2), range_at = scale_at + round256((uint64_t)p->m * 4);
+    const size_t part_at = range_at + we::kRangeWords * 4 + 256;
+    char* scratch = (char*)try_scratch(ctx, part_at + std::max(rp2.scratch_bytes, rp3.scratch_bytes));
+    if (scratch) {
+      float* inv = (float*)(scratch + scale_at);
+      uint32_t* range = (uint32_t*)(scratch + range_at);
+      two.x = three.x = scratch;
+      two.row_scale = inv;
+      two.range = range;
+      two.range_n = we::range_words(p->m);
+      two.range_most = we::planes_most_tiny(p->m, p->k);
+      two.skip_out = range + we::kRangeWords;
+      two.f32 = xs;
+      two.f32_stride = p->x_stride;
+      three.only_if = two.skip_out;
+      hipError_t e = we::launch_split_f32_f16x2(xs, WE_F32, p->m, p->k, p->x_stride, (uint16_t*)scratch, p->k, 2, 0, 1, inv,
+                                                true, range, ctx->compute);
+      if (e == hipSuccess) e = launch_planned(two, rp2, scratch + part_at);
+      if (e == hipSuccess) e = launch_planned(three, rp3, scratch + part_at);
+      if (e != hipSuccess) return hip_fail(ctx, e, "f32 plane launches");
+      launched = true;
+    }
+  }
+  if (!launched) {
+    size_t plane_bytes = 0;
+    if (planes) {
+      L = planes_launch(3);
+      plane_bytes = ((uint64_t)p->m * 3 * p->k * 2 + 255) / 256 * 256;
+    }
+    we::GemmReducePlan rp = plan_of(L);
+    char* scratch = nullptr;  // the planes of x (plane_bytes), then the split-K partial sums
+    if (ctx->tune.gemm_splitk < 0 && !noalloc && rp.scratch_bytes) {
       scratch = (char*)try_scratch(ctx, plane_bytes + rp.scratch_bytes);
       if (!scratch) rp = we::gemm_reduce_plan(L);
     }
-  }
-  const size_t part_bytes = rp.scratch_bytes;
-  if (!scratch && plane_bytes + part_bytes) {
-    if (noalloc) {
-      // the device's fixed scratch array: no allocation, a hard size limit
-      if (part_bytes > we::kNoallocScratchBytes)
-        return fail(ctx, WE_EINVAL,
-                    "this GEMM (M %u, N %u, K %u) needs %zu bytes of split-K scratch; the allocation-free entry "
-                    "point has %zu (use we_matmul)",
-                    p->m, p->n, p->k, part_bytes, we::kNoallocScratchBytes);
-      scratch = (char*)we::noalloc_scratch(ctx->device);
-      if (!scratch) return fail(ctx, WE_EHIP, "allocation-free scratch of device %d is not set up", ctx->device);
-    } else {
-      const int rc = ensure_scratch(ctx, plane_bytes + part_bytes);
-      if (rc) return rc;
-      scratch = (char*)ctx->scratch;
+    const size_t part_bytes = rp.scratch_bytes;
+    if (!scratch && plane_bytes + part_bytes) {
+      if (noalloc) {
+        // the device's fixed scratch array: no allocation, a hard size limit
+        if (part_bytes > we::kNoallocScratchBytes)
+          return fail(ctx, WE_EINVAL,
+                      "this GEMM (M %u, N %u, K %u) needs %zu bytes of split-K scratch; the allocation-free entry "
+                      "point has %zu (use we_matmul)",
+                      p->m, p->n, p->k, part_bytes, we::kNoallocScratchBytes);
+        scratch = (char*)we::noalloc_scratch(ctx->device);
+        if (!scratch) return fail(ctx, WE_EHIP, "allocation-free scratch of device %d is not set up", ctx->device);
+      } else {
+        const int rc = ensure_scratch(ctx, plane_bytes + part_bytes);
+        if (rc) return rc;
+        scratch = (char*)ctx->scratch;
+      }
     }
-  }
-  if (plane_bytes) {
-    L.x = scratch;
-    const float* xs = (const float*)x + p->x_offset;
-    hipError_t e;
-    if (scale_at) {
-      float* inv = (float*)(scratch + scale_at);
-      L.row_scale = inv;
-      e = we::launch_split_f32_f16x2(xs, WE_F32, p->m, p->k, p->x_stride, (uint16_t*)scratch, p->k, 2, 0, 1, inv,
-                                     nullptr, ctx->compute);
-    } else {
-      e = we::launch_split_f32_planes(xs, p->m, p->k, p->x_stride, (uint16_t*)scratch, ctx->compute);
+    if (plane_bytes) {
+      L.x = scratch;
+      const hipError_t e =
+          we::launch_split_f32_planes(xs, p->m, p->k, p->x_stride, (uint16_t*)scratch, ctx->compute);
+      if (e != hipSuccess) return hip_fail(ctx, e, "f32 plane split launch");
     }
-    if (e != hipSuccess) return hip_fail(ctx, e, "f32 plane split launch");
+    const hipError_t e = launch_planned(L, rp, scratch + plane_bytes);
+    if (e != hipSuccess) return hip_fail(ctx, e, "gemm launch");
+    qk_fused = has_qk && L.qk_cols;
   }
-  if (part_bytes) {
-    L.scratch = scratch + plane_bytes;
-    L.rsplits = rp.rsplits;
-    L.rkc = rp.rkc;
-    L.tail_splits = rp.tail_splits;
-  }
-  L.rcfg = rp.rcfg;
-  const bool qk_fused = has_qk && we::gemm_qk_fusable(L);
-  if (!qk_fused) L.qk_cols = L.q_cols = 0;  // the plain GEMM, then the q/k pass below
-  hipError_t e = we::gemm_launch(L, ctx->compute);
-  if (e != hipSuccess) return hip_fail(ctx, e, "gemm launch");
+  hipError_t e;
   if (qk && !qk_fused) {
     // no head-aligned tile for this shape: the q and k heads in a pass of their own, in place
     const uint64_t yb = elem_bytes(y_dtype);
