@@ -125,3 +125,33 @@ def test_fused_qkv_refusals(graph):
         graph.matmul_qk_norm_rope(p, we.BF16, b, we.FP8, b, we.BF16, b, 1, 1, 1e-6, 1.0, b, b, flags=we.EPI_GELU)
     with pytest.raises(we.WeError, match="cos and sin go together"):
         graph.matmul_qk_norm_rope(p, we.BF16, b, we.FP8, b, we.BF16, b, 1, 1, 1e-6, 1.0, b, b, 0, b, None)
+
+
+@pytest.mark.parametrize("m,heads,kv_heads,k", [(333, 24, 24, 3072), (400, 24, 24, 3072), (1100, 32, 8, 4096)])
+def test_planned_tiles_keep_the_norm_on_unrounded_values(graph, m, heads, kv_heads, k):
+    """Shapes whose tiles the q / k epilogue can run on (128 x 128, 256 x 128): the planned launch normalizes the f32 sums, so q
+    and k carry one rounding to bf16 (the rms error of the rounded oracle, a tenth more for the f32 sums), not two (1.4
+    times that)."""
+    n = (heads + 2 * kv_heads) * 128
+    rng = np.random.default_rng(m)
+    x = O.bf16_rne(rng.standard_normal(m * k).astype(np.float32))
+    w = rng.integers(0, 254, n * k).astype(np.uint8)
+    w = (w + (w >= 0x7F)).astype(np.uint8)
+    nq = rng.uniform(-.3, .3, 128).astype(np.float32)
+    p = we.matmul_params(m, n, k, 0.05, graph=graph)
+    mark = graph.mark()
+    y, qb = graph.buffer(m * n * 2), graph.buffer(nq)
+    graph.matmul_qk_norm_rope(p, we.BF16, graph.buffer(x), we.FP8, graph.buffer(w), we.BF16, y, heads, kv_heads, 1e-6, 1.0,
+                              qb, qb, 0, None, None)
+    got = O.bf16_to_f32(graph.read(y).view(np.uint16)).astype(np.float64).reshape(m, n)
+    graph.release(mark)
+    err = exact = 0.0
+    cols = (heads + kv_heads) * 128
+    for r in (0, 127, 300, m - 1):
+        v = O.matmul_rows(O.matmul_params(m, n, k, 0.05), O.BF16, x, O.FP8, w, r, r + 1)[r * n:r * n + cols]
+        v = v.reshape(-1, 128)
+        want = v / np.sqrt((v ** 2).mean(axis=1, keepdims=True) + 1e-6) * (1.0 + nq.astype(np.float64))
+        rounded = O.bf16_to_f32(O.bf16_rne(want.astype(np.float32).reshape(-1))).astype(np.float64).reshape(want.shape)
+        err += ((got[r, :cols].reshape(want.shape) - want) ** 2).sum()
+        exact += ((rounded - want) ** 2).sum()
+    assert np.sqrt(err / exact) < 1.1, np.sqrt(err / exact)

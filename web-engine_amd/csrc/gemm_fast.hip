@@ -191,17 +191,23 @@ GemmReducePlan gemm_plan(const GemmLaunch& L) {
   // 256 x 192 tiles, 5% ahead of the 256 x 256 ones (91.5 us).
   GemmReducePlan best = gemm_reduce_plan(L);
   const uint32_t older = best.rsplits;
+  // Where the older choice runs the q / k epilogue, so does every other: the epilogue normalizes the f32 sums, the pass of its
+  // own the values rounded to y's type (400 x 9216 x 3072 bf16 in 64 x 64 tiles and the pass: 1.4 times the rounding error)
+  GemmLaunch O = L;
+  O.rsplits = best.rsplits;
+  O.rcfg = best.rcfg;
+  const bool fused = L.qk_cols && gemm_qk_fusable(O);
   best.rcfg = best.rcfg >= 0 ? best.rcfg : pick_fast_cfg(L.m, L.n, best.rsplits, w8);
   double best_us = 0.94 * predict(best.rcfg, best.rsplits, best.rsplits > 1 ? best.rkc : L.k);
   for (const int cfg : {GEMM_CFG_256x256, GEMM_CFG_256x192, GEMM_CFG_256x128, GEMM_CFG_128x128, GEMM_CFG_64x64}) {
-    if (cfg_bm(cfg) == 256 && L.m < 256) continue;
+    if ((cfg_bm(cfg) == 256 && L.m < 256) || (fused && !qk_fusable_cfg(cfg))) continue;
     const uint64_t tiles = (uint64_t)((L.m + cfg_bm(cfg) - 1) / cfg_bm(cfg)) * ((L.n + cfg_bn(cfg) - 1) / cfg_bn(cfg));
     // slices only where the tiles fill at most half of the CUs (128 x 128: twice that), as swept
     const uint32_t most = tiles * 2 <= kCUs * (cfg == GEMM_CFG_128x128 ? 2u : 1u) ? std::min(8u, L.k / 256) : 1u;
     // three planes of x: a multiple of the older plan's slices, whose shorter sums round less and may end with the planes
     // (800 x 4096 x 8192: error 3.3e-7 in 3 slices, 3.8e-7 in 4)
     for (uint32_t rs = 1; rs <= most; rs++) {
-      if (three && rs % older) continue;
+      if ((three && rs % older) || (fused && rs > 1)) continue;
       const uint32_t kc = (L.k + rs * BK - 1) / (rs * BK) * BK;
       if ((L.k + kc - 1) / kc != rs) continue;
       const double us = predict(cfg, rs, kc);
