@@ -172,7 +172,11 @@ int we_timer_between(we_ctx* ctx, uint32_t from, uint32_t to, float* ms);
  * Kernels that need scratch (split-K partial sums, attention's V^T) replay into the scratch block of the stream
  * they were captured on: a graph keeps that block alive until we_graph_destroy, also when a later eager call
  * outgrows it, and we_graph_launch refuses to run a graph while the other compute stream is selected. Replays
- * of graphs captured on one stream share that stream's scratch, so they run one after another in its order. */
+ * of graphs captured on one stream share that stream's scratch, so they run one after another in its order.
+ * A capture cannot make that block larger. A call that cannot do without is refused ("run the call once before capturing
+ * it"); one that has a slower path without, or with less (f32 attention, the 3x3 convolution, int4 weights for many rows, planned
+ * GEMMs of M > 64), is captured on that path, up to ten times slower and with other roundings. So run every call once
+ * at its sizes before capturing it; the same holds for a block that the allocation cap keeps from growing. */
 typedef struct we_graph we_graph;
 int we_graph_begin(we_ctx* ctx);
 int we_graph_end(we_ctx* ctx, we_graph** graph);

@@ -88,3 +88,40 @@ def test_poison_fills_freed_and_released_buffers_with_nan(ctx):
     assert np.array_equal(ctx.read(kept, dtype=np.float32), data)
     assert (ctx.read(dropped, dtype=np.uint8) == 0xFF).all()
     ctx.set_poison(False)
+
+
+def test_a_refused_larger_scratch_leaves_the_old_one():
+    """A call that would like more scratch than the allocation cap leaves runs without it, and the block that was there stays
+    for the calls that fit in it: also where a live graph holds that block."""
+    g = we.Graph(0)
+    try:
+        rng = np.random.default_rng(3)
+        m, n, k = 64, 3072, 3072
+        x = g.buffer(rng.standard_normal(m * k).astype(np.float16))
+        w = rng.integers(0, 254, n * k).astype(np.uint8)
+        w = g.buffer((w + (w >= 0x7F)).astype(np.uint8))
+        y, y2 = g.buffer(m * n * 2), g.buffer(m * n * 2)
+        p = we.matmul_params(m, n, k, 0.02, graph=g)
+        g.matmul(p, we.F16, x, we.FP8, w, we.F16, y)  # 16 MiB of scratch
+        g.graph_begin()
+        g.matmul(p, we.F16, x, we.FP8, w, we.F16, y)
+        gr = g.graph_end()
+        tokens, heads, dim = 4001, 9, 128
+        q = g.buffer(rng.standard_normal(tokens * heads * dim).astype(np.float32))
+        o = g.buffer(tokens * heads * dim * 4)
+        held = g.set_alloc_cap(0)
+        # planes of K and V: 2 x 4001 x 9 x 2 x 128 x 2 bytes and some; the block would be rounded up past the cap
+        need = 2 * ((tokens * heads * 2 * dim * 2 + 255) // 256 * 256)
+        for extra in range(0, 1 << 16, 256):
+            g.set_alloc_cap(held + need + extra)
+            g.attention(tokens, heads, heads, dim, False, we.F32, q, q, q, o)
+            if g.set_alloc_cap(0) != held:
+                break  # it fit
+            g.graph_begin()
+            g.matmul(p, we.F16, x, we.FP8, w, we.F16, y2)  # refused in a capture if the block were gone
+            g.graph_destroy(g.graph_end())
+        g.graph_launch(gr)
+        g.sync()
+        g.graph_destroy(gr)
+    finally:
+        g.destroy()

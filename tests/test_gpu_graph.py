@@ -149,3 +149,28 @@ def test_graph_keeps_its_scratch_when_an_eager_call_outgrows_it():
         g.stream(0)
     finally:
         g.destroy()
+
+
+def test_a_capture_without_scratch_takes_the_path_that_needs_none():
+    """f32 attention captured by a context that never ran it: the replay is the f32 MFMA kernel's result."""
+    g = we.Graph(0)
+    try:
+        rng = np.random.default_rng(5)
+        tokens, heads, dim = 300, 2, 128
+        h = rng.standard_normal(tokens * heads * dim).astype(np.float32)
+        q = g.buffer(h)
+        o, o2 = g.buffer(h.nbytes), g.buffer(h.nbytes)
+        g.sync()
+        g.graph_begin()
+        g.attention(tokens, heads, heads, dim, True, we.F32, q, q, q, o)
+        gr = g.graph_end()
+        g.set_tuning("attn_path", 1)
+        g.attention(tokens, heads, heads, dim, True, we.F32, q, q, q, o2)
+        want = g.read(o2).copy()
+        for _ in range(3):
+            g.write(o, np.zeros(h.nbytes, np.uint8))
+            g.graph_launch(gr)
+            assert np.array_equal(g.read(o), want)
+        g.graph_destroy(gr)
+    finally:
+        g.destroy()

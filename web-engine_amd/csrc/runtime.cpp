@@ -118,6 +118,30 @@ hipError_t scratch_free(we_ctx* ctx, void* p) {
   return hipFree(p);
 }
 
+// Gives the scratch block back: freed when the work that may still read it is done, or kept until the live graphs that
+// replay into it go.
+int drop_scratch(we_ctx* ctx) {
+  if (!ctx->scratch) return WE_OK;
+  auto held = ctx->scratch_refs.find(ctx->scratch);
+  if (held != ctx->scratch_refs.end() && held->second > 0) {
+    ctx->retired.push_back(ctx->scratch);
+  } else {
+    HIP_OK(ctx, hipStreamSynchronize(ctx->compute), "hipStreamSynchronize");
+    HIP_OK(ctx, scratch_free(ctx, ctx->scratch), "hipFree scratch");
+  }
+  ctx->scratch = nullptr;
+  ctx->scratch_bytes = 0;
+  return WE_OK;
+}
+
+size_t scratch_size(size_t bytes) { return ((bytes < (16u << 20) ? (16u << 20) : bytes) + 4095) / 4096 * 4096; }
+
+void set_scratch(we_ctx* ctx, void* p, size_t bytes) {
+  ctx->scratch_sizes[p] = bytes;
+  ctx->scratch = p;
+  ctx->scratch_bytes = bytes;
+}
+
 // Scratch for kernels of this context (split-K partial sums, attention V^T), at least `bytes`. Calls are ordered on the
 // compute stream, so one buffer serves them all; growing it waits for the work that may still read it.
 int ensure_scratch(we_ctx* ctx, size_t bytes) {
@@ -125,38 +149,38 @@ int ensure_scratch(we_ctx* ctx, size_t bytes) {
   if (ctx->capturing)
     return fail(ctx, WE_EINVAL, "scratch must grow to %zu bytes: run the call once before capturing it", bytes);
   HIP_OK(ctx, hipSetDevice(ctx->device), "hipSetDevice");
-  if (ctx->scratch) {
-    auto held = ctx->scratch_refs.find(ctx->scratch);
-    if (held != ctx->scratch_refs.end() && held->second > 0) {
-      ctx->retired.push_back(ctx->scratch);  // a live graph replays into it: keep it until that graph goes
-    } else {
-      HIP_OK(ctx, hipStreamSynchronize(ctx->compute), "hipStreamSynchronize");
-      HIP_OK(ctx, scratch_free(ctx, ctx->scratch), "hipFree scratch");
-    }
-    ctx->scratch = nullptr;
-    ctx->scratch_bytes = 0;
-  }
-  const size_t want = ((bytes < (16u << 20) ? (16u << 20) : bytes) + 4095) / 4096 * 4096;
+  const int rc = drop_scratch(ctx);
+  if (rc) return rc;
+  const size_t want = scratch_size(bytes);
   void* p = nullptr;
   const hipError_t e = capped_malloc(ctx, &p, want);
   if (e != hipSuccess) return fail(ctx, WE_ENOMEM, "scratch of %zu bytes: %s%s", want, hipGetErrorString(e),
                                    ctx->alloc_cap ? " (allocation cap set)" : "");
-  ctx->scratch_sizes[p] = want;
-  ctx->scratch = p;
-  ctx->scratch_bytes = want;
+  set_scratch(ctx, p, want);
   return WE_OK;
 }
 
-// The scratch of a path that has another one without it: null, and no error left behind, where it cannot be had (a
-// graph is being captured, the allocation cap or the device is full).
+// The scratch of a path that has another one without it: null, no error left behind and the block that was there kept, where
+// it cannot be had beside that block (a graph is being captured, the allocation cap or the device is full).
 void* try_scratch(we_ctx* ctx, size_t bytes) {
   if (bytes <= ctx->scratch_bytes) return ctx->scratch;
-  if (ctx->capturing || (ctx->alloc_cap && ctx->held_bytes + bytes > ctx->alloc_cap)) return nullptr;
+  if (ctx->capturing) return nullptr;
+  const size_t want = scratch_size(bytes);
+  void* p = nullptr;
+  if (hipSetDevice(ctx->device) != hipSuccess || capped_malloc(ctx, &p, want) != hipSuccess) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  ctx->scratch_sizes[p] = want;
   const std::string before = ctx->err;
-  if (ensure_scratch(ctx, bytes) == WE_OK) return ctx->scratch;
-  ctx->err = before;
-  (void)hipGetLastError();
-  return nullptr;
+  if (drop_scratch(ctx) != WE_OK) {
+    ctx->err = before;
+    (void)scratch_free(ctx, p);
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  set_scratch(ctx, p, want);
+  return p;
 }
 
 size_t round_size(size_t bytes) { return ((bytes < 4 ? 4 : bytes) + 255) / 256 * 256; }
