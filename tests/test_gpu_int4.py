@@ -168,10 +168,10 @@ def test_tiny_shapes(graph, m, n, k, group):
 @pytest.mark.parametrize("m,n,k,group,x_dt,y_dt,flags", [
     (33, 2061, 4096, 64, we.F16, we.F32, 0),            # 64 x 64 tiles, K slices, a ragged last column tile
     (64, 4100, 1536, 128, we.BF16, we.F16, we.EPI_BIAS),  # two 64-k blocks per scale group
-    (65, 1200, 4096, 4096, we.F16, we.F32, we.EPI_GELU),  # 128 x 128 tiles, one group per row
+    (65, 1200, 4096, 4096, we.F16, we.F32, we.EPI_GELU),  # one group per row
     (129, 700, 4096, 64, we.BF16, we.F32, 0), (300, 1024, 1344, 192, we.F16, we.BF16, 0)])
 def test_tiles_for_many_rows(graph, tune, m, n, k, group, x_dt, y_dt, flags):
-    """M > 32 with a large weight matrix: the GEMM tiles (ragged tiles, K slices, scale buffers refilled every 8 blocks)
+    """M > 32 with a large weight matrix: 64 x 64 GEMM tiles (ragged tiles, K slices, scale buffers refilled every 8 blocks)
     against the oracle, and against the GEMV kernels, which sum the same exact products in another order (f32: 2e-6)."""
     rng = np.random.default_rng(m + n)
     words, scales, x, ox = make(rng, m, n, k, group, x_dt)
@@ -188,3 +188,37 @@ def test_tiles_for_many_rows(graph, tune, m, n, k, group, x_dt, y_dt, flags):
         tune(int4_path=1)
         gemv = run(graph, m, n, k, group, words, scales, x, x_dt, y_dt, bias=bias, flags=flags)
         assert O.rel_error(got, gemv) < 2e-6
+
+
+@pytest.mark.parametrize("cfg,m,n,k,group,x_dt", [
+    (-1, 257, 5500, 1536, 128, we.F16),  # 129 tiles of 128 x 128: that shape unforced
+    (-1, 300, 11000, 768, 64, we.BF16),  # 258 of them: no K slices
+    (2, 129, 6100, 448, 64, we.F16), (3, 129, 6100, 448, 64, we.BF16),  # no slices, fewer blocks than a scale buffer holds
+    (2, 129, 700, 4096, 64, we.BF16), (2, 33, 12300, 1088, 1088, we.F16),  # slices; most of the tile's rows past M
+    (2, 300, 2061, 1344, 192, we.F16), (3, 300, 2061, 1344, 192, we.BF16)])
+def test_both_tile_shapes(graph, tune, cfg, m, n, k, group, x_dt):
+    """The 128 x 128 tiles (gemm_cfg 2: two halves of a wave's rows, four scales per thread, two stages) and the 64 x 64 ones (3),
+    with and without K slices, ragged in both directions: rows of every tile against the oracle, all of them against the GEMV
+    kernels (the same exact products in another order), plain and with a gated residual."""
+    rng = np.random.default_rng(m + n)
+    words, scales, x, ox = make(rng, m, n, k, group, x_dt)
+    tune(gemm_cfg=cfg)
+    got = run(graph, m, n, k, group, words, scales, x, x_dt, we.F32).reshape(m, n)
+    for r in sorted({0, 31, 32, min(64, m - 1), min(127, m - 1), min(128, m - 1), m - 1}):
+        want = O.matmul_rows(O.matmul_params(m, n, k, 1.0), ox, x, O.INT4, words, r, r + 1, scales=scales, group=group)
+        assert O.rel_error(got[r], want[r * n:(r + 1) * n]) < 1e-5, r
+    gate, res = rng.uniform(-1, 1, n).astype(np.float32), rng.standard_normal(m * n).astype(np.float32)
+
+    def gated():
+        mark = graph.mark()
+        y = graph.buffer(m * n * 4)
+        graph.matmul(we.matmul_params(m, n, k, 1.0, graph=graph), x_dt, graph.buffer(x), we.INT4, graph.buffer(words), we.F32, y,
+                     scales=graph.buffer(scales), group=group, gate=graph.buffer(gate), residual=graph.buffer(res))
+        v = graph.read(y, dtype=np.float32).astype(np.float64).reshape(m, n)
+        graph.release(mark)
+        return v
+
+    tiles = gated()
+    tune(int4_path=1)
+    assert O.rel_error(got, run(graph, m, n, k, group, words, scales, x, x_dt, we.F32).reshape(m, n)) < 2e-6
+    assert O.rel_error(tiles, gated()) < 2e-6

@@ -793,10 +793,10 @@ def test_conv3x3_planes_of_wide_ranges(graph, what, e, w_dt):
         assert O.rel_error(got[:, c], want[:, c]) < 1e-5, c
 
 
-@pytest.mark.parametrize("k", [128, 1024])  # two f16 planes; three bf16 planes (a K-sliced plan)
+@pytest.mark.parametrize("k", [128, 1024])  # whole and in K slices
 def test_f32_rows_of_any_scale(graph, k):
-    """The two f16 planes of an f32 row carry a power of two of the row's own: rows at 2^100, 2^-100, all zeros and with one
-    value 2^12 above the rest, each to f32's precision by its own size."""
+    """f32 rows at 2^100, 2^-100, all zeros and with one value 2^12 above the rest, each to f32's precision by its own size
+    (three bf16 planes here; test_f32_rows_of_wide_range has the shapes for two f16 planes)."""
     m, n = 70, 512
     rng = np.random.default_rng(8)
     x = rng.standard_normal((m, k)).astype(np.float32)
@@ -874,14 +874,27 @@ def test_f32_rows_of_wide_range(graph, m, n, k, e, epi):
 @pytest.mark.parametrize("m,n,k,w_dt", [(65, 1040, 2048, we.FP8), (129, 520, 4096, we.BF16), (300, 1028, 1024, we.FP8),
                                         (520, 260, 3072, we.FP8), (700, 400, 512, we.BF16)])
 def test_planned_tiles_and_slices(graph, m, n, k, w_dt):
-    """M > 64: whatever tile shape and K slices the cost model picks (few tiles: 64 x 64 and 256 x 256 in slices, ragged
-    last tiles), against the oracle."""
+    """M > 64: whatever tile shape and K slices the cost model picks (few tiles: 64 x 64 in 4 and 8 slices, 128 x 128 in 2 and
+    16, ragged last tiles), against the oracle."""
     rng = np.random.default_rng(m)
     x_store, x_oracle, ox = encode_act(rng.standard_normal(m * k).astype(np.float32), we.BF16)
     w_store, w_oracle, ow = make_weights(rng, n, k, w_dt)
     p = we.matmul_params(m, n, k, 0.05, graph=graph)
     got = run(graph, p, x_store, we.BF16, w_store, w_dt, we.F32)
     assert O.rel_error(got, O.matmul(O.matmul_params(m, n, k, 0.05), ox, x_oracle, ow, w_oracle)) < TOL_F32_OUT
+
+
+@pytest.mark.parametrize("m,n,k", [(700, 1544, 6144), (400, 3000, 8192), (700, 3072, 12288)])
+def test_planned_slices_of_256_row_tiles(graph, m, n, k):
+    """Shapes that the cost model runs in slices of 256 x 128 (6), 256 x 192 (8) and 256 x 256 (7) tiles, ragged in both
+    directions but the last: rows of every row of tiles against the oracle."""
+    rng = np.random.default_rng(n)
+    x = O.bf16_rne(rng.standard_normal(m * k).astype(np.float32))
+    w_store, w_oracle, ow = make_weights(rng, n, k, we.FP8)
+    got = run(graph, we.matmul_params(m, n, k, 0.05, graph=graph), x, we.BF16, w_store, we.FP8, we.F32).reshape(m, n)
+    for r in (0, 255, 256, 390, m - 1):
+        want = O.matmul_rows(O.matmul_params(m, n, k, 0.05), O.BF16, x, ow, w_oracle, r, r + 1)[r * n:(r + 1) * n]
+        assert O.rel_error(got[r], want) < TOL_F32_OUT, r
 
 
 F32_FAST_CASES = [
@@ -895,7 +908,7 @@ F32_FAST_CASES = [
 @pytest.mark.parametrize("m,n,k,w_dt,flags", F32_FAST_CASES)
 def test_f32_activations_on_the_fast_path(graph, tune, m, n, k, w_dt, flags):
     """f32 x, the reference's own activation dtype (src/kernels/matmul.ts:129-131), with fp8 or bf16 weights and K a
-    multiple of 64: split into two f16 planes (fp8 weights) or three exact bf16 planes (bf16 weights) and run by the
+    multiple of 64: split into three exact bf16 planes, or two f16 planes (fp8 weights, 5 GFLOP and more), and run by the
     fast kernel over all of them. It matches the float64 oracle at the reference's 1e-5 bar, and the general kernel
     (three bf16 planes tile by tile) to 4e-6: the f32 summation order differs (at K = 3072, sums of ~200 move by
     ~1.5e-6 of max|y| between two orders), the f16 planes hold x to 2^-23."""
