@@ -33,6 +33,8 @@
 // the weights are read at k mod K (K a multiple of 64, so no 64-k block spans two planes), so every epilogue applies to the
 // whole sum. The CONV kernels read x as an f16 image and gather each tap's pixels by the loads' addresses (gemm_conv.hip).
 #pragma once
+#include <cstddef>
+
 #include "common.h"
 #include "internal.h"
 
@@ -45,60 +47,67 @@ hipError_t gemm_lds_bf16_bf16(const FastArgs& a, uint32_t splits, int cfg, int r
 hipError_t gemm_lds_f16_fp8(const FastArgs& a, uint32_t splits, int cfg, int reduce_xcd, hipStream_t s);
 hipError_t gemm_lds_f16_f16(const FastArgs& a, uint32_t splits, int cfg, int reduce_xcd, hipStream_t s);
 
+// Ordered by use: a kernel's first instructions wait for the argument words they read, 64 bytes at a time, so what every
+// launch needs before its first load stands in the first 128, what its epilogue needs in the next 64, and what only some
+// launches need behind.
 struct FastArgs {
   const void* x;
   const void* w;
-  void* y;
-  const float* bias;
-  const float* gate;  // gated residual: y = res + gate[col] * v (res may be y; NULL: none)
-  const void* res;
   uint32_t x_bytes, w_bytes;  // readable bytes from x / w (their extents)
   uint32_t m, n, k;
+  uint32_t kc;
+  uint32_t x_stride, w_stride;  // x / w already point at their offsets
   // weights read at k - kwrap (k >= kwrap) and k - kwrap2 (k >= kwrap2): x holds k / kwrap planes of kwrap values per
   // row (GemmLaunch::k_wrap); 0xffffffff: no wrap
   uint32_t kwrap, kwrap2;
-  float scale;
-  uint32_t x_stride, w_stride, y_stride, y_offset;  // x / w already point at their offsets
-  uint32_t kc;
   uint32_t tiles_m, tiles_n;
-  uint32_t flags, y_dtype;
-  uint32_t vec_store;  // 1: y rows and y_offset allow 4-value vector stores
-  uint32_t store16;    // 1: y, y_offset and y rows are 16-byte aligned (whole-row staging of 16-bit outputs)
+  // A second GEMM in the same launch (gemm_fast_launch_pair; g below): tiles from grp_first on (after the XCD renumbering)
+  // compute it; grp_first 0: none.
+  uint32_t grp, grp_first;
+  // A split last round (tail_tiles > 0; GemmReducePlan::tail_splits): the tiles from tail_first on, a multiple of the CUs,
+  // run as tail_splits K slices of tail_kc each, whose raw sums go to part as dense tiles, slice-major
+  uint32_t tail_first, tail_tiles, tail_splits, tail_kc;
+  // Launches that decide on the device whether they run. skip_if: CONV kernels and reduce passes do nothing where this word
+  // is not 0 (NULL: they run); only_if: fp8 kernels for bf16 x and reduce passes do nothing where it is 0 (NULL: they run).
+  const uint32_t* skip_if;
+  const uint32_t* only_if;
   // split-K partial sums (rsplits > 1): slice z stores its raw sums at part + z * m * n (dense rows of n);
   // splitk_reduce_kernel adds the slices and runs the epilogue
   float* part;
   uint32_t rsplits;
-  // int4 weights (w: u32 [N, K / 8], rows contiguous): f16 scales [N, sc_groups], one per sc_blocks 64-k blocks
-  const uint16_t* sc;
-  uint32_t sc_groups, sc_blocks;
+  // Two f16 planes, range_n > 0: the tiny values that split_f32_f16x2_kernel counted, by workgroup; more than range_most
+  // of them and the kernel splits the f32 rows (f32, f32_stride) into three bf16 planes in the place of the two and does
+  // nothing else. Its first workgroup leaves in skip_out whether it was so.
+  uint32_t range_n;
+  void* y;
+  const float* bias;
+  const float* gate;  // gated residual: y = res + gate[col] * v (res may be y; NULL: none)
+  const void* res;
+  float scale;
+  uint32_t y_stride, y_offset;
+  uint32_t flags, y_dtype;
+  uint32_t vec_store;  // 1: y rows and y_offset allow 4-value vector stores
+  uint32_t store16;    // 1: y, y_offset and y rows are 16-byte aligned (whole-row staging of 16-bit outputs)
+  uint32_t mul;        // product epilogue with res (GemmLaunch::mul), 0: none
   // f32 operands as two f16 planes (split_f32_f16x2_kernel): the sums of row r times row_scale[r] (convolution: of column
   // c times row_scale[0] and col_scale[c]), the powers of two that the planes were scaled by. NULL: none
   const float* row_scale;
   const float* col_scale;
+  // fp8 weights for f16 x: the powers of two that the weights below k = kwrap and from there on are converted with. Two
+  // planes: 2^-5 with the lo plane, which carries 2^12, and 2^7 with the hi plane, all normal f16 values; else 1 and 1
+  float cvt_lo, cvt_hi;
+  const uint32_t* range;
+  uint32_t* skip_out;
+  const float* f32;
+  uint32_t f32_stride, range_most;
+  // int4 weights (w: u32 [N, K / 8], rows contiguous): f16 scales [N, sc_groups], one per sc_blocks 64-k blocks
+  const uint16_t* sc;
+  uint32_t sc_groups, sc_blocks;
   // 3x3 convolution input (CONV kernels): x holds an f16 image [m / conv_width, conv_width, 2 conv_cin], the lo and hi
   // plane of each pixel; k runs over segments of conv_kp (9 conv_cin rounded up to 64; tap, channel), the first with
   // the lo plane, the others with the hi plane. conv_magic = ceil(2^32 / conv_cin)
   uint32_t conv_width, conv_cin, conv_kp, conv_magic;
   uint32_t conv_hi;  // the k of the last segment: the sums before it, of products with a lo plane, are 2^12 times too large
-  // Launches that decide on the device whether they run. skip_if: CONV kernels and reduce passes do nothing where this word
-  // is not 0 (NULL: they run); only_if: fp8 kernels for bf16 x and reduce passes do nothing where it is 0 (NULL: they run).
-  // range_n > 0 (two f16 planes): the tiny values that split_f32_f16x2_kernel counted, by workgroup; more than range_most
-  // of them and the kernel splits the f32 rows (f32, f32_stride) into three bf16 planes in the place of the two and does
-  // nothing else. Its first workgroup leaves in skip_out whether it was so.
-  const uint32_t* skip_if;
-  const uint32_t* only_if;
-  const uint32_t* range;
-  uint32_t range_n, range_most;
-  uint32_t* skip_out;
-  const float* f32;
-  uint32_t f32_stride;
-  // fp8 weights for f16 x: the powers of two that the weights below k = kwrap and from there on are converted with. Two
-  // planes: 2^-5 with the lo plane, which carries 2^12, and 2^7 with the hi plane, all normal f16 values; else 1 and 1
-  float cvt_lo, cvt_hi;
-  // A split last round (tail_tiles > 0; GemmReducePlan::tail_splits): the tiles from tail_first on, a multiple of the CUs,
-  // run as tail_splits K slices of tail_kc each, whose raw sums go to part as dense tiles, slice-major
-  uint32_t tail_first, tail_tiles, tail_splits, tail_kc;
-  uint32_t mul;  // product epilogue with res (GemmLaunch::mul), 0: none
   // fused per-head RMSNorm + RoPE of the q / k columns (GemmLaunch::qk_*), qk_cols 0: none
   uint32_t qk_cols, q_cols, qk_rope_from;
   float qk_eps, qk_offset;
@@ -106,8 +115,7 @@ struct FastArgs {
   const float* qk_norm_k;
   const float* qk_cos;
   const float* qk_sin;
-  // A second GEMM in the same launch (gemm_fast_launch_pair): the same N, K, types, flags and product epilogue,
-  // operands of its own. Tiles from grp_first on (after the XCD renumbering) compute it; grp_first 0: none.
+  // the second GEMM of the launch: the same N, K, types, flags and product epilogue, operands of its own
   struct Second {
     const void* x;
     const void* w;
@@ -118,8 +126,8 @@ struct FastArgs {
     uint32_t x_bytes, w_bytes, m, x_stride, w_stride, y_stride, y_offset, tiles_m, vec_store, store16;
     float scale;
   } g;
-  uint32_t grp, grp_first;
 };
+static_assert(offsetof(FastArgs, y) == 120 && offsetof(FastArgs, row_scale) == 184, "the order above");
 
 namespace {
 
@@ -244,8 +252,8 @@ __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64) gemm_lds_kernel(FastArg
   // 243 -> 279 us, 2, each group its own share in its compute phase: 247 -> 291 us, up-projection, same box).
   // Other tiles: every wave loads its share in the memory phase.
   constexpr int LM = PP ? (B8 ? 0 : 1) : 0;
-  // Loads as inline asm (file comment): the int4 tiles and the small ones
-  constexpr bool DMA_ASM = B4 || BM <= 64;
+  // Loads as inline asm (file comment): the int4 tiles and the small ones of fp8 weights
+  constexpr bool DMA_ASM = B4 || (B8 && BM <= 64);
   constexpr int NL = LM == 1 ? NW / 2 : NW;                               // waves that issue loads
   static_assert(A_INS % NL == 0 && B_INS % NL == 0, "stage loads split evenly over the loading waves");
   constexpr int A_PW = A_INS / NL, B_PW = B_INS / NL, L = A_PW + B_PW;  // loads per loading wave per stage
@@ -282,8 +290,6 @@ __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64) gemm_lds_kernel(FastArg
         return;
       }
     }
-  } else if constexpr (B8) {
-    if (a.only_if && *a.only_if == 0) return;
   }
 
   uint32_t pid, z = blockIdx.y, kc = a.kc;
@@ -506,6 +512,10 @@ __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64) gemm_lds_kernel(FastArg
   auto block_wscale = [&](uint32_t kb) {
     if constexpr (B8 && IS_F16) wscale = kb < a.kwrap ? a.cvt_lo : a.cvt_hi;
   };
+
+  // (here and not at the top, where the branch would hold back the loads of the arguments behind it: 0.3 us per call)
+  if constexpr (B8 && !IS_F16)
+    if (a.only_if && *a.only_if == 0) return;
 
   u32x4 xf[2][TM];           // x fragments, double-buffered over steps
   u32x4 wr[2][TN];           // fp8: raw 16-B chunks (t = 0, 1); 16-bit: fragments double-buffered over steps
@@ -1199,9 +1209,11 @@ __device__ __forceinline__ void reduce_epilogue(const FastArgs& a, uint32_t row,
 // XCD (BM, BN > 0): the slices of a tile ran on one XCD (workgroups go round-robin over the 8 XCDs, and the slice
 // index adds a multiple of 8 tiles to the workgroup id), so each reduce workgroup takes a part of a tile of its own
 // XCD and reads the slices there. Otherwise one thread per 4 consecutive outputs in row-major order.
-template <int YT, int BM = 0, int BN = 0>
+// GUARD: of a launch that decides on the device whether it runs.
+template <int YT, int BM, int BN, bool GUARD>
 __global__ void __launch_bounds__(256) splitk_reduce_kernel(FastArgs a) {
-  if ((a.skip_if && *a.skip_if) || (a.only_if && !*a.only_if)) return;
+  if constexpr (GUARD)
+    if ((a.skip_if && *a.skip_if) || (a.only_if && !*a.only_if)) return;
   uint32_t row, c0;
   if constexpr (BM > 0) {
     constexpr uint32_t ITEMS = BM * BN / 4, Q = ITEMS / 256;  // reduce workgroups per tile
@@ -1248,9 +1260,10 @@ __global__ void __launch_bounds__(256) splitk_reduce_kernel(FastArgs a) {
 }
 
 // The reduce pass of a split last round: one thread per 4 consecutive outputs of a tail tile, slices in slice order.
-template <int YT, int BM, int BN>
+template <int YT, int BM, int BN, bool GUARD>
 __global__ void __launch_bounds__(256) tail_reduce_kernel(FastArgs a) {
-  if ((a.skip_if && *a.skip_if) || (a.only_if && !*a.only_if)) return;
+  if constexpr (GUARD)
+    if ((a.skip_if && *a.skip_if) || (a.only_if && !*a.only_if)) return;
   constexpr uint32_t ITEMS = BM * BN / 4, Q = ITEMS / 256;  // workgroups per tile
   const uint32_t t = blockIdx.x / Q, i = (blockIdx.x % Q) * 256 + threadIdx.x;
   const uint32_t pid = a.tail_first + t;
@@ -1280,6 +1293,20 @@ __global__ void __launch_bounds__(256) tail_reduce_kernel(FastArgs a) {
 // out). `on` 0 (Tuning::gemm_reduce_xcd): never (measurements).
 inline bool reduce_in_l2(uint64_t tiles, uint64_t weight_bytes, int on) {
   return on && tiles % 8 == 0 && weight_bytes <= (16u << 20);
+}
+
+// f(y type, guard): of a reduce kernel
+template <class F>
+void by_y_and_guard(const FastArgs& a, F&& f) {
+  auto by_y = [&](auto guard) {
+    switch (a.y_dtype) {
+      case F32: f(std::integral_constant<int, F32>{}, guard); break;
+      case F16: f(std::integral_constant<int, F16>{}, guard); break;
+      default: f(std::integral_constant<int, BF16>{}, guard); break;
+    }
+  };
+  if (a.skip_if || a.only_if) by_y(std::true_type{});
+  else by_y(std::false_type{});
 }
 
 template <int BM, int BN, int WM, int WN, bool IS_F16, int BT, int S, bool PP = false, bool CONV = false>
@@ -1312,22 +1339,15 @@ static hipError_t launch_fast_cfg(FastArgs a, uint32_t splits, int reduce_xcd, h
     // 12288 (37.7 MB of weights) 19.5 -> 20.2 us, so only up to 16 MB of weights (2 MB per XCD).
     // reduce_xcd 0: the row-major mapping (measurements)
     static_assert((BM * BN / 4) % 256 == 0, "whole reduce workgroups per tile");
-    if (reduce_in_l2(tiles, a.w_bytes, reduce_xcd)) {
-      const dim3 rg(tiles * (BM * BN / 4 / 256));
-      switch (a.y_dtype) {
-        case F32: hipLaunchKernelGGL((splitk_reduce_kernel<F32, BM, BN>), rg, dim3(256), 0, s, a); break;
-        case F16: hipLaunchKernelGGL((splitk_reduce_kernel<F16, BM, BN>), rg, dim3(256), 0, s, a); break;
-        default: hipLaunchKernelGGL((splitk_reduce_kernel<BF16, BM, BN>), rg, dim3(256), 0, s, a); break;
-      }
-      return hipGetLastError();
-    }
+    const bool in_l2 = reduce_in_l2(tiles, a.w_bytes, reduce_xcd);
     const size_t threads = (size_t)a.m * ((a.n + 3) / 4);
-    const dim3 rg((unsigned)((threads + 255) / 256));
-    switch (a.y_dtype) {
-      case F32: hipLaunchKernelGGL(splitk_reduce_kernel<F32>, rg, dim3(256), 0, s, a); break;
-      case F16: hipLaunchKernelGGL(splitk_reduce_kernel<F16>, rg, dim3(256), 0, s, a); break;
-      default: hipLaunchKernelGGL(splitk_reduce_kernel<BF16>, rg, dim3(256), 0, s, a); break;
-    }
+    const dim3 rg(in_l2 ? tiles * (BM * BN / 4 / 256) : (unsigned)((threads + 255) / 256));
+    by_y_and_guard(a, [&](auto YT, auto GUARD) {
+      constexpr int yt = decltype(YT)::value;
+      constexpr bool guard = decltype(GUARD)::value;
+      if (in_l2) hipLaunchKernelGGL((splitk_reduce_kernel<yt, BM, BN, guard>), rg, dim3(256), 0, s, a);
+      else hipLaunchKernelGGL((splitk_reduce_kernel<yt, 0, 0, guard>), rg, dim3(256), 0, s, a);
+    });
     return hipGetLastError();
   }
   switch (a.y_dtype) {
@@ -1339,11 +1359,9 @@ static hipError_t launch_fast_cfg(FastArgs a, uint32_t splits, int reduce_xcd, h
     const hipError_t err = hipGetLastError();
     if (err != hipSuccess) return err;
     const dim3 rg(a.tail_tiles * (BM * BN / 4 / 256));
-    switch (a.y_dtype) {
-      case F32: hipLaunchKernelGGL((tail_reduce_kernel<F32, BM, BN>), rg, dim3(256), 0, s, a); break;
-      case F16: hipLaunchKernelGGL((tail_reduce_kernel<F16, BM, BN>), rg, dim3(256), 0, s, a); break;
-      default: hipLaunchKernelGGL((tail_reduce_kernel<BF16, BM, BN>), rg, dim3(256), 0, s, a); break;
-    }
+    by_y_and_guard(a, [&](auto YT, auto GUARD) {
+      hipLaunchKernelGGL((tail_reduce_kernel<decltype(YT)::value, BM, BN, decltype(GUARD)::value>), rg, dim3(256), 0, s, a);
+    });
   }
   return hipGetLastError();
 }
