@@ -723,6 +723,23 @@ def test_conv3x3_planes(graph, tune, h, w, cin, cout, w_dt, y_dt, flags, cfg):
         assert O.rel_error(got.reshape(-1, cout)[:, 3], want.reshape(-1, cout)[:, 3]) < TOL[y_dt]
 
 
+@pytest.mark.parametrize("h,w,cin,cout,w_dt,small", [
+    (32, 32, 8, 32, we.F32, True), (32, 32, 16, 32, we.F32, False), (4, 4, 8, 32, we.BF16, True), (8, 8, 16, 32, we.BF16, True),
+    (16, 16, 8, 32, we.BF16, False), (2, 2, 48, 32, we.BF16, False)])
+def test_conv3x3_planes_leave_small_calls_to_the_general_kernel(graph, tune, h, w, cin, cout, w_dt, small):
+    """Calls whose K or image is too small to pay for the planes' launches are the general kernel's bit for bit; the others, on
+    both sides of the line, are another sum of the same products."""
+    rng = np.random.default_rng(h + cin)
+    x, wt = rng.standard_normal(h * w * cin).astype(np.float32), rng.standard_normal(cout * 9 * cin).astype(np.float32)
+    w_store = O.bf16_rne(wt) if w_dt == we.BF16 else wt
+    p = we.conv3x3_params(h, w, cin, cout, graph=graph)
+    got = run(graph, p, x, we.F32, w_store, w_dt, we.F32)
+    tune(gemm_generic=1)
+    general = run(graph, p, x, we.F32, w_store, w_dt, we.F32)
+    assert np.array_equal(got, general) == small
+    assert O.rel_error(got, general) < 4e-6
+
+
 def test_conv3x3_planes_leave_wide_images_to_the_general_kernel(graph, tune):
     """An image with pixels below 2^-16 of its largest value, which one scale cannot hold to f32's precision: the general
     kernel's result bit for bit. An inf poisons the pixels around it as there, and no others."""

@@ -63,6 +63,12 @@ bool make_plan(const GemmLaunch& L, Plan& p) {
   if ((uintptr_t)L.x % 16 || ((uintptr_t)L.w + (uint64_t)L.w_offset * wb) % 16 || ((uint64_t)L.w_stride * wb) % 16)
     return false;
   if (L.conv_cin > 4096) return false;  // the tap of a k (below 2^16) by one multiplication
+  // The four launches take about 15 us whatever the size; the general kernel's one is faster where K is short. f32 weights,
+  // 64 x 64 pixels -> 32 channels: from 8 channels 14.8 us there and 17.1 here, from 16 19.1 and 18.8. bf16 weights -> 32:
+  // 4 x 4 pixels of 8 channels 9.1 and 14.8, 8 x 8 of 16 13.7 and 15.8, 8 x 8 of 32 19.0 and 18.2, 16 x 16 of 8 21.9 and
+  // 15.3, 2 x 2 of 48 20.0 and 20.1. (A forced tile shape stays.)
+  const bool pays = L.w_dtype == F32 ? L.conv_cin >= 16 : L.conv_cin >= 48 || (uint64_t)L.m * L.conv_cin >= 2048;
+  if (L.cfg < 0 && !pays) return false;
   p.kp = (9 * L.conv_cin + BK - 1) / BK * BK;
   p.segments = L.w_dtype == F32 ? 3 : 2;
   const uint64_t image = (uint64_t)L.m * L.conv_cin * 4, weights = (uint64_t)L.n * p.kp * 2 * (p.segments - 1);
