@@ -197,7 +197,7 @@ def test_tiles_for_many_rows(graph, tune, m, n, k, group, x_dt, y_dt, flags):
     (2, 129, 700, 4096, 64, we.BF16), (2, 33, 12300, 1088, 1088, we.F16),  # slices; most of the tile's rows past M
     (2, 300, 2061, 1344, 192, we.F16), (3, 300, 2061, 1344, 192, we.BF16)])
 def test_both_tile_shapes(graph, tune, cfg, m, n, k, group, x_dt):
-    """The 128 x 128 tiles (gemm_cfg 2: two halves of a wave's rows, four scales per thread, two stages) and the 64 x 64 ones (3),
+    """The 128 x 128 tiles (gemm_cfg 2: four row blocks per wave, four scales per thread, two stages) and the 64 x 64 ones (3),
     with and without K slices, ragged in both directions: rows of every tile against the oracle, all of them against the GEMV
     kernels (the same exact products in another order), plain and with a gated residual."""
     rng = np.random.default_rng(m + n)

@@ -4,10 +4,10 @@
 // (src/kernels/matmul.ts:118-178).
 //
 // Structure (one workgroup per BM x BN output tile, 64 k per pipeline stage, S stages in LDS):
-//  * Operands move HBM -> LDS with direct-to-LDS buffer loads (buffer_load_dwordx4 ... lds; in the int4 tiles and those of
-//    at most 64 rows issued as inline asm: behind the builtin the compiler drains every load in flight before the next
-//    LDS read, once per 64-k block there (64 x 3072 x 3072 fp8 11.2 -> 11.0 us); the larger tiles ran 1-2% slower on the
-//    asm): each load
+//  * Operands move HBM -> LDS with direct-to-LDS buffer loads (buffer_load_dwordx4 ... lds; in the int4 tiles and the
+//    fp8 ones of at most 64 rows issued as inline asm: behind the builtin the compiler drains every load in flight before
+//    the next LDS read, once per 64-k block there (64 x 3072 x 3072 fp8 11.2 -> 11.0 us); the larger tiles ran 1-2%
+//    slower on the asm, small ones of 16-bit weights 3-5% (16 x 12288 x 3072 24.0 us against 23.4)): each load
 //    instruction of a wave fills 1 KB of LDS (lane i writes bytes [16 i, 16 i + 16)), no VGPR staging.
 //    The source address of each lane is chosen so that the LDS image is XOR-swizzled: 16-byte chunk c of
 //    row r sits at chunk position c ^ swz(r), which makes the MFMA fragment reads bank-conflict free.
@@ -29,9 +29,10 @@
 // Requirements (checked on the host): x / W rows 16-byte aligned, K and the split-K slice multiples of
 // 16, operand extents below 2^31 bytes.
 // f32 activations arrive as 16-bit planes along K (split by a pass before the GEMM): two f16 planes with a scale per row
-// (x [M, 2K], fp8 weights) or three exact bf16 planes (x [M, 3K], bf16 weights). The kernel walks k over all planes while
-// the weights are read at k mod K (K a multiple of 64, so no 64-k block spans two planes), so every epilogue applies to the
-// whole sum. The CONV kernels read x as an f16 image and gather each tap's pixels by the loads' addresses (gemm_conv.hip).
+// (x [M, 2K], large products with fp8 weights whose rows the planes hold) or three exact bf16 planes (x [M, 3K]). The kernel
+// walks k over all planes while the weights are read at k mod K (K a multiple of 64, so no 64-k block spans two planes), so
+// every epilogue applies to the whole sum. The CONV kernels read x as an f16 image and gather each tap's pixels by the loads'
+// addresses (gemm_conv.hip).
 #pragma once
 #include <cstddef>
 
@@ -663,10 +664,9 @@ __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64) gemm_lds_kernel(FastArg
       }
     }
   } else if constexpr (B4) {
-    // ---- int4. A block's sums of x q go to `part` and, times the block's scales, from there into acc. Tiles of 4 row
-    // blocks per wave run the block as two halves of 2 (H), each with its own MFMAs and scaling: half the part registers,
-    // so three workgroups fit a CU, and one half's scaling runs beside the other's MFMAs.
-    constexpr int H = TM >= 4 ? 2 : 1, TH = TM / H;
+    // ---- int4. A block's sums of x q go to `part` and, times the block's scales, from there into acc. (Tiles of 4 row
+    // blocks per wave as two halves, each with its own MFMAs and scaling and half the part registers: 509 x 18944 x 3584 f16
+    // 134.3 us against 125.9, 1024 x 3584 x 18944 232 against 220.)
     if (nk > 0) {
 #pragma unroll
       for (int p = 0; p < S; p++)
@@ -676,18 +676,17 @@ __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64) gemm_lds_kernel(FastArg
       if (nk >= S) wait_vmcnt<(S - 1) * L>();
       else wait_vmcnt<0>();
       lds_barrier();
-      u32x4 xh[2][TH];  // x fragments of a step (half u / 4, step u % 4), double-buffered
+      u32x4 xh[2][TM];  // x fragments of a step, double-buffered
       u32x4 wq[TN];     // the block's words
-      auto read_half = [&](uint32_t st_off, auto U, u32x4 (&d)[TH]) {
-        constexpr int hf = decltype(U)::value / 4, s = decltype(U)::value % 4;
+      auto read_step = [&](uint32_t st_off, int s, u32x4 (&d)[TM]) {
 #pragma unroll
-        for (int i = 0; i < TH; i++) d[i] = rd(st_off + (rda[0] ^ (s * 16)) + (hf * TH + i) * 32 * 128);
+        for (int i = 0; i < TM; i++) d[i] = rd(st_off + (rda[0] ^ (s * 16)) + i * 32 * 128);
       };
       auto read_words = [&](uint32_t st_off) {
 #pragma unroll
         for (int j = 0; j < TN; j++) wq[j] = rd(st_off + rdb[0] + j * 32 * B_ROW);
       };
-      read_half(0, std::integral_constant<int, 0>{}, xh[0]);
+      read_step(0, 0, xh[0]);
       read_words(0);
       int cur = 0;
       for (int it = 0; it < nk; ++it) {
@@ -706,11 +705,11 @@ __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64) gemm_lds_kernel(FastArg
             if constexpr (IS_F16) wf[s][j] = int4x8_to_f16(wq[j][s], 0x00f0000fu);
             else wf[s][j] = int4x8_to_bf16(wq[j][s]);
           }
-        f32x16 part[TH][TN];
-        static_for<0, 4 * H>([&](auto U) {
-          constexpr int u = decltype(U)::value, hf = u / 4, s = u % 4;
-          if constexpr (u + 1 < 4 * H) {
-            read_half(cur_off, std::integral_constant<int, u + 1>{}, xh[(u + 1) & 1]);
+        f32x16 part[TM][TN];
+        static_for<0, 4>([&](auto SI) {
+          constexpr int s = decltype(SI)::value;
+          if constexpr (s < 3) {
+            read_step(cur_off, s + 1, xh[(s + 1) & 1]);
           } else {
             // every wave has its last fragments of this block; block it + 1 must be complete
             if (it + S - 1 < nk) wait_vmcnt<(S - 2) * L>();
@@ -718,15 +717,15 @@ __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64) gemm_lds_kernel(FastArg
             lds_barrier();
             if (it + S < nk) issue(k_begin + (uint32_t)(it + S) * BK, cur);
             if (it + 1 < nk) {
-              read_half(nxt_off, std::integral_constant<int, 0>{}, xh[0]);
+              read_step(nxt_off, 0, xh[0]);
               read_words(nxt_off);
             }
           }
 #pragma unroll
-          for (int i = 0; i < TH; i++)
+          for (int i = 0; i < TM; i++)
 #pragma unroll
             for (int j = 0; j < TN; j++)
-              part[i][j] = mfma_32x32x16<IS_F16>(wf[s][j], xh[u & 1][i], s == 0 ? f32x16{} : part[i][j]);
+              part[i][j] = mfma_32x32x16<IS_F16>(wf[s][j], xh[s & 1][i], s == 0 ? f32x16{} : part[i][j]);
           if constexpr (s == 3) {
 #pragma unroll
             for (int j = 0; j < TN; j++)
@@ -734,11 +733,10 @@ __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64) gemm_lds_kernel(FastArg
               for (int q = 0; q < 4; q++) {
                 const f32x4 sv = *(const f32x4*)(sp + j * 32 + 8 * q);
 #pragma unroll
-                for (int i = 0; i < TH; i++)
+                for (int i = 0; i < TM; i++)
 #pragma unroll
                   for (int e = 0; e < 4; e++)
-                    acc[hf * TH + i][j][4 * q + e] =
-                        __builtin_fmaf(part[i][j][4 * q + e], sv[e], acc[hf * TH + i][j][4 * q + e]);
+                    acc[i][j][4 * q + e] = __builtin_fmaf(part[i][j][4 * q + e], sv[e], acc[i][j][4 * q + e]);
               }
           }
         });

@@ -57,7 +57,7 @@ struct GemmLaunch {
   const float* qk_norm_k;
   const float* qk_cos;
   const float* qk_sin;
-  // 3x3 convolution input (conv_width > 0, the general kernel only): x is a channel-last image
+  // 3x3 convolution input (conv_width > 0; the general kernel and conv_fast_launch): x is a channel-last image
   // [m / conv_width, conv_width, conv_cin] and k runs over (tap, channel), K = 9 * conv_cin
   uint32_t conv_width, conv_cin;
   const uint32_t* only_if;  // general kernel, fast kernel for fp8 weights and bf16 x: a device word, 0: the launch does nothing
@@ -138,7 +138,8 @@ struct Int4Launch {
   uint32_t rsplits, rkc;
   void* scratch;
 };
-// M > 16, 16-bit x: tiles of gemm_lds.h that share each weight read over 32 to 128 rows (gemm_int4.hip)
+// M > 32 and a large weight matrix, 16-bit x: tiles of gemm_lds.h that share each weight read over 64 or 128 rows
+// (gemm_int4.hip)
 bool int4_gemm_supported(const Int4Launch& L);
 GemmReducePlan int4_gemm_plan(const Int4Launch& L);
 hipError_t int4_gemm_launch(const Int4Launch& L, hipStream_t stream);
