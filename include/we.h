@@ -312,7 +312,7 @@ int we_qk_norm_rope(we_ctx* ctx, uint32_t tokens, uint32_t heads, uint32_t head_
  * t * q_stride elements (0 = heads * dim; k and v: 0 = kv_heads * dim; out: 0 = heads * dim), so q, k and v
  * may be slices of one fused QKV row. dtype F32 (head dim 128 from 160 tokens on, 64 from 320 on: two f16 planes per
  * operand with powers of two per channel of K and V and per row of Q, which hold a value to 2^-21 of itself down to 2^-18
- * of the largest of its channel or row; kv heads and blocks of 128 queries in which more than a few values lie further
+ * of the largest of its channel or row; kv heads and blocks of 32 queries in which more than a few values lie further
  * below, or that hold an inf or NaN, run on the f32 MFMA; else exact f32 products), BF16 or F16 (fp32 scores, softmax and
  * accumulation; probabilities rounded to the operand type). dim: a multiple of 8 (F32: 4), at most 128.
  * The reference's `chunk` only bounds its score buffer; no score matrix exists here, so it has no analogue. */

@@ -57,7 +57,7 @@ struct AttnArgs {
   int causal;
   // f32 through f16 planes (attn_planes_kernel), NULL: no planes. plane_inv: the inverse scales of K's channels
   // [kv_heads, dim], then V's. What the planes cannot hold goes to the f32 MFMA kernel: plane_head[g] != 0, kv head g
-  // with its queries; plane_rows[h * (blocks of 128 queries) + block] != 0, that block of head h
+  // with its queries; plane_rows[h * (blocks of 32 queries) + block] != 0, that block of head h (one wave's)
   const float* plane_inv;
   uint32_t* plane_head;
   uint32_t* plane_rows;
@@ -1036,9 +1036,19 @@ __global__ void __launch_bounds__(ATT_NT, 1) attn32_kernel(AttnArgs a) {
   uint32_t qb, h;
   block_coords(a, qb, h);
   const uint32_t g = h / a.group;
-  if (a.plane_head && !a.plane_head[g] && !a.plane_rows[h * a.nqb + qb]) return;  // attn_planes_kernel has these queries
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  bool store = true;  // this wave's queries are this kernel's, not attn_planes_kernel's
+  if (a.plane_head && !a.plane_head[g]) {
+    const uint32_t nb = (a.tokens + 31) / 32, b0 = qb * (ATT_BM / 32);
+    uint32_t any = 0;
+    for (uint32_t i = 0; i < ATT_BM / 32 && b0 + i < nb; i++) {
+      const uint32_t rows = a.plane_rows[h * nb + b0 + i];
+      any |= rows;
+      if ((int)i == wave) store = rows != 0;
+    }
+    if (!any) return;
+  }
   const int c = lane & 31, hf = lane >> 5;
   const uint32_t q0 = qb * ATT_BM;
   const uint32_t qw = q0 + 32 * wave;
@@ -1133,7 +1143,7 @@ __global__ void __launch_bounds__(ATT_NT, 1) attn32_kernel(AttnArgs a) {
   }
 
   const float inv = 1.0f / halves_sum(l);
-  if (qi < a.tokens) {
+  if (qi < a.tokens && store) {
     float* O = (float*)a.o + (size_t)qi * a.os + (size_t)h * a.dim;
     static_for<0, DP / 32>([&](auto D) {
       constexpr int db = D;
@@ -1159,7 +1169,7 @@ __global__ void __launch_bounds__(ATT_NT, 1) attn32_kernel(AttnArgs a) {
 // at once, computes
 //  * kv heads with more than 2 + tokens / 256 of them in a channel, with a token whose values all lie below 2^-16 of their
 //    channels' largest, with an inf or NaN, or with a K value of 2^96 or more (its inverse scale could take Q out of range),
-//  * blocks of 128 queries with a Q row that holds more than 2, or more than one to 32 others.
+//  * blocks of 32 queries with a Q row that holds more than 2, or more than one to 32 others.
 // With fewer tokens than PLANES_MIN_TOKENS (head dim 64: than twice that) the two passes over K and V and the third launch
 // cost what the products gain: 24 heads of 128, 128 tokens 23.7 us here and 24.4 us on the f32 MFMA; 16 heads, 64 tokens
 // 17.0 and 13.1, 200 tokens causal 27.1 and 41.8; head dim 64, 170 tokens causal 5% less time at an error of 2.3e-7 for 2.2e-7.
@@ -1319,22 +1329,26 @@ __global__ void __launch_bounds__(64 * NW, 1) attn_planes_kernel(AttnArgs a, con
   // Q planes: query qi, dims 16 s + 8 hf .. + 7, times K's inverse scales, scaled by the row's own power of two
   u32x4 qh[DP / 16], ql[DP / 16];
   float sc;  // scores -> log2 units
+  bool wide = false;  // the f32 MFMA kernel's queries: this wave stores nothing
   {
     float v[DP / 16][8];
-    uint32_t m = 0, tiny = 0, others = 0;
+    uint32_t m = 0, low = 0xffffffffu;  // low: the smallest nonzero |value|, as twice its bits less 1 (0: the largest)
+    // all loads before the first product (rows past the last: that one's values, not stored)
     const float* kinv = a.plane_inv + g * DP + 8 * hf;
-    static_for<0, DP / 16>([&](auto S) {
-      const float* p = (const float*)a.q + (size_t)qi * a.qs + (size_t)h * DP + 16 * S + 8 * hf;
-      f32x4 v0 = {0, 0, 0, 0}, v1 = {0, 0, 0, 0};
-      if (qi < a.tokens) v0 = *(const f32x4*)p, v1 = *(const f32x4*)(p + 4);
-      v0 *= *(const f32x4*)(kinv + 16 * S);
-      v1 *= *(const f32x4*)(kinv + 16 * S + 4);
+    const float* q = (const float*)a.q + (size_t)min(qi, a.tokens - 1u) * a.qs + (size_t)h * DP + 8 * hf;
+    f32x4 qv[DP / 8], kv[DP / 8];
+    static_for<0, DP / 8>([&](auto I) {
+      qv[I] = *(const f32x4*)(q + 16 * (I / 2) + 4 * (I % 2));
+      kv[I] = *(const f32x4*)(kinv + 16 * (I / 2) + 4 * (I % 2));
+    });
+    __builtin_amdgcn_sched_barrier(0);
+    static_for<0, DP / 8>([&](auto I) {
       static_for<0, 4>([&](auto E) {
-        constexpr int e = E;
-        v[S][e] = v0[e];
-        v[S][4 + e] = v1[e];
-        const uint32_t b0 = __float_as_uint(v0[e]) & 0x7fffffffu, b1 = __float_as_uint(v1[e]) & 0x7fffffffu;
-        m = max(m, max(b0 < 0x7f800000u ? b0 : 0u, b1 < 0x7f800000u ? b1 : 0u));
+        constexpr int i = I, e = E;
+        const float x = qv[i][e] * kv[i][e];
+        v[i / 2][4 * (i % 2) + e] = x;
+        const uint32_t b = __float_as_uint(x) & 0x7fffffffu;
+        m = max(m, b < 0x7f800000u ? b : 0u);
       });
     });
     m = max(m, (uint32_t)__shfl_xor((int)m, 32, 64));
@@ -1343,21 +1357,24 @@ __global__ void __launch_bounds__(64 * NW, 1) attn_planes_kernel(AttnArgs a, con
     static_for<0, DP / 16>([&](auto S) {
       static_for<0, 8>([&](auto E) {
         v[S][E] *= s;
-        const uint32_t b = __float_as_uint(v[S][E]) & 0x7fffffffu;
-        tiny += b && b < PLANE_TINY ? 1u : 0u;
-        others += b >= PLANE_TINY ? 1u : 0u;
+        low = min(low, (__float_as_uint(v[S][E]) << 1) - 1u);
       });
       attn_split8(v[S], qh[S], ql[S]);
     });
-    tiny += (uint32_t)__shfl_xor((int)tiny, 32, 64);
-    others += (uint32_t)__shfl_xor((int)others, 32, 64);
-    const int wide = __syncthreads_or(qi < a.tokens && (tiny > 2u || 32u * tiny > others));
-    const uint32_t nb = (a.tokens + ATT_BM - 1) / ATT_BM, b0 = q0 / ATT_BM;  // blocks of the f32 MFMA kernel
-    if (tid < NW / 4 && b0 + tid < nb) a.plane_rows[h * nb + b0 + tid] = wide ? 1u : 0u;
-    if (wide) {
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the first tile's loads write LDS
-      return;
+    if (__any(low < 2 * PLANE_TINY - 1)) {  // rarely: count
+      uint32_t tiny = 0, others = 0;
+      static_for<0, DP / 16>([&](auto S) {
+        static_for<0, 8>([&](auto E) {
+          const uint32_t b = __float_as_uint(v[S][E]) & 0x7fffffffu;
+          tiny += b && b < PLANE_TINY ? 1u : 0u;
+          others += b >= PLANE_TINY ? 1u : 0u;
+        });
+      });
+      tiny += (uint32_t)__shfl_xor((int)tiny, 32, 64);
+      others += (uint32_t)__shfl_xor((int)others, 32, 64);
+      wide = __any(qi < a.tokens && (tiny > 2u || 32u * tiny > others));
     }
+    if (lane == 0 && qw < a.tokens) a.plane_rows[h * ((a.tokens + 31) / 32) + qw / 32] = wide ? 1u : 0u;
     // a normal, finite factor: a masked score is -inf times it, and 0 (tiny or zero Q rows) would make that a NaN. Where
     // the scale leaves the range, scores round to 0 with the clamped one too.
     sc = fminf(fmaxf(a.scale_log2 * __uint_as_float((254u - se) << 23), 1.17549435e-38f), 3.40282347e38f);
@@ -1466,15 +1483,17 @@ __global__ void __launch_bounds__(64 * NW, 1) attn_planes_kernel(AttnArgs a, con
   }
 
   const float inv = 1.0f / halves_sum(l);
-  if (qi < a.tokens) {
+  if (qi < a.tokens && !wide) {
     const float* vinv = a.plane_inv + (a.kv_heads + g) * DP + 4 * hf;
+    f32x4 iv[DP / 8];
+    static_for<0, DP / 8>([&](auto I) { iv[I] = *(const f32x4*)(vinv + 8 * I); });
     float* O = (float*)a.o + (size_t)qi * a.os + (size_t)h * DP;
     static_for<0, DP / 32>([&](auto D) {
       constexpr int db = D;
       static_for<0, 4>([&](auto G) {
         constexpr int g4 = G;
         const f32x4 r = f32x4{o[db][4 * g4], o[db][4 * g4 + 1], o[db][4 * g4 + 2], o[db][4 * g4 + 3]} * inv;
-        *(f32x4*)(O + 32 * db + 8 * g4 + 4 * hf) = r * *(const f32x4*)(vinv + 32 * db + 8 * g4);
+        *(f32x4*)(O + 32 * db + 8 * g4 + 4 * hf) = r * iv[4 * db + g4];
       });
     });
   }
@@ -1516,7 +1535,7 @@ bool attn_planes_ok(const AttnLaunch& L, PlanesLayout& p) {
   p.inv = p.count + words;
   p.head = p.inv + words;
   p.rows = p.head + ((size_t)L.kv_heads * 4 + 255) / 256 * 256;
-  p.bytes = p.rows + (size_t)((L.tokens + ATT_BM - 1) / ATT_BM) * L.heads * 4;
+  p.bytes = p.rows + (size_t)((L.tokens + 31) / 32) * L.heads * 4;
   return true;
 }
 

@@ -84,13 +84,16 @@ __device__ __forceinline__ uint32_t block_sum256(uint32_t v, uint32_t* red) {
   __syncthreads();
   return red[0] + red[1] + red[2] + red[3];
 }
-// The planes of 8 values times s; counts the tiny ones.
-__device__ __forceinline__ void split_f16x2(const float (&v)[8], float s, u32x4& lo, u32x4& hi, uint32_t& tiny) {
+// Twice the bits of |v| less 1: the order of the magnitudes, with 0 as the largest.
+__device__ __forceinline__ uint32_t low_key(float v) { return (__float_as_uint(v) << 1) - 1u; }
+constexpr uint32_t kPlaneTinyKey = 2 * kPlaneTiny - 1;  // tiny: a smaller key
+
+// The planes of 8 values times s, and the smallest key of those.
+__device__ __forceinline__ void split_f16x2(const float (&v)[8], float s, u32x4& lo, u32x4& hi, uint32_t& low) {
 #pragma unroll
   for (int i = 0; i < 4; i++) {
     const float a = v[2 * i] * s, b = v[2 * i + 1] * s;
-    const uint32_t ba = __float_as_uint(a) & 0x7fffffffu, bb = __float_as_uint(b) & 0x7fffffffu;
-    tiny += (ba && ba < kPlaneTiny ? 1u : 0u) + (bb && bb < kPlaneTiny ? 1u : 0u);
+    low = min(low, min(low_key(a), low_key(b)));
     const uint32_t ha = f32_to_f16(a), hb = f32_to_f16(b);
     hi[i] = ha | (hb << 16);
     lo[i] = (uint32_t)f32_to_f16((a - f16_to_f32((uint16_t)ha)) * kPlaneLo) |
@@ -112,15 +115,12 @@ __global__ void __launch_bounds__(256) split_f32_f16x2_kernel(const void* __rest
   uint32_t total = 0;
   for (size_t row = blockIdx.x; row < m; row += gridDim.x) {
     const size_t base = row * stride;
-    uint32_t mx = 0, tiny = 0, nonzero = 0;
+    uint32_t mx = 0, low = 0xffffffffu;
     for (uint32_t i = threadIdx.x * 8; i < k; i += 2048) {
       float v[8];
       load8<DT>(src, base + i, v);
 #pragma unroll
-      for (int e = 0; e < 8; e++) {
-        mx = max(mx, finite_bits(v[e]));
-        nonzero += v[e] != 0.0f ? 1u : 0u;
-      }
+      for (int e = 0; e < 8; e++) mx = max(mx, finite_bits(v[e]));
     }
     const uint32_t se = plane_scale_exp(block_max256(mx, red));
     const float s = __uint_as_float(se << 23);
@@ -130,11 +130,21 @@ __global__ void __launch_bounds__(256) split_f32_f16x2_kernel(const void* __rest
       float v[8] = {};
       if (i < k) load8<DT>(src, base + i, v);
       u32x4 lo, hi;
-      split_f16x2(v, s, lo, hi, tiny);
+      split_f16x2(v, s, lo, hi, low);
       *(u32x4*)(dst + (size_t)hi_at * kp + i) = hi;
       if (lo_at >= 0) *(u32x4*)(dst + (size_t)lo_at * kp + i) = lo;
     }
-    if (__syncthreads_or(tiny != 0)) {  // also before the next row's maxima
+    if (__syncthreads_or(low < kPlaneTinyKey)) {  // rarely: count (the barrier stands before the next row's maxima, too)
+      uint32_t tiny = 0, nonzero = 0;
+      for (uint32_t i = threadIdx.x * 8; i < k; i += 2048) {
+        float v[8];
+        load8<DT>(src, base + i, v);
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+          tiny += low_key(v[e] * s) < kPlaneTinyKey ? 1u : 0u;
+          nonzero += v[e] != 0.0f ? 1u : 0u;
+        }
+      }
       const uint32_t t = block_sum256(tiny, red2), n = block_sum256(nonzero, red3);
       total = 64u * t > n - t ? most + 1 : min(total + t, most + 1);
       __syncthreads();
@@ -193,17 +203,20 @@ __global__ void __launch_bounds__(256) image_f16x2_kernel(const float* __restric
   const float s = __uint_as_float(se << 23);
   if (blockIdx.x == 0 && t == 0) *inv = __uint_as_float((254u - se) << 23);
   const size_t i = ((size_t)blockIdx.x * 256 + t) * 8;
-  uint32_t tiny = 0;
+  uint32_t low = 0xffffffffu;
+  float v[8] = {};
   if (i < n) {
-    float v[8];
     load8<F32>(x, i, v);
     u32x4 lo, hi;
-    split_f16x2(v, s, lo, hi, tiny);
+    split_f16x2(v, s, lo, hi, low);
     uint16_t* dst = out + i / cin * 2 * cin + i % cin;
     *(u32x4*)dst = lo;
     *(u32x4*)(dst + cin) = hi;
   }
-  if (__syncthreads_or(tiny != 0)) {
+  if (__syncthreads_or(low < kPlaneTinyKey)) {
+    uint32_t tiny = 0;
+#pragma unroll
+    for (int e = 0; e < 8; e++) tiny += low_key(v[e] * s) < kPlaneTinyKey ? 1u : 0u;
     const uint32_t count = block_sum256(tiny, red2);
     const uint32_t nonzero = block_sum256(part[kImageParts + t] + part[kImageParts + 256 + t], red3);
     if (t == 0 && atomicAdd(range + 2, count) + count > min(8u + (uint32_t)(n >> 20), nonzero / 64u)) atomicOr(range, 1u);
