@@ -210,10 +210,12 @@ int we_conv3x3_params(we_ctx* ctx, uint32_t height, uint32_t width, uint32_t cin
 int we_matmul(we_ctx* ctx, const we_matmul_params* p, int x_dtype, const void* x, int w_dtype, const void* w,
               const void* w_scales, uint32_t group, int y_dtype, void* y, const float* bias, uint32_t flags);
 /* we_matmul that allocates nothing. No counterpart in the reference: for callers that cannot allocate device memory
- * (code under HIP graph capture, tight serving or decode loops, harnesses that forbid hipMalloc). Same arguments,
- * kernels and results as we_matmul; the split-K partial sums that small-M GEMMs (M <= 64, and larger M with few
+ * (code under HIP graph capture, tight serving or decode loops, harnesses that forbid hipMalloc). Same arguments and
+ * kernels as we_matmul; the split-K partial sums that small-M GEMMs (M <= 64, and larger M with few
  * output tiles) keep in scratch go to a fixed per-GPU device array of 16 MiB instead of the context's scratch,
- * which holds every M <= 64 shape. A GEMM whose split plan needs more fails with WE_EINVAL, "... needs <n> bytes of
+ * which holds every M <= 64 shape. Results equal we_matmul's bit for bit but where that uses scratch the array cannot
+ * hold: M > 64 planned in K slices of more than 16 MiB, int4 weights for many rows likewise, f32 x (whose planes need
+ * scratch) and the 3x3 convolution of f32 images run without it and sum in another order. A GEMM whose split plan needs more fails with WE_EINVAL, "... needs <n> bytes of
  * split-K scratch; the allocation-free entry point has 16777216 (use we_matmul)". Every call on one GPU shares that
  * GPU's array, so calls that could overlap are refused rather than raced: the array belongs to the first live
  * context that calls this on the GPU until that context is destroyed (another context's call fails with WE_EINVAL),

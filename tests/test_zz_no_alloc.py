@@ -63,6 +63,25 @@ def test_noalloc_equals_we_matmul_on_two_calls_in_a_row(graph):
         assert O.rel_error(_decode(got, y_dt), want) < tol, (m, n, k)
 
 
+@pytest.mark.parametrize("m,n,k,same", [(300, 1028, 1024, True), (520, 260, 3072, True), (700, 9216, 1024, True),
+                                         (1100, 4096, 4096, False)])
+def test_noalloc_takes_the_plan_that_fits(graph, m, n, k, same):
+    """M > 64: the tile plan of we_matmul, bit for bit, where its partial sums fit the array (64 x 64 tiles in K slices, tiles
+    without slices); one that does not fit (256 x 256 in 3 slices, 54 MB) runs in whole K instead of being
+    refused, and sums in another order."""
+    rng = np.random.default_rng(m)
+    x, _, w = _operands(rng, m, n, k, we.BF16)
+    p = we.matmul_params(m, n, k, 0.02, graph=graph)
+    mark = graph.mark()
+    xb, wb, y_ref, y_na = graph.buffer(x), graph.buffer(w), graph.buffer(m * n * 4), graph.buffer(m * n * 4)
+    graph.matmul(p, we.BF16, xb, we.FP8, wb, we.F32, y_ref)
+    graph.matmul_noalloc(p, we.BF16, xb, we.FP8, wb, we.F32, y_na)
+    ref, got = graph.read(y_ref), graph.read(y_na)
+    graph.release(mark)
+    assert np.array_equal(got, ref) == same
+    assert O.rel_error(_decode(got, we.F32), _decode(ref, we.F32)) < 4e-6
+
+
 def test_noalloc_replays_under_graph_capture(graph):
     """Captured in a HIP graph (where no allocation may happen) and replayed over new inputs: every replay equals
     we_matmul run eagerly on the same inputs."""

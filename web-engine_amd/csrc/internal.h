@@ -105,8 +105,8 @@ struct GemmReducePlan {
 };
 GemmReducePlan gemm_reduce_plan(const GemmLaunch& L, uint32_t force_splits = 0);  // force_splits: sweeps
 // The tile shape and K slices by predicted time (M > 64); gemm_reduce_plan below that and with a forced tile shape. The
-// allocation-free entry point keeps gemm_reduce_plan, which says what it accepts, and so does a launch whose planned
-// scratch is not to be had.
+// allocation-free entry point accepts what gemm_reduce_plan fits its array with, and runs that where this plan does not fit;
+// so does a launch whose planned scratch is not to be had.
 GemmReducePlan gemm_plan(const GemmLaunch& L);
 // The straight-line fast path; hipErrorNotSupported when the operands do not qualify.
 hipError_t gemm_fast_launch(const GemmLaunch& L, hipStream_t stream);

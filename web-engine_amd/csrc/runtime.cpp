@@ -1115,7 +1115,10 @@ int matmul_impl(we_ctx* ctx, const we_matmul_params* p, int x_dtype, const void*
   auto plan_of = [&](const we::GemmLaunch& G) {
     if (ctx->tune.gemm_splitk > 0) return we::gemm_reduce_plan(G, (uint32_t)ctx->tune.gemm_splitk);
     if (ctx->tune.gemm_splitk == 0) return we::GemmReducePlan{1, G.k, 0, -1, 1};
-    return noalloc ? we::gemm_reduce_plan(G) : we::gemm_plan(G);
+    if (!noalloc) return we::gemm_plan(G);
+    // the same plan where the fixed array holds it; the older rules' say what is refused, and run where the plan needs more
+    const we::GemmReducePlan older = we::gemm_reduce_plan(G), plan = we::gemm_plan(G);
+    return std::max(older.scratch_bytes, plan.scratch_bytes) > we::kNoallocScratchBytes ? older : plan;
   };
   auto launch_planned = [&](we::GemmLaunch& G, const we::GemmReducePlan& rp, void* part) {
     if (rp.scratch_bytes) {
