@@ -30,7 +30,7 @@
 //   * K rows and V^T rows are XOR-swizzled by 16-byte chunk so the MFMA operand reads are bank-conflict free.
 //   * LDS is double-buffered: the next tile's loads are in flight during this tile's MFMAs, then stored to
 //     the other buffer; one barrier per tile.
-// f32: attn_planes_kernel (head dims 64 and 128, 160 tokens or more: two f16 planes per operand on the 32x32x16 f16 MFMA),
+// f32: attn_planes_kernel (head dim 128 from 160 tokens on, 64 from 320: two f16 planes per operand on the 32x32x16 f16 MFMA),
 // and attn32_kernel (32x32x2 f32 MFMA, exact f32 products, a single LDS buffer, P kept in f32) for the rest.
 #include <cstdlib>
 #include <cstring>
