@@ -205,8 +205,8 @@ int we_conv3x3_params(we_ctx* ctx, uint32_t height, uint32_t width, uint32_t cin
  * multiplied plane by plane: three bf16 planes whose sum is the f32 value exactly, or, for large products of f32 x with
  * fp8 weights and for the 3x3 convolution of an f32 image, two f16 planes scaled by powers of two (per row of x or W, per
  * image). Two planes hold a value to 2^-23 of itself down to 2^-29 of its row's or image's largest and to 2^-20 down to
- * 2^-31; operands in which more than a few nonzero values lie further below (1 to 64 others in a row or image, 8 and a
- * millionth of all) are found on the device and take the exact planes. */
+ * 2^-31; operands in which more than a few nonzero values lie further below (1 to 64 others in a row or image, 2 in a
+ * million of all) are found on the device and take the exact planes. */
 int we_matmul(we_ctx* ctx, const we_matmul_params* p, int x_dtype, const void* x, int w_dtype, const void* w,
               const void* w_scales, uint32_t group, int y_dtype, void* y, const float* bias, uint32_t flags);
 /* we_matmul that allocates nothing. No counterpart in the reference: for callers that cannot allocate device memory

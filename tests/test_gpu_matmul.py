@@ -782,17 +782,17 @@ def test_conv3x3_planes_of_large_and_small_operands(graph, ex, ew):
 
 @pytest.mark.parametrize("w_dt", [we.F32, we.BF16])
 @pytest.mark.parametrize("e", [24, 30, 40])
-@pytest.mark.parametrize("what", ["small channel", "large pixel", "large weights", "small weights"])
+@pytest.mark.parametrize("what", ["small channel", "small channel, 8 pixels", "large pixel", "large weights", "small weights"])
 def test_conv3x3_planes_of_wide_ranges(graph, what, e, w_dt):
     """Values 2^e apart that do not meet in a result: an image channel 2^-e of the others that output channel 2 alone reads;
     one pixel's value 2^e above the rest in a channel whose weights are 0; weights 2^e above the rest for a channel that
     is 0 in the image; an output channel whose weights are 2^-e of one weight that only meets zeros. Every
     output channel to 1e-5 of its own largest."""
-    h, w, cin, cout = 16, 18, 64, 40
+    h, w, cin, cout = (2, 4, 64, 40) if what.endswith("8 pixels") else (16, 18, 64, 40)
     rng = np.random.default_rng(e)
     x = rng.standard_normal((h * w, cin)).astype(np.float32)
     wt = rng.standard_normal((cout, 9, cin)).astype(np.float32)
-    if what == "small channel":
+    if what.startswith("small channel"):
         x[:, 7] *= np.float32(2.0 ** -e)
         wt[2, :, :7] = wt[2, :, 8:] = 0
     elif what == "large pixel":

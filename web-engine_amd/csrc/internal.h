@@ -197,7 +197,9 @@ hipError_t launch_split_f32_planes(const float* x, uint32_t m, uint32_t k, uint3
 // than planes_most_tiny in all where the rows are not for planes; else range[0] (cleared before) is set there.
 constexpr uint32_t kRangeWords = 2048;
 inline uint32_t range_words(uint32_t m) { return m < kRangeWords ? (m + 3) / 4 * 4 : kRangeWords; }
-inline uint32_t planes_most_tiny(uint32_t m, uint32_t k) { return (uint32_t)(8 + ((uint64_t)m * k >> 20)); }
+// 2 in a million of n values, at most 2 of few and none of very few: fewer than a row of K values, a column of 65 rows or a
+// channel of an image can hold, and five to ten times what products like silu(a) b do
+inline uint32_t planes_most_tiny(uint64_t n) { return (uint32_t)(n >= (3u << 19) ? n >> 19 : n >= (2u << 16) ? 2 : n >> 16); }
 hipError_t launch_split_f32_f16x2(const void* x, int dtype, uint32_t m, uint32_t k, uint32_t x_stride, uint16_t* out,
                                   uint32_t kp, int planes, int lo_at, int hi_at, float* inv, bool words, uint32_t* range,
                                   hipStream_t s);

@@ -44,7 +44,7 @@ __global__ void __launch_bounds__(256) split_f32_planes_kernel(const float* __re
 // 2^3, still fits), to 2^-20 of itself down to 2^-31, and to 2^-52 of that largest below. The rounding of the sums in f32
 // is larger than the first of these (rel. error of 1024 x 6144 x 6144 against f64: see the GEMM's dispatch). Values below
 // 2^-31 of the largest, but 0, are counted as tiny: with more than one of them to 64 others in a row, or more than
-// 8 + 2^-20 of all in the operand, the planes are not used: three bf16 planes (GEMM) or the general kernel (convolution) run
+// planes_most_tiny in the operand, the planes are not used: three bf16 planes (GEMM) or the general kernel (convolution) run
 // instead, chosen on the device. (Normal data holds 1e-9 of them, products like silu(a) b 1e-7; a row with an outlier, or
 // a column far below the others, many.) inf stays inf with a NaN beside it, as in the three bf16 planes.
 constexpr float kPlaneLo = 4096.0f;
@@ -104,7 +104,7 @@ __device__ __forceinline__ void split_f16x2(const float (&v)[8], float s, u32x4&
 // Rows [k values at src + row * stride] -> f16 planes at out + row * planes * kp, zeros past k: plane lo_at holds lo, plane
 // hi_at hi (lo_at < 0: hi alone). The row's inverse scale goes to inv[row]. Two reads of the row (the second from L2):
 // k % 8 == 0, rows and out 16-byte aligned. A workgroup takes the rows from blockIdx.x on in steps of the grid. Tiny values
-// (above; `most` is 8 + 2^-20 of all): WORDS, their number over the workgroup's rows to range[blockIdx.x], most + 1 where they
+// (above; `most`: planes_most_tiny): WORDS, their number over the workgroup's rows to range[blockIdx.x], most + 1 where they
 // are too many already; else they are added to range[1], and range[0] is set where they are too many.
 template <int DT, bool WORDS>
 __global__ void __launch_bounds__(256) split_f32_f16x2_kernel(const void* __restrict__ src, uint32_t m, uint32_t k,
@@ -164,7 +164,7 @@ hipError_t launch_split_f32_f16x2(const void* x, int dtype, uint32_t m, uint32_t
                     : dtype == F32 ? split_f32_f16x2_kernel<F32, false>
                                    : split_f32_f16x2_kernel<BF16, false>;
   hipLaunchKernelGGL(kern, dim3(words ? range_words(m) : m), dim3(256), 0, s, x, m, k, x_stride, out, kp, planes, lo_at,
-                     hi_at, inv, range, planes_most_tiny(m, k));
+                     hi_at, inv, range, planes_most_tiny((uint64_t)m * k));
   return hipGetLastError();
 }
 
@@ -195,7 +195,8 @@ __global__ void __launch_bounds__(256) image_amax_kernel(const float* __restrict
 }
 __global__ void __launch_bounds__(256) image_f16x2_kernel(const float* __restrict__ x, size_t n, uint32_t cin,
                                                           const uint32_t* __restrict__ part, uint16_t* __restrict__ out,
-                                                          float* __restrict__ inv, uint32_t* __restrict__ range) {
+                                                          float* __restrict__ inv, uint32_t* __restrict__ range,
+                                                          uint32_t most) {
   __shared__ uint32_t red[4], red2[4], red3[4];
   static_assert(kImageParts == 512, "two parts per thread");
   const uint32_t t = threadIdx.x, big = block_max256(max(part[t], part[256 + t]), red);
@@ -219,7 +220,7 @@ __global__ void __launch_bounds__(256) image_f16x2_kernel(const float* __restric
     for (int e = 0; e < 8; e++) tiny += low_key(v[e] * s) < kPlaneTinyKey ? 1u : 0u;
     const uint32_t count = block_sum256(tiny, red2);
     const uint32_t nonzero = block_sum256(part[kImageParts + t] + part[kImageParts + 256 + t], red3);
-    if (t == 0 && atomicAdd(range + 2, count) + count > min(8u + (uint32_t)(n >> 20), nonzero / 64u)) atomicOr(range, 1u);
+    if (t == 0 && atomicAdd(range + 2, count) + count > min(most, nonzero / 64u)) atomicOr(range, 1u);
   }
 }
 
@@ -230,7 +231,7 @@ hipError_t launch_image_f16x2(const float* x, uint32_t pixels, uint32_t cin, uin
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(image_f16x2_kernel, dim3((unsigned)((n / 8 + 255) / 256)), dim3(256), 0, s, x, n, cin, part, out, inv,
-                     range);
+                     range, planes_most_tiny(n));
   return hipGetLastError();
 }
 

@@ -1155,7 +1155,7 @@ int matmul_impl(we_ctx* ctx, const we_matmul_params* p, int x_dtype, const void*
       two.row_scale = inv;
       two.range = range;
       two.range_n = we::range_words(p->m);
-      two.range_most = we::planes_most_tiny(p->m, p->k);
+      two.range_most = we::planes_most_tiny((uint64_t)p->m * p->k);
       two.skip_out = range + we::kRangeWords;
       two.f32 = xs;
       two.f32_stride = p->x_stride;
