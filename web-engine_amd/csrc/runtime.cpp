@@ -4,9 +4,9 @@
 // points that hand off to the kernels.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
 #include <cstdarg>
-#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -1135,13 +1135,13 @@ int matmul_impl(we_ctx* ctx, const we_matmul_params* p, int x_dtype, const void*
   // Two f16 planes [M, 2K] (lo | hi) for fp8 weights (exact in f16), each row scaled by a power of two of its own: a third
   // fewer products and fewer f32 roundings than three bf16 planes (1024 x 6144 x 6144: error against f64 9.1e-7 -> 4.2e-7).
   // Rows with values too far apart for them (kernels_misc.hip) are found on the device: then the launch writes the three
-  // exact planes [M, 3K] over the two, and the GEMM over them runs behind, which otherwise returns at once. Not for M <= 64 and shapes that three planes run in more
-  // than two K slices: those short sums round less than the f16 planes do (17 x 6144 x 2048 1.1e-7 with three planes,
-  // 1.4e-7 with two; 128 x 2048 x 8192 1.6e-7 and 2.5e-7); nor where the products are too few to pay for the launches.
+  // exact planes [M, 3K] over the two, and the GEMM over them runs behind, which otherwise returns at once. Not for M <= 64
+  // and shapes that three planes run in more than two K slices: those short sums round less than the f16 planes do (17 x
+  // 6144 x 2048 1.1e-7 with three planes, 1.4e-7 with two; 128 x 2048 x 8192 1.6e-7 and 2.5e-7); nor where the products are
+  // too few to pay for the launch behind, nor with the q / k epilogue, which one of the two plans may lack.
   if (planes && w_dtype == WE_FP8_E4M3 && p->m > 64 && !(has_qk && y_dtype != WE_F32) &&
       2.0 * p->m * p->n * p->k >= kTwoPlanesWork && p->k >= kTwoPlanesK &&
-      we::gemm_reduce_plan(planes_launch(3)).rsplits <= 2 &&
-      we::gemm_fast_supported(planes_launch(2))) {
+      we::gemm_reduce_plan(planes_launch(3)).rsplits <= 2 && we::gemm_fast_supported(planes_launch(2))) {
     we::GemmLaunch two = planes_launch(2), three = planes_launch(3);
     const we::GemmReducePlan rp2 = plan_of(two), rp3 = we::gemm_reduce_plan(three);  // three: as few launches as can be
     auto round256 = [](uint64_t n) { return (size_t)((n + 255) / 256 * 256); };
@@ -1199,8 +1199,7 @@ int matmul_impl(we_ctx* ctx, const we_matmul_params* p, int x_dtype, const void*
     }
     if (plane_bytes) {
       L.x = scratch;
-      const hipError_t e =
-          we::launch_split_f32_planes(xs, p->m, p->k, p->x_stride, (uint16_t*)scratch, ctx->compute);
+      const hipError_t e = we::launch_split_f32_planes(xs, p->m, p->k, p->x_stride, (uint16_t*)scratch, ctx->compute);
       if (e != hipSuccess) return hip_fail(ctx, e, "f32 plane split launch");
     }
     const hipError_t e = launch_planned(L, rp, scratch + plane_bytes);
