@@ -294,3 +294,24 @@ def test_f32_planes_of_one_large_value(graph, tune, e):
     got, want = got.reshape(tokens, heads, dim), want.reshape(tokens, heads, dim)
     assert np.abs(got[:-1] - want[:-1]).max() < 1e-5
     assert np.abs(got[:-1, :2, 9] - want[:-1, :2, 9]).max() < 1e-5
+
+
+@pytest.mark.parametrize("tokens,heads,dim", [(300, 4, 128), (700, 48, 64)])  # 4 and 8 waves per workgroup
+def test_f32_planes_in_place(graph, tokens, heads, dim):
+    """The output over the queries, with query rows of too wide a range in some blocks of 32 and one kv head for the f32 MFMA
+    kernel: what a separate output holds, bit for bit, and the oracle's values."""
+    kv_heads = heads // 2
+    q, k, v = lcg_random(tokens, [tokens * heads * dim, tokens * kv_heads * dim, tokens * kv_heads * dim])
+    q3, k3 = q.reshape(tokens, heads, dim), k.reshape(tokens, kv_heads, dim)
+    for t, h in ((5, 0), (40, 1), (tokens - 1, 0)):
+        q3[t, h, ::2] *= np.float32(2.0 ** -30)
+    k3[7, 1] *= np.float32(2.0 ** -20)
+    shape = we.AttentionShape(tokens, heads, kv_heads, dim, causal=True)
+    apart = run(graph, q, k, v, shape, we.F32)
+    mark = graph.mark()
+    qb = graph.buffer(q)
+    graph.attention(tokens, heads, kv_heads, dim, True, we.F32, qb, graph.buffer(k), graph.buffer(v), qb)
+    inside = graph.read(qb, dtype=np.float32).astype(np.float64)
+    graph.release(mark)
+    assert np.array_equal(inside, apart)
+    assert np.abs(apart - O.attention(q, k, v, tokens, heads, kv_heads, dim, True)).max() < 1e-5
